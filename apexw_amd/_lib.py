@@ -13,7 +13,7 @@ import numpy as np
 
 from ._build import LIB_PATH
 
-ABI_VERSION = 24
+ABI_VERSION = 25
 
 # dtype codes
 F32, BF16, F16, U8, I8 = 0, 1, 2, 3, 4
@@ -52,6 +52,7 @@ HP_LION = 1 << 12
 HP_SLOW = 1 << 13
 HP_LERP3_HI = 1 << 14
 HP_GRAD_DTYPES = 1 << 15
+HP_ROW_SUMSQ = 1 << 16
 
 STATUS = {0: "ok", 1: "invalid argument", 2: "unsupported dtype combination", 3: "launch failed",
           4: "misaligned pointer", 5: "exceeds the fixed workspace of the allocation-free entry point"}
@@ -175,6 +176,7 @@ SIGNATURES = {
     "apexw_grad_prep_units": (ctypes.c_int64, [_vp]),
     "apexw_grad_prepare": (ctypes.c_int, [_vp, _i32, _vp, _i64, _f32, _u32, _vp, _vp]),
     "apexw_grad_row_means": (ctypes.c_int, [_vp, _i32, _vp, _i64, _f32, _u32, _vp, _vp]),
+    "apexw_grad_row_stats": (ctypes.c_int, [_vp, _i32, _vp, _i64, _f32, _u32, _vp, _vp]),
     "apexw_gemm_grouped_items": (ctypes.c_int64, [_vp, _i32]),
     "apexw_gemm_grouped_schedule": (ctypes.c_int, [_vp, _i32, _vp, _i64, _i32, ctypes.POINTER(ctypes.c_int64), _vp,
                                                    ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(ctypes.c_int32)]),

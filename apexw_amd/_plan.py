@@ -408,9 +408,11 @@ class StepPlan:
         prep["n"] = [p.numel() for p in self.params]
         prep["dtype"] = [_DT[gd] for gd in self.grad_dtypes]
         if self.gc_fold:
-            self.gc_means = [torch.empty(max(p.numel() // int(prep["row_len"][i]), 1) if prep["row_len"][i] else 1,
-                                         dtype=torch.float32, device=self.device)
-                             for i, p in enumerate(self.params)]
+            # each row's mean; the buffer holds as many floats again behind them, for the rows' sums
+            # of squares of a step with a clip
+            n_rows = [max(p.numel() // int(prep["row_len"][i]), 1) if prep["row_len"][i] else 1
+                      for i, p in enumerate(self.params)]
+            self.gc_means = [torch.empty(2 * k, dtype=torch.float32, device=self.device)[:k] for k in n_rows]
             prep["out"] = [m.data_ptr() for m in self.gc_means]
             tab = self.host_table
             rows = prep["row_len"] > 0
@@ -448,12 +450,15 @@ class StepPlan:
         self.n_prep_units = len(units)
         self.d_prep_units = _upload(units.view(np.uint8), self.device)
 
-    def _prepare_grads(self, inv_scale, stream, amp_dyn=None):
+    def _prepare_grads(self, inv_scale, stream, amp_dyn=None, clip=False):
         """Sanitize, unscale and centralize into the prepared-grad buffers, or (folded
-        path) only the row means of the sanitized, unscaled grads.  amp_dyn: device
-        scalars of a GradScaler step (the unscale factor is read there)."""
+        path) only the row means of the sanitized, unscaled grads, with each row's sum of
+        squares when a clip follows.  amp_dyn: device scalars of a GradScaler step (the
+        unscale factor is read there)."""
         flags = L.HP_SANITIZE | (L.HP_UNSCALE if inv_scale is not None else 0)
-        fn = self._lib.apexw_grad_row_means if self.gc_fold else self._lib.apexw_grad_prepare
+        fn = self._lib.apexw_grad_prepare
+        if self.gc_fold:
+            fn = self._lib.apexw_grad_row_stats if clip else self._lib.apexw_grad_row_means
         st = fn(self.d_prep.data_ptr(), len(self.params), self.d_prep_units.data_ptr(), self.n_prep_units,
                 1.0 if inv_scale is None else inv_scale, flags, amp_dyn, stream)
         L.check(st, "apexw_grad_row_means" if self.gc_fold else "apexw_grad_prepare")
@@ -635,7 +640,8 @@ class StepPlan:
             self.d_table.data_ptr(), len(self.params), self.d_units.data_ptr(), self.n_units, unit,
             self.d_unit_begin.data_ptr(), part.data_ptr(), norms.data_ptr(), float(clip),
             1.0 if inv_scale is None else inv_scale,
-            (L.HP_SANITIZE if sanitize else 0) | (L.HP_UNSCALE if inv_scale is not None else 0), coef.data_ptr(),
+            (L.HP_SANITIZE if sanitize else 0) | (L.HP_UNSCALE if inv_scale is not None else 0)
+            | (L.HP_ROW_SUMSQ if self.gc_fold else 0), coef.data_ptr(),
             amp_dyn, self.d_rows.data_ptr() if self.d_rows is not None else None, stream)
         L.check(st, "apexw_grad_clip_coef")
         return coef
@@ -912,7 +918,7 @@ class StepPlan:
             lr, b1, b2, eps = prog.amp_scalars
             self._amp_prepare(prog.amp, prog.amp_groups, lr, b1, b2, eps, stream)
         if prog.prep is not None:
-            self._prepare_grads(prog.prep[0], stream, prog.prep[1])
+            self._prepare_grads(prog.prep[0], stream, prog.prep[1], prog.clip is not None)
         if prog.clip is not None:
             self._clip(prog.clip, prog.sanitize, prog.inv_scale, stream, prog.amp_dyn)
         table = self.d_table.data_ptr()

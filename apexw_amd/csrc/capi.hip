@@ -35,7 +35,7 @@ int apexw_launch_muon_coordwise(float*, const void*, int32_t, void*, int32_t, in
 int apexw_launch_grad_prep(const apexw_grad_prep*, const apexw_unit*, int64_t, float, uint32_t, const apexw_amp_dyn*,
                            hipStream_t);
 int apexw_launch_row_means(const apexw_grad_prep*, const apexw_unit*, int64_t, float, uint32_t, const apexw_amp_dyn*,
-                           hipStream_t);
+                           bool, hipStream_t);
 int apexw_launch_gemm_grouped(const apexw_gemm_problem*, const uint32_t*, const int32_t*, int32_t, int32_t,
                               const apexw_amp_dyn*, hipStream_t);
 int apexw_launch_muon_prepare(float*, const void*, int32_t, int64_t, int64_t, float, float, int32_t, float, float,
@@ -642,7 +642,15 @@ int apexw_grad_row_means(const apexw_grad_prep* preps, int32_t n_preps, const ap
   if (!preps || !units || n_preps <= 0 || n_units < 0) return APEXW_ERR_ARG;
   if (flags & ~(APEXW_HP_SANITIZE | APEXW_HP_UNSCALE)) return APEXW_ERR_ARG;
   if ((flags & APEXW_HP_UNSCALE) && !amp && !apexw_inv_scale_ok(grad_inv_scale)) return APEXW_ERR_ARG;
-  return apexw_launch_row_means(preps, units, n_units, grad_inv_scale, flags, amp, (hipStream_t)stream);
+  return apexw_launch_row_means(preps, units, n_units, grad_inv_scale, flags, amp, false, (hipStream_t)stream);
+}
+
+int apexw_grad_row_stats(const apexw_grad_prep* preps, int32_t n_preps, const apexw_unit* units, int64_t n_units,
+                         float grad_inv_scale, uint32_t flags, const apexw_amp_dyn* amp, void* stream) {
+  if (!preps || !units || n_preps <= 0 || n_units < 0) return APEXW_ERR_ARG;
+  if (flags & ~(APEXW_HP_SANITIZE | APEXW_HP_UNSCALE)) return APEXW_ERR_ARG;
+  if ((flags & APEXW_HP_UNSCALE) && !amp && !apexw_inv_scale_ok(grad_inv_scale)) return APEXW_ERR_ARG;
+  return apexw_launch_row_means(preps, units, n_units, grad_inv_scale, flags, amp, true, (hipStream_t)stream);
 }
 
 int apexw_amp_prepare(const float* found_inf, const float* grad_scale, int32_t* skips, int32_t skips_folded,

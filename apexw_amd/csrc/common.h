@@ -129,6 +129,39 @@ template <int DT> APEXW_DEV void store8(void* base, int64_t i, const float (&x)[
   }
 }
 
+// Raw 16-byte loads of 8 consecutive elements of dtype DT (two for fp32), and
+// their values.
+template <int DT> struct Raw8 {
+  u32x4 w[DT == APEXW_F32 ? 2 : 1];
+};
+template <int DT> APEXW_DEV void raw_load8(const void* base, int64_t i, Raw8<DT>& r) {
+  if constexpr (DT == APEXW_F32) {
+    auto p = APEXW_GLOBAL(const u32x4, (const float*)base + i);
+    r.w[0] = __builtin_nontemporal_load(p);
+    r.w[1] = __builtin_nontemporal_load(p + 1);
+  } else {
+    r.w[0] = __builtin_nontemporal_load(APEXW_GLOBAL(const u32x4, (const uint16_t*)base + i));
+  }
+}
+template <int DT> APEXW_DEV void unpack8(const Raw8<DT>& r, float (&x)[8]) {
+#pragma unroll
+  for (int q = 0; q < (DT == APEXW_F32 ? 2 : 1); ++q) {
+    const uint32_t w[4] = {r.w[q].x, r.w[q].y, r.w[q].z, r.w[q].w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if constexpr (DT == APEXW_F32) {
+        x[4 * q + k] = __uint_as_float(w[k]);
+      } else if constexpr (DT == APEXW_BF16) {
+        x[2 * k] = bf16_bits_to_f32(w[k] & 0xFFFFu);
+        x[2 * k + 1] = __uint_as_float(w[k] & 0xFFFF0000u);
+      } else {
+        x[2 * k] = f16_bits_to_f32(w[k] & 0xFFFFu);
+        x[2 * k + 1] = f16_bits_to_f32(w[k] >> 16);
+      }
+    }
+  }
+}
+
 template <int DT> APEXW_DEV float load1(const void* base, int64_t i) {
   if constexpr (DT == APEXW_F32) return APEXW_GLOBAL(const float, base)[i];
   else if constexpr (DT == APEXW_BF16) return bf16_bits_to_f32(APEXW_GLOBAL(const uint16_t, base)[i]);

@@ -8,8 +8,11 @@
 //
 // Three short launches, deterministic (no atomics):
 //   1. one wavefront per work unit of the chunk table -> sum of squares
-//   2. one wavefront per tensor sums its (contiguous) units -> rounded norm
+//   2. one wavefront per tensor (a workgroup for a tensor of many units) sums its
+//      (contiguous) units -> rounded norm
 //   3. one workgroup combines the tensor norms -> coefficient
+// With grad centralization the pass that forms the row means also forms each row's
+// sum of squares about its mean (apexw_grad_row_stats), and 1 skips those tensors.
 #include <mutex>
 
 #include "common.h"
@@ -120,13 +123,20 @@ __global__ __launch_bounds__(256) void sumsq_kernel(const apexw_tensor* __restri
   if (amp) inv = amp->grad_inv_scale;
   const uint32_t wave = uniform(threadIdx.x >> 6);
   const bool san = flags & APEXW_HP_SANITIZE, unscale = flags & APEXW_HP_UNSCALE;
+  const bool row_sums = flags & APEXW_HP_ROW_SUMSQ;
   // a workgroup walks a contiguous chunk of 64 units, its waves interleaved, one
   // workgroup per chunk (the dispatcher balances the tail): at C4 (2.08 B grads)
   // 0.631 ms against 0.679 ms for a resident grid striding by 4 units
-  for (int64_t base = (int64_t)blockIdx.x * 64; base < n_units; base += (int64_t)gridDim.x * 64)
-  for (int64_t u = base + wave, u_end = base + 64 < n_units ? base + 64 : n_units; u < u_end; u += 4) {
+  for (int64_t base = (int64_t)blockIdx.x * 64; base < n_units; base += (int64_t)gridDim.x * 64) {
+  const int64_t u_end = base + 64 < n_units ? base + 64 : n_units;
+  // a chunk inside one tensor whose row sums the row pass has formed: nothing to do
+  // (a tensor's units are contiguous)
+  const uint32_t t0 = units[base].tensor;
+  if (row_sums && (tensors[t0].flags & APEXW_FLAG_GC) && units[u_end - 1].tensor == t0) continue;
+  for (int64_t u = base + wave; u < u_end; u += 4) {
     const apexw_unit un = units[u];
     const apexw_tensor& t = tensors[un.tensor];
+    if (row_sums && (t.flags & APEXW_FLAG_GC)) continue;
     const int64_t us = unit_size > 0 ? unit_size : (t.block > 0 ? (int64_t)t.block : 64);
     const int64_t start = (int64_t)un.unit * us;
     const int64_t cnt = (t.n - start) < us ? (t.n - start) : us;
@@ -145,21 +155,81 @@ __global__ __launch_bounds__(256) void sumsq_kernel(const apexw_tensor* __restri
     else s = unit_sumsq<APEXW_F16>(t, start, cnt, san, unscale, inv, means, rl);
     if (lane_id() == 0) partial[u] = s;
   }
+  }
 }
 
-__global__ __launch_bounds__(256) void tensor_norm_kernel(const apexw_tensor* __restrict__ tensors, int32_t n_tensors,
-                                                          const int64_t* __restrict__ unit_begin,
-                                                          const float* __restrict__ partial, float* __restrict__ norm) {
-  const uint32_t wave = uniform(threadIdx.x >> 6);
-  const int64_t stride = (int64_t)gridDim.x * 4;
-  for (int64_t t = (int64_t)blockIdx.x * 4 + wave; t < n_tensors; t += stride) {
-    float acc = 0.0f;
-    for (int64_t u = unit_begin[t] + lane_id(); u < unit_begin[t + 1]; u += 64) acc += partial[u];
-    acc = wave_sum(acc);
+// The partial sums of one tensor: its units' (from sumsq_kernel), or, for a
+// centralized tensor under APEXW_HP_ROW_SUMSQ, its rows' (written after its row means
+// by row_means_kernel<true>).
+struct NormSpan {
+  const float* p;
+  int64_t n;
+};
+APEXW_DEV NormSpan norm_span(const apexw_tensor* tensors, int64_t t, const int64_t* unit_begin, const float* partial,
+                             uint32_t flags, const apexw_row_means* rows) {
+  const apexw_tensor& d = tensors[t];
+  if ((flags & APEXW_HP_ROW_SUMSQ) && (d.flags & APEXW_FLAG_GC)) {
+    const float* means = rows ? rows[t].means : d.m_scale;
+    const int64_t n_rows = d.n / (rows ? rows[t].row_len : (int64_t)d.block);
+    return {means + n_rows, n_rows};
+  }
+  return {partial + unit_begin[t], unit_begin[t + 1] - unit_begin[t]};
+}
+
+// The sum of `s` by `step` lanes, this one the `first`: eight loads in flight and
+// eight running sums (a plain loop waits for memory at each addition).
+APEXW_DEV float span_sum(const NormSpan& s, int64_t first, int64_t step) {
+  float a[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  int64_t i = first;
+  for (; i + 7 * step < s.n; i += 8 * step) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) a[j] += s.p[i + j * step];
+  }
+  for (; i < s.n; i += step) a[0] += s.p[i];
+  return ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+}
+
+// Each tensor's norm, rounded to its grad dtype, as torch._foreach_norm does.  A
+// workgroup of 16 waves takes `per` tensors (16, or 1 when there are few), a wave
+// each; a tensor of more than kNormWave partials is summed by the whole workgroup:
+// one wave alone walks the 28,672 units of a 14336 x 4096 matrix serially (123 us for
+// the 36 tensors of four Llama layers, 6 us so; 68 -> 5 us for GPT-2-small).
+constexpr int kNormWaves = 16;
+constexpr int64_t kNormWave = 1024;
+__global__ __launch_bounds__(kNormWaves * 64) void tensor_norm_kernel(
+    const apexw_tensor* __restrict__ tensors, int32_t n_tensors, const int64_t* __restrict__ unit_begin,
+    const float* __restrict__ partial, float* __restrict__ norm, int32_t per, uint32_t flags,
+    const apexw_row_means* __restrict__ rows) {
+  __shared__ float s_part[kNormWaves];
+  const int wave = (int)uniform(threadIdx.x >> 6);
+  auto store = [&](int64_t t, float acc) {
     const uint32_t gd = (tensors[t].flags >> APEXW_FLAG_GDT_SHIFT) & 3u;
     float nrm = sqrtf(acc);
     nrm = gd == APEXW_BF16 ? rnd<APEXW_BF16>(nrm) : (gd == APEXW_F16 ? rnd<APEXW_F16>(nrm) : nrm);
-    if (lane_id() == 0) norm[t] = nrm;
+    norm[t] = nrm;
+  };
+  for (int64_t t0 = (int64_t)blockIdx.x * per; t0 < n_tensors; t0 += (int64_t)gridDim.x * per) {
+    const int64_t t_end = t0 + per < n_tensors ? t0 + per : n_tensors;
+    if (t0 + wave < t_end) {
+      const NormSpan s = norm_span(tensors, t0 + wave, unit_begin, partial, flags, rows);
+      if (s.n <= kNormWave) {
+        const float acc = wave_sum(span_sum(s, lane_id(), 64));
+        if (lane_id() == 0) store(t0 + wave, acc);
+      }
+    }
+    for (int64_t t = t0; t < t_end; ++t) {
+      const NormSpan s = norm_span(tensors, t, unit_begin, partial, flags, rows);
+      if (s.n <= kNormWave) continue;
+      const float acc = wave_sum(span_sum(s, threadIdx.x, kNormWaves * 64));
+      if (lane_id() == 0) s_part[wave] = acc;
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        float tot = 0.0f;
+        for (int w = 0; w < kNormWaves; ++w) tot += s_part[w];
+        store(t, tot);
+      }
+      __syncthreads();   // s_part is the next large tensor's
+    }
   }
 }
 
@@ -264,40 +334,100 @@ APEXW_DEV void prep_unit(const apexw_grad_prep& d, int64_t unit, bool san, bool 
 // Row means only (the fold of centralization into the step kernels): one wave per
 // row of a descriptor with row_len > 0; d.out is a float array of one mean per
 // row, each the grad dtype's rounding of the fp32 row sum over row_len of the
-// sanitized, unscaled grads.  A lane sums its 8-element vectors (four loads issued
-// before they are added; eight measured slower at C3), then the wave's lanes are
-// summed.
-template <int GD>
-APEXW_DEV void mean_row(const apexw_grad_prep& d, int64_t row, bool san, bool unscale, float inv) {
+// sanitized, unscaled grads.  SUMSQ (a clip follows): the row's sum of squares about
+// that mean, each difference rounded to the grad dtype, goes to d.out[rows + row].
+//
+// Bound by the read of the grads.  A lane holds its first kRowVecs 8-element vectors
+// (rows of up to 4096 16-bit elements whole), loaded before they are added, so the
+// second sum reads nothing again; a longer row's rest is read in batches of four and,
+// for the second sum, again.  Sanitizing changes only NaN / +-Inf grads, and one of
+// those makes the row's sum non-finite: the sums are formed without it, and a row
+// whose sum is not finite (rare) forms them again with it.
+// Four Llama layers (0.87 B bf16 grads, 1.75 GB, all centralized): 723 us for the means and
+// 644 us for the clip's own pass over them before, 527 us for both here.
+// Sixteen rows to a workgroup: enough workgroups for small models, whose rows are few.
+constexpr int64_t kRowChunk = 16;
+template <int GD> constexpr int kRowVecs = GD == APEXW_F32 ? 4 : 8;
+
+template <int GD, bool SAN>
+APEXW_DEV float row_value(float x, bool unscale, float inv) {
+  if constexpr (SAN) x = sanitize<GD>(x);
+  return unscale ? rnd<GD>(x * inv) : x;
+}
+
+// The row's sum (MEAN false) or its sum of squares about mean (MEAN true) over a lane's
+// share: the held vectors r, the rest of [a, b) and the ragged ends.
+template <int GD, bool SAN, bool MEAN>
+APEXW_DEV float row_sum(const apexw_grad_prep& d, const Raw8<GD> (&r)[kRowVecs<GD>], const PrepSpan& sp, int64_t lo,
+                        int64_t hi, bool unscale, float inv, float mean) {
+  constexpr int NV = kRowVecs<GD>;
   const int lane = lane_id();
-  const int64_t lo = row * d.row_len, hi = lo + d.row_len;
-  const PrepSpan sp = prep_span<GD>(d, lo, hi);
-  const int64_t head = sp.a - lo, n_end = head + (hi - sp.b);
   float s = 0.0f;
+  auto add = [&](float x) {
+    x = row_value<GD, SAN>(x, unscale, inv);
+    if constexpr (MEAN) {
+      x = rnd<GD>(x - mean);
+      s = fmaf(x, x, s);
+    } else {
+      s += x;
+    }
+  };
   int64_t i = sp.a + (int64_t)lane * 8;
+#pragma unroll
+  for (int q = 0; q < NV; ++q, i += 512) {
+    if (i < sp.b) {
+      float x[8];
+      unpack8<GD>(r[q], x);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) add(x[j]);
+    }
+  }
   for (; i + 3 * 512 < sp.b; i += 4 * 512) {
     float x[4][8];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) prep_vec8<GD>(d.g, i + q * 512, san, unscale, inv, x[q]);
+    for (int q = 0; q < 4; ++q) load8<GD>(d.g, i + q * 512, x[q]);
 #pragma unroll
     for (int q = 0; q < 4; ++q)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) s += x[q][j];
+      for (int j = 0; j < 8; ++j) add(x[q][j]);
   }
   for (; i < sp.b; i += 512) {
     float x[8];
-    prep_vec8<GD>(d.g, i, san, unscale, inv, x);
+    load8<GD>(d.g, i, x);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) s += x[j];
+    for (int j = 0; j < 8; ++j) add(x[j]);
   }
-  for (int64_t k = lane; k < n_end; k += 64) {
-    const int64_t i = k < head ? lo + k : sp.b + (k - head);
-    s += prep_value<GD>(d.g, i, san, unscale, inv);
-  }
-  s = wave_sum(s);
-  if (lane == 0) ((float*)d.out)[row] = rnd<GD>(s / (float)d.row_len);
+  // ragged ends: [lo, a) and [b, hi) (the whole row when not vectorized)
+  const int64_t head = sp.a - lo, n_end = head + (hi - sp.b);
+  for (int64_t k = lane; k < n_end; k += 64) add(load1<GD>(d.g, k < head ? lo + k : sp.b + (k - head)));
+  return wave_sum(s);
 }
 
+template <int GD, bool SUMSQ>
+APEXW_DEV void mean_row(const apexw_grad_prep& d, int64_t row, bool san, bool unscale, float inv) {
+  constexpr int NV = kRowVecs<GD>;
+  const int lane = lane_id();
+  const int64_t lo = row * d.row_len, hi = lo + d.row_len;
+  const PrepSpan sp = prep_span<GD>(d, lo, hi);
+  Raw8<GD> r[NV];
+#pragma unroll
+  for (int q = 0; q < NV; ++q) {
+    const int64_t i = sp.a + (int64_t)lane * 8 + q * 512;
+    if (i < sp.b) raw_load8<GD>(d.g, i, r[q]);
+  }
+  float s = row_sum<GD, false, false>(d, r, sp, lo, hi, unscale, inv, 0.0f);
+  const bool redo = san && !(s - s == 0.0f);   // wave-uniform: every lane holds the sum
+  if (redo) s = row_sum<GD, true, false>(d, r, sp, lo, hi, unscale, inv, 0.0f);
+  const float mean = rnd<GD>(s / (float)d.row_len);
+  if (lane == 0) ((float*)d.out)[row] = mean;
+  if constexpr (SUMSQ) {
+    const float q = redo ? row_sum<GD, true, true>(d, r, sp, lo, hi, unscale, inv, mean)
+                         : row_sum<GD, false, true>(d, r, sp, lo, hi, unscale, inv, mean);
+    if (lane == 0) ((float*)d.out)[d.n / d.row_len + row] = q;
+  }
+}
+
+template <bool SUMSQ>
 __global__ __launch_bounds__(256) void row_means_kernel(const apexw_grad_prep* __restrict__ preps,
                                                         const apexw_unit* __restrict__ units, int64_t n_units,
                                                         float inv, uint32_t flags,
@@ -305,14 +435,14 @@ __global__ __launch_bounds__(256) void row_means_kernel(const apexw_grad_prep* _
   if (amp) inv = amp->grad_inv_scale;
   const bool san = flags & APEXW_HP_SANITIZE, unscale = flags & APEXW_HP_UNSCALE;
   const uint32_t wave = uniform(threadIdx.x >> 6);
-  // workgroup b takes a contiguous chunk of 64 rows, its waves interleaved
-  for (int64_t base = (int64_t)blockIdx.x * 64; base < n_units; base += (int64_t)gridDim.x * 64)
-  for (int64_t u = base + wave, u_end = base + 64 < n_units ? base + 64 : n_units; u < u_end; u += 4) {
+  // workgroup b takes a contiguous chunk of kRowChunk rows, its waves interleaved
+  for (int64_t base = (int64_t)blockIdx.x * kRowChunk; base < n_units; base += (int64_t)gridDim.x * kRowChunk)
+  for (int64_t u = base + wave, u_end = base + kRowChunk < n_units ? base + kRowChunk : n_units; u < u_end; u += 4) {
     const apexw_unit un = units[u];
     const apexw_grad_prep& d = preps[un.tensor];
-    if (d.dtype == APEXW_F32) mean_row<APEXW_F32>(d, un.unit, san, unscale, inv);
-    else if (d.dtype == APEXW_BF16) mean_row<APEXW_BF16>(d, un.unit, san, unscale, inv);
-    else mean_row<APEXW_F16>(d, un.unit, san, unscale, inv);
+    if (d.dtype == APEXW_F32) mean_row<APEXW_F32, SUMSQ>(d, un.unit, san, unscale, inv);
+    else if (d.dtype == APEXW_BF16) mean_row<APEXW_BF16, SUMSQ>(d, un.unit, san, unscale, inv);
+    else mean_row<APEXW_F16, SUMSQ>(d, un.unit, san, unscale, inv);
   }
 }
 
@@ -350,11 +480,16 @@ int apexw_launch_clip(const apexw_tensor* tensors, int32_t n_tensors, const apex
                       const apexw_row_means* rows, hipStream_t stream);
 
 int apexw_launch_row_means(const apexw_grad_prep* preps, const apexw_unit* units, int64_t n_units, float inv,
-                           uint32_t flags, const apexw_amp_dyn* amp, hipStream_t stream) {
+                           uint32_t flags, const apexw_amp_dyn* amp, bool sumsq, hipStream_t stream) {
   if (n_units <= 0) return APEXW_OK;
-  const int64_t chunks = (n_units + 63) / 64;
+  const int64_t chunks = (n_units + kRowChunk - 1) / kRowChunk;
   const unsigned grid = (unsigned)(chunks < INT32_MAX ? chunks : INT32_MAX);
-  hipLaunchKernelGGL(row_means_kernel, dim3(grid), dim3(256), 0, stream, preps, units, n_units, inv, flags, amp);
+  if (sumsq)
+    hipLaunchKernelGGL(row_means_kernel<true>, dim3(grid), dim3(256), 0, stream, preps, units, n_units, inv, flags,
+                       amp);
+  else
+    hipLaunchKernelGGL(row_means_kernel<false>, dim3(grid), dim3(256), 0, stream, preps, units, n_units, inv, flags,
+                       amp);
   return hipGetLastError() == hipSuccess ? APEXW_OK : APEXW_ERR_LAUNCH;
 }
 
@@ -425,9 +560,12 @@ int apexw_launch_clip(const apexw_tensor* tensors, int32_t n_tensors, const apex
                        unit_partial, flags, inv, amp, rows);
   }
   if (n_tensors > 0) {
-    const int grid_tensors = apexw_resident_grid((const void*)tensor_norm_kernel, n_tensors);
-    hipLaunchKernelGGL(tensor_norm_kernel, dim3(grid_tensors), dim3(256), 0, stream, tensors, n_tensors, unit_begin,
-                       unit_partial, tensor_norm);
+    // a workgroup per tensor while that fills the chip at most a few times over, 16
+    // tensors to a workgroup beyond (small tensors then dominate the count)
+    const int32_t per = n_tensors <= 2048 ? 1 : kNormWaves;
+    const int32_t grid_tensors = (n_tensors + per - 1) / per;
+    hipLaunchKernelGGL(tensor_norm_kernel, dim3(grid_tensors), dim3(kNormWaves * 64), 0, stream, tensors, n_tensors,
+                       unit_begin, unit_partial, tensor_norm, per, flags, rows);
   }
   hipLaunchKernelGGL(clip_coef_kernel, dim3(1), dim3(1024), 0, stream, tensor_norm, n_tensors, clip, coef);
   return hipGetLastError() == hipSuccess ? APEXW_OK : APEXW_ERR_LAUNCH;

@@ -44,7 +44,7 @@
 extern "C" {
 #endif
 
-#define APEXW_ABI_VERSION 24
+#define APEXW_ABI_VERSION 25
 
 /* status codes */
 enum apexw_status {
@@ -201,6 +201,9 @@ typedef struct apexw_unit {
                                           when this flag is set and skipped otherwise.  The grads are
                                           prepared in their own dtype and read as fp32 values, as the
                                           reference's foreach order does. */
+#define APEXW_HP_ROW_SUMSQ (1u << 16)  /* apexw_grad_clip_coef: the centralized tensors' sums of squares are
+                                          those that apexw_grad_row_stats wrote after their row means in
+                                          this step; their grads are not read again */
 
 /* Step scalars of one launch, written on the device by apexw_amp_prepare (32 bytes). */
 typedef struct apexw_amp_dyn {
@@ -513,6 +516,15 @@ int apexw_grad_prepare(const apexw_grad_prep* preps, int32_t n_preps, const apex
  * (apexw/optimizer.py:238-243) without writing a prepared copy of the grads.
  */
 int apexw_grad_row_means(const apexw_grad_prep* preps, int32_t n_preps, const apexw_unit* units, int64_t n_units,
+                         float grad_inv_scale, uint32_t flags, const apexw_amp_dyn* amp, void* stream);
+
+/*
+ * apexw_grad_row_means with the global-norm clip's sums in the same pass: out holds
+ * 2 n / row_len floats, and entry n / row_len + r receives the sum of squares of
+ * dtype_round(g - mean) over row r.  The clip of the same step then takes
+ * APEXW_HP_ROW_SUMSQ.
+ */
+int apexw_grad_row_stats(const apexw_grad_prep* preps, int32_t n_preps, const apexw_unit* units, int64_t n_units,
                          float grad_inv_scale, uint32_t flags, const apexw_amp_dyn* amp, void* stream);
 
 /* Validate one descriptor (host copy) of apexw_grad_row_means: row_len > 0 divides n, out holds
