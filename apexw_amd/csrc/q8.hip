@@ -156,6 +156,17 @@ APEXW_DEV float lerp_to(float a, float b, float coef, bool hi) {
   return hi ? fmaf(coef, b - a, b) : fmaf(coef, b - a, a);
 }
 
+// ... of 8 elements, its orientation one uniform branch
+APEXW_DEV void lerp8(const float (&a)[8], const float (&b)[8], float (&x)[8], float coef, bool hi) {
+  if (hi) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = fmaf(coef, b[j] - a[j], b[j]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = fmaf(coef, b[j] - a[j], a[j]);
+  }
+}
+
 // NF4 nearest code, searchsorted(mids, x) over the 14 decision points (ties to the
 // lower code), through the 64-bucket midpoint table (LDS copy of kNf4MidTab):
 // one lookup and one comparison.
@@ -181,11 +192,11 @@ APEXW_DEV uint32_t nf4_sr(float x, float u, const float* code) {
 
 APEXW_DEV float unit_uniform(uint32_t r16) { return ((float)(r16 & 0xFFFFu) + 0.5f) * (1.0f / 65536.0f); }
 
-// log-uint8 code of v given the block scale (ratio floor 2^-24, 254 codes per 24 octaves).
-APEXW_DEV uint32_t logu8_code(float v, float vmax, bool sr, uint32_t r16) {
+// log-uint8 code of v given its ratio to the block scale (ratio floor 2^-24, 254 codes
+// per 24 octaves).  ratio >= 2^-24 is a normal number, where log2f is v_log_f32 itself.
+APEXW_DEV uint32_t logu8_code(float v, float ratio, bool sr, uint32_t r16) {
   if (!(v > 0.0f)) return 0u;
-  const float r = fmaxf(v / vmax, 0x1p-24f);
-  float q = log2f(r) * 0x1.52aaaap+3f;  // fp32(254/24)
+  float q = __builtin_amdgcn_logf(fmaxf(ratio, 0x1p-24f)) * 0x1.52aaaap+3f;  // fp32(254/24)
   q = q + 255.0f;
   if (sr) q = q + (unit_uniform(r16) - 0.5f);
   q = rintf(q);
@@ -295,191 +306,275 @@ APEXW_DEV float q8_param(float p, float upd, float decay, uint32_t tflags, bool 
   return rnd<PD>(x);
 }
 
-// One quantization block per wavefront, any layout (INT8 m, fp32 params, other
-// block sizes, unaligned tensors).  Runs in its own kernel so that its register
-// footprint does not lower the occupancy of the bf16 NF4 kernel below.
+// The general kernels' arithmetic, by instruction count (they are bound by vector issue
+// before memory): one quotient, root or rounding costs a few instructions instead of an
+// IEEE sequence, and results go to 16-bit and 8-bit words without an fp32 round trip.
+//
+// sqrt(x) for finite x >= 0, rounded to nearest: s = x y with y ~ rsqrt(x), then one FMA
+// residual (Markstein), wrong only within ~2^-45 of a rounding midpoint.  Below 2^-126
+// the result is off by at most 2^-63, added by every caller to an eps of kFastEps or more.
+APEXW_DEV float sqrt_shared(float x) {
+  // (an integer maximum: the float one first quiets NaNs)
+  const float y = __builtin_amdgcn_rsqf(__uint_as_float((uint32_t)max((int)__float_as_uint(x), 0x00800000)));
+  const float s = x * y;
+  return fmaf(fmaf(-s, s, x), 0.5f * y, s);
+}
+// x / y rounded to nearest for a normal y > 0 and a finite quotient, likewise: the
+// hardware reciprocal and one FMA residual.
+APEXW_DEV float div_once(float x, float y) {
+  const float r = __builtin_amdgcn_rcpf(y), q = x * r;
+  return fmaf(fmaf(-q, y, x), r, q);
+}
+// ... both with every denominator at least this (any real eps is)
+constexpr float kFastEps = 1e-12f;
+
+// x rounded to DT in place, and stored rounded to DT: bf16 in pairs
+// (v_cvt_pk_bf16_f32).
+template <int DT> APEXW_DEV void rnd8(float (&x)[8]) {
+#pragma unroll
+  for (int j = 0; j < 8; j += 2) {
+    if constexpr (DT == APEXW_BF16) {
+      const uint32_t w = pack_bf16x2(x[j], x[j + 1]);
+      x[j] = __uint_as_float(w << 16);
+      x[j + 1] = __uint_as_float(w & 0xFFFF0000u);
+    } else {
+      x[j] = rnd<DT>(x[j]);
+      x[j + 1] = rnd<DT>(x[j + 1]);
+    }
+  }
+}
+template <int DT> APEXW_DEV void store8_rnd(void* base, int64_t i, float (&x)[8]) {
+  if constexpr (DT == APEXW_BF16) {
+    const u32x4 w = {pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3]), pack_bf16x2(x[4], x[5]),
+                     pack_bf16x2(x[6], x[7])};
+    __builtin_nontemporal_store(w, APEXW_GLOBAL(u32x4, (uint16_t*)base + i));
+  } else {
+    store8<DT>(base, i, x);   // fp16 rounds there
+  }
+}
+
+// The four INT8 codes of a word times a scale: bytes biased by 128 convert in one
+// instruction each, and fma(b, s, -128 s) is the exact (b - 128) s rounded once.
+APEXW_DEV void i8_decode4(uint32_t w, float s, float* x) {
+  const uint32_t u = w ^ 0x80808080u;
+  const float z = -128.0f * s;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) x[j] = fmaf((float)((u >> (8 * j)) & 0xFFu), s, z);
+}
+// Four INT8 codes from m / scale: clamped to +-127, rounded to nearest even by adding
+// 1.5 x 2^23 (the code is then the low byte), gathered by byte permutes.
+APEXW_DEV uint32_t i8_encode4(const float* y) {
+  uint32_t z[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) z[j] = __float_as_uint(__builtin_amdgcn_fmed3f(y[j], -127.0f, 127.0f) + 12582912.0f);
+  const uint32_t lo = __builtin_amdgcn_perm(z[1], z[0], 0x0c0c0400u), hi = __builtin_amdgcn_perm(z[3], z[2], 0x0c0c0400u);
+  return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
+// unit_uniform(r) - 1/2 for the 16 bits r = h >> 16, exact in one FMA.
+APEXW_DEV float half_noise(uint32_t h) { return fmaf((float)(h >> 16), 0x1p-16f, 0x1p-17f - 0.5f); }
+
+// Maximum over a workgroup of 4 waves of two non-negative values; red: 8 floats of LDS,
+// alternated between two such buffers by the caller so that one barrier suffices.
+APEXW_DEV void block_max2(float& a, float& b, float* red) {
+  a = wave_max(a);
+  b = wave_max(b);
+  const int w = (int)(threadIdx.x >> 6);
+  if (lane_id() == 0) {
+    red[w] = a;
+    red[4 + w] = b;
+  }
+  __syncthreads();
+  a = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  b = fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7]));
+}
+
+// One quantization block per workgroup, any layout (INT8 m, fp32 params, other block
+// sizes, unaligned tensors): each of the four waves takes 512 of the up to 2048
+// elements, 8 per lane, and the block's two maxima meet in LDS.
+//
+// The block's serial path is what bounds small launches (16 blocks of 2048 elements:
+// 35 us when one wave walked a block's four groups, 9 us here) and its instruction
+// count the large ones: so one division per denominator (rcp_refined, div_shared)
+// instead of an IEEE sequence per element, the noise hashed once, and 8 elements'
+// state per lane instead of 32 (159 -> 96 VGPRs).  25 M parameters of a convolutional
+// network, nearly all INT8 rows: 140 -> 87 us per step.
 // SINGLE: the per-parameter in-backward update (ApexW._step_single_param_fused,
 // apexw/optimizer.py:2411-2457): raw fp32 grads, m = b1 m + (1-b1) g,
 // lookahead b1 m' + (1-b1) g, denominator sqrt(v) + eps_scaled without the eps
 // floor, p decayed in fp32 then p + (-step_size * num) / den, INT8 m
 // requantised from its own absmax (no EMA, no SR).
 template <int PD, bool NF4, bool QUAD, bool SINGLE>
-APEXW_DEV void q8_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, const Q8Ctx& c) {
+APEXW_DEV void q8_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, const Q8Ctx& c, float* red) {
   constexpr int GD = PD;
+  constexpr int NV = QUAD ? 2 : 8;   // second moments per lane
   const apexw_hparams& hp = *c.hp;
   const bool sr = hp.flags & APEXW_HP_SR;
   const uint32_t tflags = t.flags;
-  const bool vec = !(tflags & APEXW_FLAG_SCALAR);
   const int64_t bs = t.block;
   const int64_t start = (int64_t)blk * bs;
   const int64_t cnt_blk = (t.n - start) < bs ? (t.n - start) : bs;
-  const int lane = lane_id();
   const float ms_old = t.m_scale[blk];
   const float vs_old = t.v_scale[blk];
-  const uint32_t key = rng_key(hp.seed, tix, hp.step, 1u, (uint32_t)(start >> 32));
-  const uint32_t keyv = rng_key(hp.seed, tix, hp.step, 2u, (uint32_t)(start >> 32));
   const bool generic = tflags & APEXW_FLAG_GENERIC;
-
-  float mnew[4][8], vnew[4][8];
+  const int64_t rel = (int64_t)threadIdx.x * 8;
+  const int cnt = rel >= cnt_blk ? 0 : (int)((cnt_blk - rel) < 8 ? (cnt_blk - rel) : 8);
+  const int64_t e0 = start + rel;
+  const bool full = !(tflags & APEXW_FLAG_SCALAR) && cnt == 8;
+  float m[8], v[NV];
+  uint32_t h[8];
   float amax = 0.0f, vmax = 0.0f;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int64_t rel = (int64_t)(k * 64 + lane) * 8;
-    const int cnt = rel >= cnt_blk ? 0 : (int)((cnt_blk - rel) < 8 ? (cnt_blk - rel) : 8);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) { mnew[k][j] = 0.0f; vnew[k][j] = 0.0f; }
-    if (cnt == 0) continue;
-    const int64_t e0 = start + rel;
-    const bool full = vec && cnt == 8;
-    float p[8], g[8], m[8], v[8];
+  if (cnt) {
+    float p[8], g[8];
     // ---- load
     if (full) {
-      load8<PD>(t.p, e0, p);
-      load8<GD>(t.g, e0, g);
+      Raw8<PD> rp;
+      Raw8<GD> rg;
+      raw_load8<PD>(t.p, e0, rp);
+      raw_load8<GD>(t.g, e0, rg);
+      uint32_t mw[2], vw[2];
+      if constexpr (NF4) {
+        mw[0] = __builtin_nontemporal_load(APEXW_GLOBAL(const uint32_t, (const uint8_t*)t.m + (e0 >> 1)));
+      } else {
+        const u32x2 w = __builtin_nontemporal_load(APEXW_GLOBAL(const u32x2, (const int8_t*)t.m + e0));
+        mw[0] = w.x;
+        mw[1] = w.y;
+      }
+      if constexpr (QUAD) {
+        vw[0] = __builtin_nontemporal_load(APEXW_GLOBAL(const uint16_t, (const uint8_t*)t.v + (e0 >> 2)));
+      } else {
+        const u32x2 w = __builtin_nontemporal_load(APEXW_GLOBAL(const u32x2, (const uint8_t*)t.v + e0));
+        vw[0] = w.x;
+        vw[1] = w.y;
+      }
+      unpack8<PD>(rp, p);
+      unpack8<GD>(rg, g);
+      if constexpr (NF4) {
+        // even element in the high nibble of its byte
+#pragma unroll
+        for (int j = 0; j < 8; ++j) m[j] = c.code[(mw[0] >> (8 * (j >> 1) + ((j & 1) ? 0 : 4))) & 15u] * ms_old;
+      } else {
+        i8_decode4(mw[0], ms_old, m);
+        i8_decode4(mw[1], ms_old, m + 4);
+      }
+#pragma unroll
+      for (int j = 0; j < NV; ++j) v[j] = c.vlut[(vw[j >> 2] >> (8 * (j & 3))) & 0xFFu] * vs_old;
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        p[j] = j < cnt ? load1<PD>(t.p, e0 + j) : 0.0f;
-        g[j] = j < cnt ? load1<GD>(t.g, e0 + j) : 0.0f;
-      }
-    }
-    if constexpr (NF4) {
-      uint32_t codes[8];
-      if (full) {
-        const uint32_t w = __builtin_nontemporal_load((const uint32_t*)((const uint8_t*)t.m + (e0 >> 1)));
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const uint32_t byte = (w >> (8 * b)) & 0xFFu;
-          codes[2 * b] = byte >> 4;
-          codes[2 * b + 1] = byte & 15u;
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const uint32_t byte = j < cnt ? ((const uint8_t*)t.m)[(e0 + j) >> 1] : 0x77u;
-          codes[j] = ((e0 + j) & 1) ? (byte & 15u) : (byte >> 4);
+        const bool ok = j < cnt;
+        p[j] = ok ? load1<PD>(t.p, e0 + j) : 0.0f;
+        g[j] = ok ? load1<GD>(t.g, e0 + j) : 0.0f;
+        if constexpr (NF4) {
+          const uint32_t byte = ok ? ((const uint8_t*)t.m)[(e0 + j) >> 1] : 0x77u;
+          m[j] = c.code[((e0 + j) & 1) ? (byte & 15u) : (byte >> 4)] * ms_old;
+        } else {
+          m[j] = ok ? (float)((const int8_t*)t.m)[e0 + j] * ms_old : 0.0f;
         }
       }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) m[j] = c.code[codes[j]] * ms_old;
-    } else {
-      if (full) {
-        const u32x2 w = __builtin_nontemporal_load((const u32x2*)((const int8_t*)t.m + e0));
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const uint32_t word = j < 4 ? w.x : w.y;
-          m[j] = (float)(int8_t)((word >> (8 * (j & 3))) & 0xFFu) * ms_old;
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) m[j] = j < cnt ? (float)((const int8_t*)t.m)[e0 + j] * ms_old : 0.0f;
-      }
-    }
-    if constexpr (QUAD) {
-      uint32_t vc[2];
-      if (full) {
-        const uint32_t w = __builtin_nontemporal_load((const uint16_t*)((const uint8_t*)t.v + (e0 >> 2)));
-        vc[0] = w & 0xFFu;
-        vc[1] = (w >> 8) & 0xFFu;
-      } else {
-        vc[0] = cnt >= 4 ? ((const uint8_t*)t.v)[e0 >> 2] : 0u;
-        vc[1] = cnt >= 8 ? ((const uint8_t*)t.v)[(e0 >> 2) + 1] : 0u;
-      }
-      v[0] = c.vlut[vc[0]] * vs_old;
-      v[1] = c.vlut[vc[1]] * vs_old;
-    } else {
-      if (full) {
-        const u32x2 w = __builtin_nontemporal_load((const u32x2*)((const uint8_t*)t.v + e0));
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = c.vlut[((j < 4 ? w.x : w.y) >> (8 * (j & 3))) & 0xFFu] * vs_old;
+      if constexpr (QUAD) {
+        v[0] = c.vlut[cnt >= 4 ? ((const uint8_t*)t.v)[e0 >> 2] : 0u] * vs_old;
+        v[1] = c.vlut[cnt >= 8 ? ((const uint8_t*)t.v)[(e0 >> 2) + 1] : 0u] * vs_old;
       } else {
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = j < cnt ? c.vlut[((const uint8_t*)t.v)[e0 + j]] * vs_old : 0.0f;
       }
     }
     // ---- update
-    uint32_t h[8];
-    float mean[8];
-    q8_means8(c, t, e0, mean);
+    if (sr) {
+      const uint32_t key = rng_key(hp.seed, tix, hp.step, 1u, (uint32_t)(start >> 32));
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      h[j] = sr ? rng_at(key, (uint32_t)(e0 + j)) : 0u;
-      if constexpr (SINGLE) {
-        m[j] = fmaf(hp.one_minus_beta1, g[j], m[j] * hp.beta1);
-      } else {
-        g[j] = q8_grad<GD>(g[j], tflags, c, mean[j]);
-        m[j] = lerp_to(m[j], g[j], hp.lerp_coef, hp.flags & APEXW_HP_LERP_HI);
-      }
+      for (int j = 0; j < 8; ++j) h[j] = rng_at(key, (uint32_t)(e0 + j));
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) h[j] = 0u;
     }
     float num[8];
+    if constexpr (SINGLE) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float look = SINGLE ? fmaf(hp.one_minus_beta1, g[j], m[j] * hp.beta1)
-                                : lerp_to(g[j], m[j], hp.look_coef, hp.flags & APEXW_HP_LOOK_HI);
-      num[j] = look * ((m[j] * g[j] >= 0.0f) ? c.gain_hi : c.gain_lo);
+      for (int j = 0; j < 8; ++j) {
+        m[j] = fmaf(hp.one_minus_beta1, g[j], m[j] * hp.beta1);
+        num[j] = fmaf(hp.one_minus_beta1, g[j], m[j] * hp.beta1);
+      }
+    } else {
+      float mean[8];
+      q8_means8(c, t, e0, mean);
+      q8_prep8<GD>(g, tflags, c, mean);
+      lerp8(m, g, m, hp.lerp_coef, hp.flags & APEXW_HP_LERP_HI);
+      lerp8(g, m, num, hp.look_coef, hp.flags & APEXW_HP_LOOK_HI);
     }
-    float dens[8] = {1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f};  // SINGLE: denominators
-    float upd[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) num[j] *= (m[j] * g[j] >= 0.0f) ? c.gain_hi : c.gain_lo;
+    // second moments: vr as computed (the per-parameter update divides by it), v what is stored
+    float vr[NV];
     if constexpr (QUAD) {
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
-        if (4 * q >= cnt) break;
         const int b = 4 * q;
         float s = g[b] * g[b];
         s = s + g[b + 1] * g[b + 1];
         s = s + g[b + 2] * g[b + 2];
         s = s + g[b + 3] * g[b + 3];
-        float vq = fmaf(hp.one_minus_beta2, s * 0.25f, v[q] * hp.beta2);
-        if constexpr (SINGLE) {
-          // the update sees v as computed; the quantizer's nan_to_num only affects the stored codes
-          const float den = sqrtf(vq) + hp.eps_scaled;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) dens[b + i] = den;
-        }
-        if (!(fabsf(vq) <= 3.402823466e38f)) vq = 0.0f;  // nan_to_num(0, 0, 0)
-        v[q] = vq;
-        const float den = fmaxf(sqrtf(vq) + hp.eps_scaled, hp.eps);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) upd[b + i] = (num[b + i] / den) * hp.step_size;
+        vr[q] = fmaf(hp.one_minus_beta2, s * 0.25f, v[q] * hp.beta2);
       }
     } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        float vf = fmaf(hp.one_minus_beta2 * g[j], g[j], v[j] * hp.beta2);
-        if constexpr (SINGLE) dens[j] = sqrtf(vf) + hp.eps_scaled;
-        if (!(fabsf(vf) <= 3.402823466e38f)) vf = 0.0f;
-        v[j] = vf;
-        const float den = fmaxf(sqrtf(vf) + hp.eps_scaled, hp.eps);
-        upd[j] = (num[j] / den) * hp.step_size;
-      }
+      for (int j = 0; j < 8; ++j) vr[j] = fmaf(hp.one_minus_beta2 * g[j], g[j], v[j] * hp.beta2);
     }
+#pragma unroll
+    for (int j = 0; j < NV; ++j) v[j] = (fabsf(vr[j]) <= 3.402823466e38f) ? vr[j] : 0.0f;  // nan_to_num(0, 0, 0)
     if constexpr (SINGLE) {
       // p.mul_(wd) (fp32, on a float copy for 16-bit p), p.addcdiv_(num, den, -step_size),
       // then SR or round-to-nearest into a 16-bit parameter
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
+        const float den = sqrtf(vr[QUAD ? j >> 2 : j]) + hp.eps_scaled;
         const float pp = (tflags & APEXW_FLAG_WD) ? p[j] * hp.wd_factor : p[j];
-        const float x = pp + (-hp.step_size * num[j]) / dens[j];
+        const float x = pp + (-hp.step_size * num[j]) / den;
         if constexpr (PD == APEXW_F32) p[j] = x;
         else p[j] = sr ? sr_round<PD>(x, h[j]) : rnd<PD>(x);
       }
-    } else if constexpr (PD == APEXW_F32) {
-      if (generic) {
-        // p.mul_(decay); p.addcdiv_(num, den, value=-step_size)
+    } else {
+      // generic fp32 rows: p.mul_(decay); p.addcdiv_(num, den, value=-step_size)
+      const bool addcdiv = PD == APEXW_F32 && generic;
+      if (addcdiv) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          float pp = (tflags & APEXW_FLAG_WD) ? p[j] * hp.wd_factor : p[j];
-          const float den = QUAD ? fmaxf(sqrtf(v[j >> 2]) + hp.eps_scaled, hp.eps)
-                                 : fmaxf(sqrtf(v[j]) + hp.eps_scaled, hp.eps);
-          p[j] = pp + (-hp.step_size * num[j]) / den;
+        for (int j = 0; j < 8; ++j) num[j] *= -hp.step_size;
+      }
+      float q[8];
+      bool ieee = !(hp.eps_scaled >= kFastEps && hp.eps >= kFastEps);
+      if (!ieee) {
+        float den[NV];
+#pragma unroll
+        for (int j = 0; j < NV; ++j) den[j] = fmaxf(sqrt_shared(v[j]) + hp.eps_scaled, hp.eps);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j] = div_once(num[j], den[QUAD ? j >> 2 : j]);
+        ieee = q8_any_nonfinite8(q);   // an overflowing quotient (rare)
+      }
+      if (ieee) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j] = num[j] / fmaxf(sqrtf(v[QUAD ? j >> 2 : j]) + hp.eps_scaled, hp.eps);
+      }
+      if (addcdiv) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) p[j] = ((tflags & APEXW_FLAG_WD) ? p[j] * hp.wd_factor : p[j]) + q[j];
+      } else if (PD == APEXW_BF16 && generic && !(QUAD && sr)) {
+        // p.mul_(decay), then p -= bf16(update), each rounded: q8_param's generic order in pairs
+        if (tflags & APEXW_FLAG_WD) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) p[j] = p[j] * hp.wd_factor;
+          rnd8<PD>(p);
         }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j] = q[j] * hp.step_size;
+        rnd8<PD>(q);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) p[j] = p[j] - q[j];
+        rnd8<PD>(p);
       } else {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) p[j] = q8_param<PD>(p[j], upd[j], hp.wd_factor, tflags, sr, QUAD, h[j]);
+        for (int j = 0; j < 8; ++j)
+          p[j] = q8_param<PD>(p[j], q[j] * hp.step_size, hp.wd_factor, tflags, sr, QUAD, h[j]);
       }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) p[j] = q8_param<PD>(p[j], upd[j], hp.wd_factor, tflags, sr, QUAD, h[j]);
     }
     if (full) {
       store8<PD>(t.p, e0, p);
@@ -489,116 +584,100 @@ APEXW_DEV void q8_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, const
         if (j < cnt) store1<PD>(t.p, e0 + j, p[j]);
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (j < cnt) {
-        mnew[k][j] = m[j];
-        amax = fmaxf(amax, fabsf(m[j]));
-      }
-    }
-    if constexpr (QUAD) {
-      vnew[k][0] = v[0];
-      vnew[k][1] = cnt >= 8 ? v[1] : 0.0f;
-      vmax = fmaxf(vmax, fmaxf(vnew[k][0], vnew[k][1]));
-    } else {
+    for (int j = 0; j < 8; ++j)
+      if (j < cnt) amax = fmaxf(amax, fabsf(m[j]));
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        if (j < cnt) {
-          vnew[k][j] = v[j];
-          vmax = fmaxf(vmax, v[j]);
-        }
-      }
+    for (int j = 0; j < NV; ++j) {
+      // a second moment of quad rows counts where its four elements are all there
+      if (QUAD ? 4 * (j + 1) <= cnt : j < cnt) vmax = fmaxf(vmax, v[j]);
     }
   }
   // ---- block scales (EMA-max smoothing against the previous scales)
-  amax = wave_max(amax);
-  vmax = wave_max(vmax);
+  block_max2(amax, vmax, red);
   float ms = fmaxf(amax, 1e-12f);
   if (!NF4) ms = ms / 127.0f;
   if (NF4 || !SINGLE) ms = fmaxf(ms, ms_old * 0.9f);
   float vs = fmaxf(vmax, 1e-12f);
   vs = fmaxf(vs, vs_old * 0.95f);
-  if (lane == 0) {
+  if (threadIdx.x == 0) {
     t.m_scale[blk] = ms;
     t.v_scale[blk] = vs;
   }
+  if (!cnt) return;
   // ---- requantize
+  float mq[8], vq[NV];
+  if (ms < 1e30f && vs < 1e30f) {   // both at least 1e-12 / 127: normal reciprocals
+    const float rms = rcp_refined(ms), rvs = rcp_refined(vs);
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int64_t rel = (int64_t)(k * 64 + lane) * 8;
-    const int cnt = rel >= cnt_blk ? 0 : (int)((cnt_blk - rel) < 8 ? (cnt_blk - rel) : 8);
-    if (cnt == 0) continue;
-    const int64_t e0 = start + rel;
-    const bool full = vec && cnt == 8;
+    for (int j = 0; j < 8; ++j) mq[j] = div_shared(m[j], ms, rms);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) vq[j] = div_shared(v[j], vs, rvs);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) mq[j] = m[j] / ms;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) vq[j] = v[j] / vs;
+  }
+  if constexpr (NF4) {
     uint32_t mc[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const uint32_t r = sr ? (rng_at(key, (uint32_t)(e0 + j)) >> 16) : 0u;
-      if constexpr (NF4) {
-        const float x = fminf(fmaxf(mnew[k][j] / ms, -1.0f), 1.0f);
-        mc[j] = sr ? nf4_sr(x, unit_uniform(r), c.code) : nf4_rne_tab(x, c.midtab);
-      } else {
-        float y = mnew[k][j] / ms;
-        if (sr && !SINGLE) y = y + (unit_uniform(r) - 0.5f);
-        y = fminf(fmaxf(rintf(y), -127.0f), 127.0f);
-        mc[j] = (uint32_t)(int32_t)y & 0xFFu;
-      }
+      const float x = fminf(fmaxf(mq[j], -1.0f), 1.0f);
+      mc[j] = sr ? nf4_sr(x, unit_uniform(h[j] >> 16), c.code) : nf4_rne_tab(x, c.midtab);
     }
-    if constexpr (NF4) {
-      if (full) {
-        uint32_t w = 0;
+    if (full) {
+      uint32_t w = 0;
 #pragma unroll
-        for (int b = 0; b < 4; ++b) w |= ((mc[2 * b] << 4) | mc[2 * b + 1]) << (8 * b);
-        __builtin_nontemporal_store(w, (uint32_t*)((uint8_t*)t.m + (e0 >> 1)));
-      } else {
-        // element pairs (2i, 2i+1) share a byte; e0 is even, odd tails pad with code 7
+      for (int b = 0; b < 4; ++b) w |= ((mc[2 * b] << 4) | mc[2 * b + 1]) << (8 * b);
+      __builtin_nontemporal_store(w, APEXW_GLOBAL(uint32_t, (uint8_t*)t.m + (e0 >> 1)));
+    } else {
+      // element pairs (2i, 2i+1) share a byte; e0 is even, odd tails pad with code 7
 #pragma unroll
-        for (int j = 0; j < 8; j += 2) {
-          if (j < cnt) {
-            const uint32_t lo = (j + 1 < cnt) ? mc[j + 1] : 7u;
-            ((uint8_t*)t.m)[(e0 + j) >> 1] = (uint8_t)((mc[j] << 4) | lo);
-          }
+      for (int j = 0; j < 8; j += 2) {
+        if (j < cnt) {
+          const uint32_t lo = (j + 1 < cnt) ? mc[j + 1] : 7u;
+          ((uint8_t*)t.m)[(e0 + j) >> 1] = (uint8_t)((mc[j] << 4) | lo);
         }
       }
-    } else {
-      if (full) {
-        u32x2 w = {mc[0] | (mc[1] << 8) | (mc[2] << 16) | (mc[3] << 24),
-                   mc[4] | (mc[5] << 8) | (mc[6] << 16) | (mc[7] << 24)};
-        __builtin_nontemporal_store(w, (u32x2*)((int8_t*)t.m + e0));
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (j < cnt) ((uint8_t*)t.m)[e0 + j] = (uint8_t)mc[j];
-      }
     }
-    if constexpr (QUAD) {
-      uint32_t vc[2];
+  } else {
+    if (sr && !SINGLE) {
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const uint32_t r = sr ? rng_at(keyv, (uint32_t)((e0 >> 2) + q)) : 0u;
-        vc[q] = logu8_code(vnew[k][q], vs, sr, r);
-      }
-      if (full) {
-        __builtin_nontemporal_store((uint16_t)(vc[0] | (vc[1] << 8)), (uint16_t*)((uint8_t*)t.v + (e0 >> 2)));
-      } else {
-        if (cnt >= 4) ((uint8_t*)t.v)[e0 >> 2] = (uint8_t)vc[0];
-        if (cnt >= 8) ((uint8_t*)t.v)[(e0 >> 2) + 1] = (uint8_t)vc[1];
-      }
+      for (int j = 0; j < 8; ++j) mq[j] = mq[j] + half_noise(h[j]);
+    }
+    const u32x2 w = {i8_encode4(mq), i8_encode4(mq + 4)};
+    if (full) {
+      __builtin_nontemporal_store(w, APEXW_GLOBAL(u32x2, (int8_t*)t.m + e0));
     } else {
-      uint32_t vc[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const uint32_t r = sr ? rng_at(keyv, (uint32_t)(e0 + j)) : 0u;
-        vc[j] = logu8_code(vnew[k][j], vs, sr, r);
-      }
-      if (full) {
-        u32x2 w = {vc[0] | (vc[1] << 8) | (vc[2] << 16) | (vc[3] << 24),
-                   vc[4] | (vc[5] << 8) | (vc[6] << 16) | (vc[7] << 24)};
-        __builtin_nontemporal_store(w, (u32x2*)((uint8_t*)t.v + e0));
-      } else {
+      for (int j = 0; j < 8; ++j)
+        if (j < cnt) ((uint8_t*)t.m)[e0 + j] = (uint8_t)((j < 4 ? w.x : w.y) >> (8 * (j & 3)));
+    }
+  }
+  const uint32_t keyv = sr ? rng_key(hp.seed, tix, hp.step, 2u, (uint32_t)(start >> 32)) : 0u;
+  uint32_t vc[NV];
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (j < cnt) ((uint8_t*)t.v)[e0 + j] = (uint8_t)vc[j];
-      }
+  for (int j = 0; j < NV; ++j) {
+    const uint32_t at = QUAD ? (uint32_t)((e0 >> 2) + j) : (uint32_t)(e0 + j);
+    vc[j] = logu8_code(v[j], vq[j], sr, sr ? rng_at(keyv, at) : 0u);
+  }
+  if constexpr (QUAD) {
+    if (full) {
+      __builtin_nontemporal_store((uint16_t)(vc[0] | (vc[1] << 8)),
+                                  APEXW_GLOBAL(uint16_t, (uint8_t*)t.v + (e0 >> 2)));
+    } else {
+      if (cnt >= 4) ((uint8_t*)t.v)[e0 >> 2] = (uint8_t)vc[0];
+      if (cnt >= 8) ((uint8_t*)t.v)[(e0 >> 2) + 1] = (uint8_t)vc[1];
+    }
+  } else {
+    if (full) {
+      u32x2 w = {vc[0] | (vc[1] << 8) | (vc[2] << 16) | (vc[3] << 24),
+                 vc[4] | (vc[5] << 8) | (vc[6] << 16) | (vc[7] << 24)};
+      __builtin_nontemporal_store(w, APEXW_GLOBAL(u32x2, (uint8_t*)t.v + e0));
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (j < cnt) ((uint8_t*)t.v)[e0 + j] = (uint8_t)vc[j];
     }
   }
 }
@@ -1062,8 +1141,8 @@ APEXW_DEV void q8_block_fast(const apexw_tensor& t, uint32_t tix, uint32_t blk, 
 
 // Dense m and v (bf16 or fp32): the fallback branch of _step_ultra
 // (optimizer.py:4688-4735) for 8-bit tensors under 64 elements and the small
-// tensors of precision "ultra" (fp32 m/v).  One 2048-element unit per wave,
-// one element per lane at a time (these tensors are small).
+// tensors of precision "ultra" (fp32 m/v).  One 2048-element unit per workgroup,
+// one element per thread at a time (these tensors are small).
 // SINGLE: the per-parameter in-backward update of such a tensor
 // (apexw/optimizer.py:2458-2471): p.mul_(wd) in the parameter dtype, fp32
 // moments, p.addcdiv_ rounded once, m and v rounded once on store.
@@ -1073,7 +1152,7 @@ APEXW_DEV void q8_dense(const apexw_tensor& t, uint32_t unit, const Q8Ctx& c) {
   const apexw_hparams& hp = *c.hp;
   const int64_t start = (int64_t)unit * 2048;
   const int64_t end = (t.n - start) < 2048 ? t.n : start + 2048;
-  for (int64_t i = start + lane_id(); i < end; i += 64) {
+  for (int64_t i = start + threadIdx.x; i < end; i += blockDim.x) {
     float p = load1<PD>(t.p, i);
     if constexpr (SINGLE) {
       const float g = load1<GD>(t.g, i);
@@ -1104,46 +1183,45 @@ APEXW_DEV void q8_dense(const apexw_tensor& t, uint32_t unit, const Q8Ctx& c) {
   }
 }
 
-// Precision "ultra" (optimizer.py:4640-4686): one INT8 block of m per wave
-// (t.block = 2048 or 256 elements, scales EMA-max smoothed as for 8-bit) and a
-// dense v in VD.  m = lerp(dequant(m), g, 1 - beta1); v = beta2 v + (1 - beta2) g^2
-// in fp32, stored rounded to VD; the denominator sqrt(v) + eps_scaled comes from
-// the unrounded v, with no eps floor and no lookahead gain; p is decayed (rounded
-// to its dtype), then p - update rounded to p's dtype.
+// Precision "ultra" (optimizer.py:4640-4686): one INT8 block of m per workgroup
+// (t.block = 2048 or 256 elements, scales EMA-max smoothed as for 8-bit; 8 elements per
+// thread) and a dense v in VD.  m = lerp(dequant(m), g, 1 - beta1); v = beta2 v +
+// (1 - beta2) g^2 in fp32, stored rounded to VD; the denominator sqrt(v) + eps_scaled
+// comes from the unrounded v, with no eps floor and no lookahead gain; p is decayed
+// (rounded to its dtype), then p - update rounded to p's dtype.
+// Bound by vector issue when every quotient, root and scale division was an IEEE
+// sequence and one wave held a block's 32 elements per lane (134 VGPRs): four Llama
+// layers (0.87 B bf16 parameters, 10.5 GB) 2610 -> 2013 us per step, 5.2 TB/s.
 template <int PD, int VD>
-APEXW_DEV void ultra_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, const Q8Ctx& c) {
+APEXW_DEV void ultra_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, const Q8Ctx& c, float* red) {
   constexpr int GD = PD;
   const apexw_hparams& hp = *c.hp;
   const bool sr = hp.flags & APEXW_HP_SR;
-  const bool vec = !(t.flags & APEXW_FLAG_SCALAR);
   const int64_t bs = t.block;
   const int64_t start = (int64_t)blk * bs;
   const int64_t cnt_blk = (t.n - start) < bs ? (t.n - start) : bs;
-  const int lane = lane_id();
   const float ms_old = t.m_scale[blk];
-  const uint32_t key = rng_key(hp.seed, tix, hp.step, 1u, (uint32_t)(start >> 32));
-  float mnew[4][8];
-  float amax = 0.0f;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int64_t rel = (int64_t)(k * 64 + lane) * 8;
-    const int cnt = rel >= cnt_blk ? 0 : (int)((cnt_blk - rel) < 8 ? (cnt_blk - rel) : 8);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) mnew[k][j] = 0.0f;
-    if (cnt == 0) continue;
-    const int64_t e0 = start + rel;
-    const bool full = vec && cnt == 8;
-    float p[8], g[8], m[8], v[8];
+  const int64_t rel = (int64_t)threadIdx.x * 8;
+  const int cnt = rel >= cnt_blk ? 0 : (int)((cnt_blk - rel) < 8 ? (cnt_blk - rel) : 8);
+  const int64_t e0 = start + rel;
+  const bool full = !(t.flags & APEXW_FLAG_SCALAR) && cnt == 8;
+  float m[8];
+  float amax = 0.0f, none = 0.0f;
+  if (cnt) {
+    float p[8], g[8], v[8];
     if (full) {
-      load8<PD>(t.p, e0, p);
-      load8<GD>(t.g, e0, g);
-      load8<VD>(t.v, e0, v);
-      const u32x2 w = __builtin_nontemporal_load((const u32x2*)((const int8_t*)t.m + e0));
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const uint32_t word = j < 4 ? w.x : w.y;
-        m[j] = (float)(int8_t)((word >> (8 * (j & 3))) & 0xFFu) * ms_old;
-      }
+      Raw8<PD> rp;
+      Raw8<GD> rg;
+      Raw8<VD> rv;
+      raw_load8<PD>(t.p, e0, rp);
+      raw_load8<GD>(t.g, e0, rg);
+      raw_load8<VD>(t.v, e0, rv);
+      const u32x2 w = __builtin_nontemporal_load(APEXW_GLOBAL(const u32x2, (const int8_t*)t.m + e0));
+      unpack8<PD>(rp, p);
+      unpack8<GD>(rg, g);
+      unpack8<VD>(rv, v);
+      i8_decode4(w.x, ms_old, m);
+      i8_decode4(w.y, ms_old, m + 4);
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -1156,160 +1234,87 @@ APEXW_DEV void ultra_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, co
     }
     float mean[8];
     q8_means8(c, t, e0, mean);
+    q8_prep8<GD>(g, t.flags, c, mean);
+    if (t.flags & APEXW_FLAG_WD) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) p[j] = p[j] * hp.wd_factor;
+      rnd8<PD>(p);
+    }
+    float num[8], vf[8];
+    lerp8(m, g, m, hp.lerp_coef, hp.flags & APEXW_HP_LERP_HI);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      g[j] = q8_grad<GD>(g[j], t.flags, c, mean[j]);
-      if (t.flags & APEXW_FLAG_WD) p[j] = rnd<PD>(p[j] * hp.wd_factor);
-      m[j] = lerp_to(m[j], g[j], hp.lerp_coef, hp.flags & APEXW_HP_LERP_HI);
-      const float vf = fmaf(hp.one_minus_beta2 * g[j], g[j], v[j] * hp.beta2);
-      v[j] = rnd<VD>(vf);
-      // Nesterov: torch.lerp(g, m, beta1) on the fp32 m (optimizer.py:4667-4670)
-      float num = (hp.flags & APEXW_HP_NESTEROV)
-                      ? lerp_to(g[j], m[j], hp.look_coef, hp.flags & APEXW_HP_LOOK_HI) : m[j];
-      // cautious: num * (mask / mean(mask)), mask = num g >= 0 (optimizer.py:4672-4675)
-      if (hp.flags & APEXW_HP_CAUTIOUS) num = num * ((num * g[j] >= 0.0f) ? c.gain_hi : 0.0f);
-      const float upd = (num / (sqrtf(vf) + hp.eps_scaled)) * hp.step_size;
-      if constexpr (PD == APEXW_F32) p[j] = p[j] - upd;
-      else p[j] = rnd<PD>(p[j] - rnd<PD>(upd));
+      num[j] = m[j];
+      vf[j] = fmaf(hp.one_minus_beta2 * g[j], g[j], v[j] * hp.beta2);
     }
+    if (hp.flags & APEXW_HP_NESTEROV) {
+      // torch.lerp(g, m, beta1) on the fp32 m (optimizer.py:4667-4670)
+      lerp8(g, m, num, hp.look_coef, hp.flags & APEXW_HP_LOOK_HI);
+    }
+    if (hp.flags & APEXW_HP_CAUTIOUS) {
+      // num * (mask / mean(mask)), mask = num g >= 0 (optimizer.py:4672-4675)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) num[j] = num[j] * ((num[j] * g[j] >= 0.0f) ? c.gain_hi : 0.0f);
+    }
+    float q[8];
+    bool ieee = !(hp.eps_scaled >= kFastEps);
+    if (!ieee) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = div_once(num[j], sqrt_shared(vf[j]) + hp.eps_scaled);
+      ieee = q8_any_nonfinite8(q);   // an overflowed second moment or quotient (rare)
+    }
+    if (ieee) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = num[j] / (sqrtf(vf[j]) + hp.eps_scaled);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) q[j] = q[j] * hp.step_size;
+    rnd8<PD>(q);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) p[j] = p[j] - q[j];
     if (full) {
-      store8<PD>(t.p, e0, p);
-      store8<VD>(t.v, e0, v);
+      store8_rnd<PD>(t.p, e0, p);
+      store8_rnd<VD>(t.v, e0, vf);
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         if (j < cnt) {
-          store1<PD>(t.p, e0 + j, p[j]);
-          store1<VD>(t.v, e0 + j, v[j]);
+          store1<PD>(t.p, e0 + j, rnd<PD>(p[j]));
+          store1<VD>(t.v, e0 + j, rnd<VD>(vf[j]));
         }
       }
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (j < cnt) {
-        mnew[k][j] = m[j];
-        amax = fmaxf(amax, fabsf(m[j]));
-      }
-    }
+    for (int j = 0; j < 8; ++j)
+      if (j < cnt) amax = fmaxf(amax, fabsf(m[j]));
   }
   // the block scale and the INT8 codes, as the 8-bit step's (quantize_blockwise_int8)
-  amax = wave_max(amax);
+  block_max2(amax, none, red);
   const float ms = fmaxf(fmaxf(amax, 1e-12f) / 127.0f, ms_old * 0.9f);
-  if (lane == 0) t.m_scale[blk] = ms;
+  if (threadIdx.x == 0) t.m_scale[blk] = ms;
+  if (!cnt) return;
+  const uint32_t key = sr ? rng_key(hp.seed, tix, hp.step, 1u, (uint32_t)(start >> 32)) : 0u;
+  float y[8];
+  if (ms < 1e30f) {
+    const float rms = rcp_refined(ms);
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int64_t rel = (int64_t)(k * 64 + lane) * 8;
-    const int cnt = rel >= cnt_blk ? 0 : (int)((cnt_blk - rel) < 8 ? (cnt_blk - rel) : 8);
-    if (cnt == 0) continue;
-    const int64_t e0 = start + rel;
-    uint32_t mc[8];
+    for (int j = 0; j < 8; ++j) y[j] = div_shared(m[j], ms, rms);
+  } else {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float y = mnew[k][j] / ms;
-      if (sr) y = y + (unit_uniform(rng_at(key, (uint32_t)(e0 + j)) >> 16) - 0.5f);
-      y = fminf(fmaxf(rintf(y), -127.0f), 127.0f);
-      mc[j] = (uint32_t)(int32_t)y & 0xFFu;
-    }
-    if (vec && cnt == 8) {
-      u32x2 w = {mc[0] | (mc[1] << 8) | (mc[2] << 16) | (mc[3] << 24),
-                 mc[4] | (mc[5] << 8) | (mc[6] << 16) | (mc[7] << 24)};
-      __builtin_nontemporal_store(w, (u32x2*)((int8_t*)t.m + e0));
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (j < cnt) ((uint8_t*)t.m)[e0 + j] = (uint8_t)mc[j];
-    }
+    for (int j = 0; j < 8; ++j) y[j] = m[j] / ms;
   }
-}
-
-
-// A whole 2048-element "ultra" block (the arithmetic of ultra_block): the loads of
-// KB of the wave's four 8-element groups per lane are issued before their
-// arithmetic (all four for bf16 p and v, two at a time when p or v is fp32), so the
-// block waits on memory once or twice instead of four times.
-template <int PD, int VD>
-APEXW_DEV void ultra_block_full(const apexw_tensor& t, uint32_t tix, uint32_t blk, const Q8Ctx& c) {
-  constexpr int GD = PD;
-  constexpr int KB = (PD == APEXW_F32 || VD == APEXW_F32) ? 2 : 4;
-  const apexw_hparams& hp = *c.hp;
-  const bool sr = hp.flags & APEXW_HP_SR;
-  const bool wd = t.flags & APEXW_FLAG_WD;
-  const int64_t start = (int64_t)blk * 2048;
-  const int lane = lane_id();
-  const float ms_old = t.m_scale[blk];
-  const uint32_t key = rng_key(hp.seed, tix, hp.step, 1u, (uint32_t)(start >> 32));
-  float mnew[4][8];
-  float amax = 0.0f;
+  if (sr) {
 #pragma unroll
-  for (int k0 = 0; k0 < 4; k0 += KB) {
-    Raw8<PD> rp[KB];
-    Raw8<GD> rg[KB];
-    Raw8<VD> rv[KB];
-    u32x2 rm[KB];
-#pragma unroll
-    for (int b = 0; b < KB; ++b) {
-      const int64_t e0 = start + (int64_t)((k0 + b) * 64 + lane) * 8;
-      raw_load8<PD>(t.p, e0, rp[b]);
-      raw_load8<GD>(t.g, e0, rg[b]);
-      raw_load8<VD>(t.v, e0, rv[b]);
-      rm[b] = __builtin_nontemporal_load(APEXW_GLOBAL(const u32x2, (const int8_t*)t.m + e0));
-    }
-#pragma unroll
-    for (int b = 0; b < KB; ++b) {
-      const int k = k0 + b;
-      const int64_t e0 = start + (int64_t)(k * 64 + lane) * 8;
-      float p[8], g[8], v[8];
-      unpack8<PD>(rp[b], p);
-      unpack8<GD>(rg[b], g);
-      unpack8<VD>(rv[b], v);
-      float mean[8];
-      q8_means8(c, t, e0, mean);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const uint32_t word = j < 4 ? rm[b].x : rm[b].y;
-        const float m = (float)(int8_t)((word >> (8 * (j & 3))) & 0xFFu) * ms_old;
-        g[j] = q8_grad<GD>(g[j], t.flags, c, mean[j]);
-        if (wd) p[j] = rnd<PD>(p[j] * hp.wd_factor);
-        mnew[k][j] = lerp_to(m, g[j], hp.lerp_coef, hp.flags & APEXW_HP_LERP_HI);
-        amax = fmaxf(amax, fabsf(mnew[k][j]));
-        const float vf = fmaf(hp.one_minus_beta2 * g[j], g[j], v[j] * hp.beta2);
-        v[j] = rnd<VD>(vf);
-        float num = (hp.flags & APEXW_HP_NESTEROV)
-                        ? lerp_to(g[j], mnew[k][j], hp.look_coef, hp.flags & APEXW_HP_LOOK_HI) : mnew[k][j];
-        if (hp.flags & APEXW_HP_CAUTIOUS) num = num * ((num * g[j] >= 0.0f) ? c.gain_hi : 0.0f);
-        const float upd = (num / (sqrtf(vf) + hp.eps_scaled)) * hp.step_size;
-        if constexpr (PD == APEXW_F32) p[j] = p[j] - upd;
-        else p[j] = rnd<PD>(p[j] - rnd<PD>(upd));
-      }
-      store8<PD>(t.p, e0, p);
-      store8<VD>(t.v, e0, v);
-    }
+    for (int j = 0; j < 8; ++j) y[j] = y[j] + half_noise(rng_at(key, (uint32_t)(e0 + j)));
   }
-  amax = wave_max(amax);
-  const float ms = fmaxf(fmaxf(amax, 1e-12f) / 127.0f, ms_old * 0.9f);
-  if (lane == 0) t.m_scale[blk] = ms;
+  const u32x2 w = {i8_encode4(y), i8_encode4(y + 4)};
+  if (full) {
+    __builtin_nontemporal_store(w, APEXW_GLOBAL(u32x2, (int8_t*)t.m + e0));
+  } else {
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int64_t e0 = start + (int64_t)(k * 64 + lane) * 8;
-    uint32_t mc[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float y = mnew[k][j] / ms;
-      if (sr) y = y + (unit_uniform(rng_at(key, (uint32_t)(e0 + j)) >> 16) - 0.5f);
-      y = fminf(fmaxf(rintf(y), -127.0f), 127.0f);
-      mc[j] = (uint32_t)(int32_t)y & 0xFFu;
-    }
-    u32x2 w = {mc[0] | (mc[1] << 8) | (mc[2] << 16) | (mc[3] << 24),
-               mc[4] | (mc[5] << 8) | (mc[6] << 16) | (mc[7] << 24)};
-    __builtin_nontemporal_store(w, (u32x2*)((int8_t*)t.m + e0));
+    for (int j = 0; j < 8; ++j)
+      if (j < cnt) ((uint8_t*)t.m)[e0 + j] = (uint8_t)((j < 4 ? w.x : w.y) >> (8 * (j & 3)));
   }
-}
-
-template <int PD, int VD>
-APEXW_DEV void ultra_unit(const apexw_tensor& t, uint32_t tix, uint32_t blk, const Q8Ctx& c) {
-  const bool whole = t.block == 2048 && (int64_t)(blk + 1) * 2048 <= t.n && !(t.flags & APEXW_FLAG_SCALAR);
-  if (whole) ultra_block_full<PD, VD>(t, tix, blk, c);
-  else ultra_block<PD, VD>(t, tix, blk, c);
 }
 
 // Dense m / v rows by dtype: m in the parameter's compact dtype (bf16; fp16 for fp16
@@ -1361,9 +1366,10 @@ __global__ __launch_bounds__(256) void ultra_step_kernel(const apexw_tensor* __r
   c.coef = (hp.flags & APEXW_HP_CLIP) ? *hp.clip_coef : 1.0f;
   c.gc_means = nullptr;
   c.gc_rl = 0;
-  const uint32_t wave = uniform(threadIdx.x >> 6);
-  const int64_t stride = (int64_t)gridDim.x * kWaves;
-  for (int64_t u = (int64_t)blockIdx.x * kWaves + wave; u < n_units; u += stride) {
+  // block_max2's two buffers, exchanged after each unit that meets its barrier
+  __shared__ float s_red[2][8];
+  int par = 0;
+  for (int64_t u = blockIdx.x; u < n_units; u += gridDim.x) {
     const apexw_unit un = units[u];
     const apexw_tensor& t = tensors[un.tensor];
     q8_set_rows(c, t, un.tensor);
@@ -1375,17 +1381,19 @@ __global__ __launch_bounds__(256) void ultra_step_kernel(const apexw_tensor* __r
     if (f & APEXW_FLAG_DENSE) {
       dense_dispatch<false>(t, un.unit, c, pd, md, vd);
     } else if (f & APEXW_FLAG_ULTRA) {
+      // (the flags are the workgroup's: every wave takes the same branch)
       // v in the parameter's compact dtype (fp16 for fp16 parameters, else bf16) or fp32
       if (pd == APEXW_F32) {
-        if (vd == APEXW_F32) ultra_unit<APEXW_F32, APEXW_F32>(t, un.tensor, un.unit, c);
-        else ultra_unit<APEXW_F32, APEXW_BF16>(t, un.tensor, un.unit, c);
+        if (vd == APEXW_F32) ultra_block<APEXW_F32, APEXW_F32>(t, un.tensor, un.unit, c, s_red[par]);
+        else ultra_block<APEXW_F32, APEXW_BF16>(t, un.tensor, un.unit, c, s_red[par]);
       } else if (pd == APEXW_BF16) {
-        if (vd == APEXW_F32) ultra_unit<APEXW_BF16, APEXW_F32>(t, un.tensor, un.unit, c);
-        else ultra_unit<APEXW_BF16, APEXW_BF16>(t, un.tensor, un.unit, c);
+        if (vd == APEXW_F32) ultra_block<APEXW_BF16, APEXW_F32>(t, un.tensor, un.unit, c, s_red[par]);
+        else ultra_block<APEXW_BF16, APEXW_BF16>(t, un.tensor, un.unit, c, s_red[par]);
       } else {
-        if (vd == APEXW_F32) ultra_unit<APEXW_F16, APEXW_F32>(t, un.tensor, un.unit, c);
-        else ultra_unit<APEXW_F16, APEXW_F16>(t, un.tensor, un.unit, c);
+        if (vd == APEXW_F32) ultra_block<APEXW_F16, APEXW_F32>(t, un.tensor, un.unit, c, s_red[par]);
+        else ultra_block<APEXW_F16, APEXW_F16>(t, un.tensor, un.unit, c, s_red[par]);
       }
+      par ^= 1;
     }
   }
 }
@@ -1486,9 +1494,10 @@ __global__ __launch_bounds__(256) void q8_step_kernel(const apexw_tensor* __rest
   c.coef = (hp.flags & APEXW_HP_CLIP) ? *hp.clip_coef : 1.0f;
   c.gc_means = nullptr;
   c.gc_rl = 0;
-  const uint32_t wave = uniform(threadIdx.x >> 6);
-  const int64_t stride = (int64_t)gridDim.x * kWaves;
-  for (int64_t u = (int64_t)blockIdx.x * kWaves + wave; u < n_units; u += stride) {
+  // block_max2's two buffers, exchanged after each unit that meets its barrier
+  __shared__ float s_red[2][8];
+  int par = 0;
+  for (int64_t u = blockIdx.x; u < n_units; u += gridDim.x) {
     const apexw_unit un = units[u];
     const apexw_tensor& t = tensors[un.tensor];
     q8_set_rows(c, t, un.tensor);
@@ -1505,18 +1514,19 @@ __global__ __launch_bounds__(256) void q8_step_kernel(const apexw_tensor* __rest
     if (f & APEXW_FLAG_ULTRA) continue;
     const bool nf4 = f & APEXW_FLAG_NF4, quad = f & APEXW_FLAG_QUAD;
     if (pd == APEXW_F32) {
-      if (nf4 && quad) q8_block<APEXW_F32, true, true, SINGLE>(t, un.tensor, un.unit, c);
-      else if (nf4) q8_block<APEXW_F32, true, false, SINGLE>(t, un.tensor, un.unit, c);
-      else q8_block<APEXW_F32, false, false, SINGLE>(t, un.tensor, un.unit, c);
+      if (nf4 && quad) q8_block<APEXW_F32, true, true, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
+      else if (nf4) q8_block<APEXW_F32, true, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
+      else q8_block<APEXW_F32, false, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
     } else if (pd == APEXW_BF16) {
-      if (nf4 && quad) q8_block<APEXW_BF16, true, true, SINGLE>(t, un.tensor, un.unit, c);
-      else if (nf4) q8_block<APEXW_BF16, true, false, SINGLE>(t, un.tensor, un.unit, c);
-      else q8_block<APEXW_BF16, false, false, SINGLE>(t, un.tensor, un.unit, c);
+      if (nf4 && quad) q8_block<APEXW_BF16, true, true, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
+      else if (nf4) q8_block<APEXW_BF16, true, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
+      else q8_block<APEXW_BF16, false, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
     } else {
-      if (nf4 && quad) q8_block<APEXW_F16, true, true, SINGLE>(t, un.tensor, un.unit, c);
-      else if (nf4) q8_block<APEXW_F16, true, false, SINGLE>(t, un.tensor, un.unit, c);
-      else q8_block<APEXW_F16, false, false, SINGLE>(t, un.tensor, un.unit, c);
+      if (nf4 && quad) q8_block<APEXW_F16, true, true, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
+      else if (nf4) q8_block<APEXW_F16, true, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
+      else q8_block<APEXW_F16, false, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
     }
+    par ^= 1;
   }
 }
 
@@ -1625,13 +1635,15 @@ bool apexw_q8_flags_ok(uint32_t flags, uint32_t block, int64_t n) {
 
 int apexw_launch_q8(const apexw_tensor* tensors, int64_t n_units, const apexw_unit* units,
                     const apexw_hparams* hp, hipStream_t stream) {
-  if (hp->mode == APEXW_MODE_SINGLE) {
-    const int grid = apexw_resident_grid((const void*)q8_step_kernel<true>, n_units);
+  // a unit per workgroup at a time (fewer workgroups, each walking more units, measured no
+  // faster: 87 -> 90 us for 25 M parameters with 2 instead of 16 per resident slot)
+  const bool single = hp->mode == APEXW_MODE_SINGLE;
+  const void* kernel = single ? (const void*)q8_step_kernel<true> : (const void*)q8_step_kernel<false>;
+  const int grid = apexw_resident_grid(kernel, n_units * kWaves);
+  if (single)
     hipLaunchKernelGGL(q8_step_kernel<true>, dim3(grid), dim3(256), 0, stream, tensors, units, n_units, *hp);
-  } else {
-    const int grid = apexw_resident_grid((const void*)q8_step_kernel<false>, n_units);
+  else
     hipLaunchKernelGGL(q8_step_kernel<false>, dim3(grid), dim3(256), 0, stream, tensors, units, n_units, *hp);
-  }
   return hipGetLastError() == hipSuccess ? APEXW_OK : APEXW_ERR_LAUNCH;
 }
 
@@ -1649,7 +1661,7 @@ int apexw_launch_q8_cautious_count(const apexw_tensor* tensors, int32_t n_tensor
 
 int apexw_launch_ultra(const apexw_tensor* tensors, int64_t n_units, const apexw_unit* units,
                        const apexw_hparams* hp, hipStream_t stream) {
-  const int grid = apexw_resident_grid((const void*)ultra_step_kernel, n_units);
+  const int grid = apexw_resident_grid((const void*)ultra_step_kernel, n_units * kWaves);
   hipLaunchKernelGGL(ultra_step_kernel, dim3(grid), dim3(256), 0, stream, tensors, units, n_units, *hp);
   return hipGetLastError() == hipSuccess ? APEXW_OK : APEXW_ERR_LAUNCH;
 }
