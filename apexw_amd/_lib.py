@@ -126,6 +126,17 @@ GEMM_PROBLEM_DTYPE = np.dtype([
     ("wd_factor", np.float32), ("neg_lr", np.float32), ("reserved2", np.uint32),
 ])
 assert GEMM_PROBLEM_DTYPE.itemsize == 120
+# apexw_gemm_launch: one grouped launch of a sequence (apexw_gemm_nt_grouped_run)
+GEMM_LAUNCH_DTYPE = np.dtype([("problems", np.uint64), ("items", np.uint64), ("queue_offsets", np.uint64),
+                              ("n_workgroups", np.int32), ("kind", np.int32)])
+assert GEMM_LAUNCH_DTYPE.itemsize == 32
+# apexw_muon_item: one matrix of a grouped momentum / work-matrix preparation
+MUON_ITEM_DTYPE = np.dtype([("buf", np.uint64), ("g", np.uint64), ("x", np.uint64), ("xt", np.uint64),
+                            ("partial", np.uint64), ("rows", np.int64), ("cols", np.int64), ("ldx", np.int64),
+                            ("ldxt", np.int64), ("mu", np.float32), ("one_minus_mu", np.float32),
+                            ("g_dtype", np.uint32), ("layout", np.uint32), ("nesterov", np.uint32),
+                            ("reserved", np.uint32)])
+assert MUON_ITEM_DTYPE.itemsize == 96
 _GEMM_APPLY_ZERO = (0, 0, 0, 0, 0.0, 0.0, 0)
 
 
@@ -184,6 +195,10 @@ SIGNATURES = {
     "apexw_muon_workspace_floats": (ctypes.c_int64, [_i64, _i64]),
     "apexw_muon_prepare": (ctypes.c_int, [_vp, _vp, _i32, _i64, _i64, _f32, _f32, _i32, _f32, _f32, _vp, _vp, _i64,
                                           _i64, _i32, _vp, _vp, _vp]),
+    "apexw_gemm_nt_grouped_run": (ctypes.c_int, [_vp, _i32, _vp, _vp]),
+    "apexw_check_muon_items": (ctypes.c_int, [_vp, _i32]),
+    "apexw_muon_prepare_units": (ctypes.c_int64, [_i64, _i64, _i32]),
+    "apexw_muon_prepare_grouped": (ctypes.c_int, [_vp, _i32, _vp, _i64, _vp, _i64, _f32, _f32, _vp, _vp]),
     "apexw_muon_apply": (ctypes.c_int, [_vp, _i32, _vp, _i64, _i64, _i64, _i32, _i32, _f32, _i32, _f32, _vp, _vp]),
     "apexw_factored_layout": (ctypes.c_int64, [_vp, _i32, ctypes.POINTER(ctypes.c_int64),
                                                ctypes.POINTER(ctypes.c_int64)]),

@@ -29,7 +29,7 @@ bool apexw_compact_flags_ok(uint32_t flags);
 int apexw_launch_gemm_nt(const uint16_t*, const uint16_t*, const uint16_t*, uint16_t*, uint16_t*, int32_t, int32_t,
                          int32_t, int32_t, int32_t, int32_t, int32_t, int32_t, int32_t, int64_t, int64_t, int64_t,
                          int64_t, int64_t, float, float, hipStream_t);
-int apexw_muon_partials(int64_t n);
+int64_t apexw_muon_units(int64_t rows, int64_t cols, bool tiles);
 int apexw_launch_muon_coordwise(float*, const void*, int32_t, void*, int32_t, int64_t, float, float, int32_t, float,
                                 float, int32_t, float, const apexw_amp_dyn*, hipStream_t);
 int apexw_launch_grad_prep(const apexw_grad_prep*, const apexw_unit*, int64_t, float, uint32_t, const apexw_amp_dyn*,
@@ -38,8 +38,8 @@ int apexw_launch_row_means(const apexw_grad_prep*, const apexw_unit*, int64_t, f
                            bool, hipStream_t);
 int apexw_launch_gemm_grouped(const apexw_gemm_problem*, const uint32_t*, const int32_t*, int32_t, int32_t,
                               const apexw_amp_dyn*, hipStream_t);
-int apexw_launch_muon_prepare(float*, const void*, int32_t, int64_t, int64_t, float, float, int32_t, float, float,
-                              uint16_t*, uint16_t*, int64_t, int64_t, bool, float*, const apexw_amp_dyn*, hipStream_t);
+int apexw_launch_muon_prepare(const apexw_muon_item*, const apexw_muon_item*, const apexw_unit*, int64_t,
+                              const apexw_unit*, int64_t, float, float, const apexw_amp_dyn*, hipStream_t);
 int apexw_launch_muon_apply(void*, int32_t, const uint16_t*, int64_t, int64_t, int64_t, bool, int32_t, float, int32_t,
                             float, const apexw_amp_dyn*, hipStream_t);
 bool apexw_q8_flags_ok(uint32_t flags, uint32_t block, int64_t n);
@@ -531,37 +531,104 @@ int apexw_gemm_grouped_schedule(const apexw_gemm_problem* problems, int32_t n_pr
   return APEXW_OK;
 }
 
-int apexw_gemm_nt_grouped(const apexw_gemm_problem* problems, const uint32_t* items, const int32_t* queue_offsets,
-                          int32_t n_workgroups, int32_t kind, const apexw_amp_dyn* amp, void* stream) {
+namespace {
+
+int check_grouped(const apexw_gemm_problem* problems, const uint32_t* items, const int32_t* queue_offsets,
+                  int32_t n_workgroups, int32_t kind, const apexw_amp_dyn* amp) {
   if (!problems || !items || !queue_offsets) return APEXW_ERR_ARG;
   if ((uintptr_t)amp & 15u) return APEXW_ERR_ALIGN;
   if (n_workgroups <= 0 || n_workgroups % APEXW_GEMM_QUEUES) return APEXW_ERR_ARG;
   if (kind <= 0 || kind > 31 || !(kind & (APEXW_GEMM_OUT_C | APEXW_GEMM_OUT_CT))) return APEXW_ERR_ARG;
   if ((kind & APEXW_GEMM_KIND_NN) && (kind & APEXW_GEMM_OUT_CT)) return APEXW_ERR_ARG;
   if (((uintptr_t)problems | (uintptr_t)items | (uintptr_t)queue_offsets) & 3u) return APEXW_ERR_ALIGN;
+  return APEXW_OK;
+}
+
+}  // namespace
+
+int apexw_gemm_nt_grouped(const apexw_gemm_problem* problems, const uint32_t* items, const int32_t* queue_offsets,
+                          int32_t n_workgroups, int32_t kind, const apexw_amp_dyn* amp, void* stream) {
+  const int st = check_grouped(problems, items, queue_offsets, n_workgroups, kind, amp);
+  if (st != APEXW_OK) return st;
   return apexw_launch_gemm_grouped(problems, items, queue_offsets, n_workgroups, kind, amp, (hipStream_t)stream);
 }
 
+int apexw_gemm_nt_grouped_run(const apexw_gemm_launch* launches, int32_t n_launches, const apexw_amp_dyn* amp,
+                              void* stream) {
+  if (!launches || n_launches < 0) return APEXW_ERR_ARG;
+  for (int32_t i = 0; i < n_launches; ++i) {
+    const apexw_gemm_launch& l = launches[i];
+    const int st = check_grouped(l.problems, l.items, l.queue_offsets, l.n_workgroups, l.kind, amp);
+    if (st != APEXW_OK) return st;
+  }
+  for (int32_t i = 0; i < n_launches; ++i) {
+    const apexw_gemm_launch& l = launches[i];
+    const int st = apexw_launch_gemm_grouped(l.problems, l.items, l.queue_offsets, l.n_workgroups, l.kind, amp,
+                                             (hipStream_t)stream);
+    if (st != APEXW_OK) return st;
+  }
+  return APEXW_OK;
+}
+
 int64_t apexw_muon_workspace_floats(int64_t rows, int64_t cols) {
-  return rows > 0 && cols > 0 ? apexw_muon_partials(rows * cols) : 0;
+  return rows > 0 && cols > 0 ? apexw_muon_units(rows, cols, false) : 0;
+}
+
+namespace {
+
+int check_muon_item(const apexw_muon_item& t) {
+  if (!t.buf || !t.g || !t.x || !t.partial || t.rows <= 0 || t.cols <= 0 || t.nesterov > 1 || t.reserved)
+    return APEXW_ERR_ARG;
+  if (t.g_dtype != APEXW_F32 && t.g_dtype != APEXW_BF16 && t.g_dtype != APEXW_F16) return APEXW_ERR_DTYPE;
+  if (t.layout != APEXW_LAYOUT_ROWS && t.layout != APEXW_LAYOUT_PANEL) return APEXW_ERR_ARG;
+  // work matrix X is [min x max], X^T is [max x min] (optional)
+  const int64_t lo = t.rows < t.cols ? t.rows : t.cols, hi = t.rows < t.cols ? t.cols : t.rows;
+  if (t.ldx < hi || (t.xt && t.ldxt < lo)) return APEXW_ERR_ARG;
+  if (t.layout == APEXW_LAYOUT_PANEL && ((t.ldx & 31) || (t.xt && (t.ldxt & 31)))) return APEXW_ERR_ALIGN;
+  // one workgroup per 64 x 64 tile, the grid's x extent
+  if (apexw_muon_units(t.rows, t.cols, true) > INT32_MAX) return APEXW_ERR_ARG;
+  return APEXW_OK;
+}
+
+}  // namespace
+
+int apexw_check_muon_items(const apexw_muon_item* items, int32_t n_items) {
+  if (!items || n_items <= 0) return APEXW_ERR_ARG;
+  for (int32_t i = 0; i < n_items; ++i) {
+    const int st = check_muon_item(items[i]);
+    if (st != APEXW_OK) return st;
+  }
+  return APEXW_OK;
+}
+
+int64_t apexw_muon_prepare_units(int64_t rows, int64_t cols, int32_t which) {
+  if (rows <= 0 || cols <= 0 || which < 0 || which > 1) return -APEXW_ERR_ARG;
+  return apexw_muon_units(rows, cols, which == 1);
 }
 
 int apexw_muon_prepare(float* buf, const void* g, int32_t g_dtype, int64_t rows, int64_t cols, float mu,
                        float one_minus_mu, int32_t nesterov, float eps, float grad_inv_scale, void* x, void* xt,
                        int64_t ldx, int64_t ldxt, int32_t layout, float* workspace, const apexw_amp_dyn* amp,
                        void* stream) {
-  if (!buf || !g || !x || !workspace || rows <= 0 || cols <= 0) return APEXW_ERR_ARG;
   if ((uintptr_t)amp & 15u) return APEXW_ERR_ALIGN;
-  if (g_dtype != APEXW_F32 && g_dtype != APEXW_BF16 && g_dtype != APEXW_F16) return APEXW_ERR_DTYPE;
-  if (layout != APEXW_LAYOUT_ROWS && layout != APEXW_LAYOUT_PANEL) return APEXW_ERR_ARG;
-  // work matrix X is [min x max], X^T is [max x min] (optional)
-  const int64_t lo = rows < cols ? rows : cols, hi = rows < cols ? cols : rows;
-  if (ldx < hi || (xt && ldxt < lo)) return APEXW_ERR_ARG;
-  if (layout == APEXW_LAYOUT_PANEL && ((ldx & 31) || (xt && (ldxt & 31)))) return APEXW_ERR_ALIGN;
+  const apexw_muon_item one{buf, g, x, xt, workspace, rows, cols, ldx, ldxt, mu, one_minus_mu, (uint32_t)g_dtype,
+                            (uint32_t)layout, nesterov ? 1u : 0u, 0u};
+  const int st = check_muon_item(one);
+  if (st != APEXW_OK) return st;
   if (!amp && !(grad_inv_scale > 0.0f)) return APEXW_ERR_ARG;
-  return apexw_launch_muon_prepare(buf, g, g_dtype, rows, cols, mu, one_minus_mu, nesterov, eps, grad_inv_scale,
-                                   (uint16_t*)x, (uint16_t*)xt, ldx, ldxt, layout == APEXW_LAYOUT_PANEL, workspace,
-                                   amp, (hipStream_t)stream);
+  return apexw_launch_muon_prepare(nullptr, &one, nullptr, apexw_muon_units(rows, cols, false), nullptr,
+                                   apexw_muon_units(rows, cols, true), eps, grad_inv_scale, amp, (hipStream_t)stream);
+}
+
+int apexw_muon_prepare_grouped(const apexw_muon_item* items, int32_t n_items, const apexw_unit* units_m,
+                               int64_t n_units_m, const apexw_unit* units_x, int64_t n_units_x, float eps,
+                               float grad_inv_scale, const apexw_amp_dyn* amp, void* stream) {
+  if (!items || !units_m || !units_x || n_items <= 0 || n_units_m <= 0 || n_units_x <= 0) return APEXW_ERR_ARG;
+  if (n_units_m > INT32_MAX || n_units_x > INT32_MAX) return APEXW_ERR_ARG;
+  if (((uintptr_t)amp & 15u) || ((uintptr_t)items & 7u)) return APEXW_ERR_ALIGN;
+  if (!amp && !(grad_inv_scale > 0.0f)) return APEXW_ERR_ARG;
+  return apexw_launch_muon_prepare(items, nullptr, units_m, n_units_m, units_x, n_units_x, eps, grad_inv_scale, amp,
+                                   (hipStream_t)stream);
 }
 
 int apexw_muon_apply(void* p, int32_t p_dtype, const void* u, int64_t rows, int64_t cols, int64_t ldu,

@@ -591,103 +591,207 @@ APEXW_DEV float nesterov_source(float g, float m, float mu) {
   return mu < 0.5f ? fmaf(mu, m - g, g) : fmaf(mu - 1.0f, m - g, m);
 }
 
-// VEC: 8 elements per thread with 16-byte accesses (buf and grad 16-byte
-// aligned); the n % 8 tail and unaligned tensors take the element-wise loop.
-template <int GD, bool VEC>
-__global__ __launch_bounds__(256) void muon_momentum_kernel(float* __restrict__ buf, const void* __restrict__ grad,
-                                                            int64_t n, float mu, float one_minus_mu, int nesterov,
-                                                            float inv, float* __restrict__ partial,
+// The matrices of a preparation launch: a device table with unit tables, or, for a
+// single matrix, one item passed by value (items == nullptr; the unit is the workgroup).
+struct PrepArgs {
+  const apexw_muon_item* items;
+  const apexw_unit* units;
+  apexw_muon_item one;
+};
+APEXW_DEV uint32_t prep_item(const PrepArgs& a, apexw_muon_item& it) {
+  if (!a.items) {
+    it = a.one;
+    return blockIdx.x;
+  }
+  const apexw_unit u = a.units[blockIdx.x];
+  it = a.items[u.tensor];
+  return u.unit;
+}
+
+// Momentum: a workgroup takes one chunk of a matrix (at most kMuonChunks chunks, so
+// that the second pass sums a matrix's partials with one load per thread), two
+// 8-element vectors per thread in flight with 16-byte accesses where buf and grad are
+// aligned for them; the n % 8 tail and unaligned tensors element by element.  Bound by
+// memory, or for small matrices by the launch: one launch for all of a step's matrices
+// (the 48 matrices of GPT-2-small, 85 M elements: 309 us in 48 launches, 171 us here).
+constexpr int64_t kMuonChunks = 256, kMuonChunkMin = 2048;
+__host__ __device__ inline int64_t muon_chunk(int64_t n) {
+  return (n + kMuonChunks * kMuonChunkMin - 1) / (kMuonChunks * kMuonChunkMin) * kMuonChunkMin;
+}
+
+template <int GD>
+APEXW_DEV float muon_momentum_chunk(const apexw_muon_item& it, uint32_t chunk, float inv) {
+  const int64_t n = it.rows * it.cols, size = muon_chunk(n), lo = chunk * size;
+  const int64_t hi = lo + size < n ? lo + size : n;
+  const bool vec = (((uintptr_t)it.buf | (uintptr_t)it.g) & 15u) == 0;
+  const float mu = it.mu, one_minus_mu = it.one_minus_mu;
+  const bool nesterov = it.nesterov;
+  float s = 0.0f;
+  const int64_t v_end = vec ? hi / 8 * 8 : lo;   // lo is a multiple of 8
+  auto update = [&](float (&g)[8], float (&m)[8], int64_t i) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (inv != 1.0f) g[j] = rnd<GD>(g[j] * inv);
+      if (__builtin_isnan(g[j])) g[j] = 0.0f;
+      else if (__builtin_isinf(g[j])) g[j] = g[j] > 0.0f ? 65504.0f : -65504.0f;
+      m[j] = fmaf(one_minus_mu, g[j], m[j] * mu);
+      const float x = rnd<APEXW_BF16>(nesterov ? nesterov_source(g[j], m[j], mu) : m[j]);
+      s = fmaf(x, x, s);
+    }
+    store8<APEXW_F32>(it.buf, i, m);
+  };
+  int64_t i = lo + (int64_t)threadIdx.x * 8;
+  for (; i + 2048 < v_end; i += 4096) {
+    float g[2][8], m[2][8];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      load8<GD>(it.g, i + q * 2048, g[q]);
+      load8<APEXW_F32>(it.buf, i + q * 2048, m[q]);
+    }
+    update(g[0], m[0], i);
+    update(g[1], m[1], i + 2048);
+  }
+  if (i < v_end) {
+    float g[8], m[8];
+    load8<GD>(it.g, i, g);
+    load8<APEXW_F32>(it.buf, i, m);
+    update(g, m, i);
+  }
+  for (i = v_end + threadIdx.x; i < hi; i += 256) {
+    const float g = muon_grad<GD>(it.g, i, inv);
+    const float m = fmaf(one_minus_mu, g, APEXW_GLOBAL(float, it.buf)[i] * mu);
+    APEXW_GLOBAL(float, it.buf)[i] = m;
+    const float x = rnd<APEXW_BF16>(nesterov ? nesterov_source(g, m, mu) : m);
+    s = fmaf(x, x, s);
+  }
+  return s;
+}
+
+__global__ __launch_bounds__(256) void muon_momentum_kernel(PrepArgs a, float inv,
                                                             const apexw_amp_dyn* __restrict__ amp) {
   if (amp) {
     if (amp->skip) return;
     inv = amp->grad_inv_scale;
   }
-  float s = 0.0f;
-  const int64_t tid = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
-  const int64_t n_vec = VEC ? n / 8 * 8 : 0;
-  if constexpr (VEC) {
-    for (int64_t i = tid * 8; i < n_vec; i += stride * 8) {
-      float g[8], m[8];
-      load8<GD>(grad, i, g);
-      load8<APEXW_F32>(buf, i, m);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        if (inv != 1.0f) g[j] = rnd<GD>(g[j] * inv);
-        if (__builtin_isnan(g[j])) g[j] = 0.0f;
-        else if (__builtin_isinf(g[j])) g[j] = g[j] > 0.0f ? 65504.0f : -65504.0f;
-        m[j] = fmaf(one_minus_mu, g[j], m[j] * mu);
-        const float x = rnd<APEXW_BF16>(nesterov ? nesterov_source(g[j], m[j], mu) : m[j]);
-        s = fmaf(x, x, s);
-      }
-      store8<APEXW_F32>(buf, i, m);
-    }
-  }
-  for (int64_t i = n_vec + tid; i < n; i += stride) {
-    const float g = muon_grad<GD>(grad, i, inv);
-    const float m = fmaf(one_minus_mu, g, APEXW_GLOBAL(float, buf)[i] * mu);
-    APEXW_GLOBAL(float, buf)[i] = m;
-    const float x = rnd<APEXW_BF16>(nesterov ? nesterov_source(g, m, mu) : m);
-    s = fmaf(x, x, s);
-  }
+  apexw_muon_item it;
+  const uint32_t chunk = prep_item(a, it);
+  float s;
+  if (it.g_dtype == APEXW_F32) s = muon_momentum_chunk<APEXW_F32>(it, chunk, inv);
+  else if (it.g_dtype == APEXW_BF16) s = muon_momentum_chunk<APEXW_BF16>(it, chunk, inv);
+  else s = muon_momentum_chunk<APEXW_F16>(it, chunk, inv);
   s = wave_sum(s);
   __shared__ float red[4];
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
-  if (threadIdx.x == 0) partial[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+  if (threadIdx.x == 0) it.partial[chunk] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-// X = bf16(bf16(buf) / d) with d = bf16(bf16(||bf16(buf)||_F) + eps) (the bf16
+// X = bf16(bf16(s) / d) with d = bf16(bf16(||bf16(s)||_F) + eps) (the bf16
 // torch ops of zeropower_via_newtonschulz5), written as the work matrix in both
-// orientations.  The work matrix is buf itself when rows <= cols, else buf^T.
-// 64 x 64 tiles through LDS so both are written along their rows; panel: the
-// outputs are stored in 32 x 32 panels (the grouped GEMM's APEXW_GEMM_PANEL).
+// orientations.  The work matrix is s itself when rows <= cols, else s^T.
+// A workgroup takes a 64 x 64 tile, 8 consecutive elements of a row per thread and half
+// tile; the transposed orientation goes through LDS and leaves as 8 elements of its
+// row.  Every access is 16 bytes where the shapes and pointers allow (32 x 32 panels
+// (APEXW_GEMM_PANEL) always do for the outputs).  Bound by memory; the same 48 matrices:
+// 812 us in 48 launches with 2-byte stores, 131 us here.
 template <int GD>
-__global__ __launch_bounds__(256) void muon_normalize_kernel(const float* __restrict__ buf, const void* __restrict__ grad,
-                                                             int64_t rows, int64_t cols, float mu, int nesterov,
-                                                             float inv, const float* __restrict__ partial, int n_partial,
-                                                             float eps, int tall, uint16_t* __restrict__ x,
-                                                             uint16_t* __restrict__ xt, int64_t ldx, int64_t ldxt,
-                                                             bool panel, const apexw_amp_dyn* __restrict__ amp) {
+APEXW_DEV void muon_source8(const apexw_muon_item& it, int64_t r, int64_t c, bool vec, float inv, float (&v)[8]) {
+  const int64_t i = r * it.cols + c;
+  const int cnt = (int)(it.cols - c < 8 ? it.cols - c : 8);
+  if (vec && cnt == 8) {
+    load8<APEXW_F32>(it.buf, i, v);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = j < cnt ? APEXW_GLOBAL(const float, it.buf)[i + j] : 0.0f;
+  }
+  if (it.nesterov) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (j < cnt) v[j] = nesterov_source(muon_grad<GD>(it.g, i + j, inv), v[j], it.mu);
+  }
+}
+
+// 8 consecutive elements (r, c) .. (r, c + 7) of an output, those below `cnt`
+APEXW_DEV void muon_put8(uint16_t* out, int64_t r, int64_t c, int64_t ld, bool panel, bool vec, int cnt,
+                         const uint32_t (&w)[4]) {
+  uint16_t* dst = out + poff64(r, c, ld, panel);
+  if (vec && cnt == 8) {
+    *APEXW_GLOBAL(u32x4, dst) = u32x4{w[0], w[1], w[2], w[3]};
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    if (j < cnt) APEXW_GLOBAL(uint16_t, dst)[j] = (uint16_t)(w[j >> 1] >> (16 * (j & 1)));
+}
+
+__global__ __launch_bounds__(256) void muon_normalize_kernel(PrepArgs a, float inv, float eps,
+                                                             const apexw_amp_dyn* __restrict__ amp) {
   __shared__ float red[4];
-  __shared__ uint16_t tile[64][66];
+  __shared__ __attribute__((aligned(16))) uint16_t tile[64][72];   // rows of 144 bytes
   if (amp) {
     if (amp->skip) return;
     inv = amp->grad_inv_scale;
   }
-  float s = 0.0f;
-  for (int i = threadIdx.x; i < n_partial; i += 256) s += partial[i];
+  apexw_muon_item it;
+  const uint32_t unit = prep_item(a, it);
+  const int64_t rows = it.rows, cols = it.cols, n = rows * cols;
+  const int n_partial = (int)((n + muon_chunk(n) - 1) / muon_chunk(n));   // at most 256
+  const int tid = threadIdx.x;
+  float s = tid < n_partial ? it.partial[tid] : 0.0f;
+  // this thread's part of tile (tr, tc) of s in its own [rows x cols] layout: 8 columns of
+  // rows r8 and r8 + 32
+  const uint32_t tiles_x = (uint32_t)((cols + 63) / 64);
+  const int64_t tr = (int64_t)(unit / tiles_x) * 64, tc = (int64_t)(unit % tiles_x) * 64;
+  const int r8 = tid >> 3, c8 = (tid & 7) * 8;
+  const bool vec_in = (cols & 7) == 0 && ((uintptr_t)it.buf & 15u) == 0;
+  float v[2][8];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int64_t r = tr + r8 + 32 * h, c = tc + c8;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[h][j] = 0.0f;
+    if (r < rows && c < cols) {
+      if (it.g_dtype == APEXW_F32) muon_source8<APEXW_F32>(it, r, c, vec_in, inv, v[h]);
+      else if (it.g_dtype == APEXW_BF16) muon_source8<APEXW_BF16>(it, r, c, vec_in, inv, v[h]);
+      else muon_source8<APEXW_F16>(it, r, c, vec_in, inv, v[h]);
+    }
+  }
   s = wave_sum(s);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  if ((tid & 63) == 0) red[tid >> 6] = s;
   __syncthreads();
   const float total = (red[0] + red[1]) + (red[2] + red[3]);
   const float d = rnd<APEXW_BF16>(rnd<APEXW_BF16>(sqrtf(total)) + eps);
-  // tile (tr, tc) of buf in its own [rows x cols] layout
-  const int64_t tr = (int64_t)blockIdx.y * 64, tc = (int64_t)blockIdx.x * 64;
-  for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-    const int r = e >> 6, cidx = e & 63;
-    const int64_t gr = tr + r, gc = tc + cidx;
-    float v = 0.0f;
-    if (gr < rows && gc < cols) {
-      const int64_t i = gr * cols + gc;
-      float m = APEXW_GLOBAL(const float, buf)[i];
-      if (nesterov) m = nesterov_source(muon_grad<GD>(grad, i, inv), m, mu);
-      v = rnd<APEXW_BF16>(m) / d;
-    }
-    tile[r][cidx] = to_bf(v);
+  // direct layout D[r][c] = s-shaped; transposed layout T[c][r]; xt may be null (only the
+  // wide work matrix is wanted)
+  const bool tall = rows > cols, panel = it.layout == APEXW_LAYOUT_PANEL;
+  uint16_t* direct = (uint16_t*)(tall ? it.xt : it.x);
+  uint16_t* trans = (uint16_t*)(tall ? it.x : it.xt);
+  const int64_t ld_direct = tall ? it.ldxt : it.ldx, ld_trans = tall ? it.ldx : it.ldxt;
+  const bool vec_d = ((uintptr_t)direct & 15u) == 0 && (ld_direct & 7) == 0;
+  const bool vec_t = ((uintptr_t)trans & 15u) == 0 && (ld_trans & 7) == 0;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int64_t r = tr + r8 + 32 * h, c = tc + c8;
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      w[j] = pack_bf16x2(rnd<APEXW_BF16>(v[h][2 * j]) / d, rnd<APEXW_BF16>(v[h][2 * j + 1]) / d);
+    *(u32x4*)&tile[r8 + 32 * h][c8] = u32x4{w[0], w[1], w[2], w[3]};
+    if (direct && r < rows && c < cols)
+      muon_put8(direct, r, c, ld_direct, panel, vec_d, (int)(cols - c < 8 ? cols - c : 8), w);
   }
+  if (!trans) return;
   __syncthreads();
-  // direct layout D[r][c] = buf-shaped; transposed layout T[c][r]; xt may be
-  // null (only the wide work matrix is wanted)
-  uint16_t* direct = tall ? xt : x;
-  uint16_t* trans = tall ? x : xt;
-  const int64_t ld_direct = tall ? ldxt : ldx, ld_trans = tall ? ldx : ldxt;
-  for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-    const int r = e >> 6, cidx = e & 63;
-    // direct[tr + r][tc + cidx] = D(tr + r, tc + cidx); trans[tc + r][tr + cidx] = D(tr + cidx, tc + r)
-    if (direct && tr + r < rows && tc + cidx < cols)
-      APEXW_GLOBAL(uint16_t, direct)[poff64(tr + r, tc + cidx, ld_direct, panel)] = tile[r][cidx];
-    if (trans && tc + r < cols && tr + cidx < rows)
-      APEXW_GLOBAL(uint16_t, trans)[poff64(tc + r, tr + cidx, ld_trans, panel)] = tile[cidx][r];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    // row tc + cc of the transposed layout, its elements tr + c8 .. + 7
+    const int cc = r8 + 32 * h;
+    const int64_t r = tr + c8, c = tc + cc;
+    if (c >= cols || r >= rows) continue;
+    uint32_t w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = (uint32_t)tile[c8 + 2 * j][cc] | ((uint32_t)tile[c8 + 2 * j + 1][cc] << 16);
+    muon_put8(trans, c, r, ld_trans, panel, vec_t, (int)(rows - r < 8 ? rows - r : 8), w);
   }
 }
 
@@ -892,38 +996,18 @@ int apexw_launch_gemm_grouped(const apexw_gemm_problem* probs, const uint32_t* i
                                         : launch_grouped<false>(probs, items, offsets, n_wg, base, amp, stream);
 }
 
-int apexw_muon_partials(int64_t n) { return grid_for(n) < 1024 ? grid_for(n) : 1024; }
-
-template <int GD>
-void launch_prepare(float* buf, const void* g, int64_t rows, int64_t cols, float mu, float one_minus_mu, int nesterov,
-                    float eps, float inv, uint16_t* x, uint16_t* xt, int64_t ldx, int64_t ldxt, bool panel,
-                    float* partial, const apexw_amp_dyn* amp, hipStream_t stream) {
+int64_t apexw_muon_units(int64_t rows, int64_t cols, bool tiles) {
   const int64_t n = rows * cols;
-  const int nb = apexw_muon_partials(n);
-  if ((((uintptr_t)buf | (uintptr_t)g) & 15u) == 0)
-    hipLaunchKernelGGL((muon_momentum_kernel<GD, true>), dim3(nb), dim3(256), 0, stream, buf, g, n, mu, one_minus_mu,
-                       nesterov, inv, partial, amp);
-  else
-    hipLaunchKernelGGL((muon_momentum_kernel<GD, false>), dim3(nb), dim3(256), 0, stream, buf, g, n, mu, one_minus_mu,
-                       nesterov, inv, partial, amp);
-  dim3 grid((unsigned)((cols + 63) / 64), (unsigned)((rows + 63) / 64));
-  hipLaunchKernelGGL(muon_normalize_kernel<GD>, grid, dim3(256), 0, stream, buf, g, rows, cols, mu, nesterov, inv,
-                     partial, nb, eps, (int)(rows > cols), x, xt, ldx, ldxt, panel, amp);
+  return tiles ? ((rows + 63) / 64) * ((cols + 63) / 64) : (n + muon_chunk(n) - 1) / muon_chunk(n);
 }
 
-int apexw_launch_muon_prepare(float* buf, const void* g, int32_t g_dtype, int64_t rows, int64_t cols, float mu,
-                              float one_minus_mu, int32_t nesterov, float eps, float inv, uint16_t* x, uint16_t* xt,
-                              int64_t ldx, int64_t ldxt, bool panel, float* partial, const apexw_amp_dyn* amp,
-                              hipStream_t stream) {
-  if (g_dtype == APEXW_F32)
-    launch_prepare<APEXW_F32>(buf, g, rows, cols, mu, one_minus_mu, nesterov, eps, inv, x, xt, ldx, ldxt, panel,
-                              partial, amp, stream);
-  else if (g_dtype == APEXW_BF16)
-    launch_prepare<APEXW_BF16>(buf, g, rows, cols, mu, one_minus_mu, nesterov, eps, inv, x, xt, ldx, ldxt, panel,
-                               partial, amp, stream);
-  else
-    launch_prepare<APEXW_F16>(buf, g, rows, cols, mu, one_minus_mu, nesterov, eps, inv, x, xt, ldx, ldxt, panel,
-                              partial, amp, stream);
+// One matrix (items == nullptr, its units the grids) or a step's matrices.
+int apexw_launch_muon_prepare(const apexw_muon_item* items, const apexw_muon_item* one, const apexw_unit* units_m,
+                              int64_t n_m, const apexw_unit* units_x, int64_t n_x, float eps, float inv,
+                              const apexw_amp_dyn* amp, hipStream_t stream) {
+  PrepArgs m{items, units_m, one ? *one : apexw_muon_item{}}, x{items, units_x, one ? *one : apexw_muon_item{}};
+  hipLaunchKernelGGL(muon_momentum_kernel, dim3((unsigned)n_m), dim3(256), 0, stream, m, inv, amp);
+  hipLaunchKernelGGL(muon_normalize_kernel, dim3((unsigned)n_x), dim3(256), 0, stream, x, inv, eps, amp);
   return hipGetLastError() == hipSuccess ? APEXW_OK : APEXW_ERR_LAUNCH;
 }
 

@@ -5,8 +5,8 @@ the fp32-momentum configuration: same constructor, defaults, ``state`` keys
 (``step``, ``work_dtype``, ``momentum``) and ``load_state_dict`` dtype
 handling.  The step runs through libapexw_hip.so:
 
-* ``apexw_muon_prepare``: fp32 momentum update, the bf16 work matrix (the
-  wide orientation) normalised by its Frobenius norm;
+* ``apexw_muon_prepare_grouped``: fp32 momentum update, the bf16 work matrix (the
+  wide orientation) normalised by its Frobenius norm, of every matrix in two launches;
 * ``NSPlan``: per iteration three bf16 MFMA GEMMs
   (``A = X X^T``; ``B = c A A + b A``; ``X = B X + a X``), each one grouped
   launch (``apexw_gemm_nt_grouped``) over every Muon matrix of the step; the
@@ -103,6 +103,9 @@ class NSWorkspace:
         lib = _lib.load()
         per = int(lib.apexw_muon_workspace_floats(m, n))
         self.partial = torch.empty(batch, max(per, 1), dtype=torch.float32, device=device)
+        # per entry the addresses the preparation writes: X, X^T and the norm's partial sums
+        self.rows = [(self.x[0][e].data_ptr(), self.xt[0][e].data_ptr(), self.partial[e].data_ptr())
+                     for e in range(batch)]
 
     def rows_of(self, buf):
         """One matrix of x, a or b as a row-major tensor (a copy when in panels)."""
@@ -166,6 +169,11 @@ class NSPlan:
             self.exec_flops += ws.batch * s * (tri * (2 * ws.mp ** 2 * ws.np_ + 2 * ws.mp ** 3) + 2 * ws.mp ** 2 * ws.np_)
         self.device = device
         self._applied = {}      # id(host table) -> (applies key, device table with the fused update)
+        # the preparation's unit tables (momentum chunks, 64 x 64 tiles) over every matrix, in order
+        self.n_items = sum(ws.batch for ws in wss)
+        self._prep_units = None
+        self._prepared = None   # (bytes of the last item table, its device copy)
+        self._seq = None        # host array of the launch sequence
         built = {}
         self.iters = []
         for i in range(max(steps, default=0)):
@@ -204,20 +212,49 @@ class NSPlan:
         key = None
         if applies is not None:
             key = (tuple(tuple(a) for a in applies), bool(keep_result))
-        for phases in self.iters:
-            for launches in phases:
-                for probs, items, offsets, n_wg, kind, host, fin in launches:
-                    if fin and applies is not None:
-                        # the fused update's table changes only with the parameters' addresses
-                        # or the step's scalars: reuse the last upload while they hold
-                        hit = self._applied.get(id(host))
-                        if hit is not None and hit[0] == key:
-                            probs = hit[1]
-                        else:
-                            probs = self._upload_applies(lib, probs, host, fin, applies, keep_result)
-                            self._applied[id(host)] = (key, probs)
-                    _lib.check(lib.apexw_gemm_nt_grouped(probs.data_ptr(), items.data_ptr(), offsets.data_ptr(),
-                                                         n_wg, kind, amp, stream), "apexw_gemm_nt_grouped")
+        # the tables never move, but for the fused update's, whose rows change with the
+        # parameters' addresses and the step's scalars
+        if self._seq is None:
+            flat = [l for phases in self.iters for launches in phases for l in launches]
+            self._seq = np.array([(p.data_ptr(), i.data_ptr(), o.data_ptr(), n_wg, kind)
+                                  for p, i, o, n_wg, kind, _, _ in flat], dtype=_lib.GEMM_LAUNCH_DTYPE)
+            self._seq_final = [(k, l) for k, l in enumerate(flat) if l[6]]
+        for k, (probs, _, _, _, _, host, fin) in self._seq_final:
+            if applies is not None:
+                hit = self._applied.get(id(host))
+                if hit is None or hit[0] != key:
+                    hit = self._applied[id(host)] = (key, self._upload_applies(lib, probs, host, fin, applies,
+                                                                               keep_result))
+                probs = hit[1]
+            self._seq["problems"][k] = probs.data_ptr()
+        if len(self._seq):
+            _lib.check(lib.apexw_gemm_nt_grouped_run(self._seq.ctypes.data, len(self._seq), amp, stream),
+                       "apexw_gemm_nt_grouped_run")
+
+    def prepare(self, stream, items, inv_scale, amp=None):
+        """Momentum and normalised work matrices of every matrix (MUON_ITEM_DTYPE rows in the
+        plan's order) in two launches."""
+        lib = _lib.load()
+        if self._prep_units is None:
+            tables = []
+            for which in (0, 1):
+                counts = np.array([int(lib.apexw_muon_prepare_units(int(t["rows"]), int(t["cols"]), which))
+                                   for t in items], dtype=np.int64)
+                units = np.zeros(int(counts.sum()), dtype=_lib.UNIT_DTYPE)
+                units["tensor"] = np.repeat(np.arange(len(items), dtype=np.uint32), counts)
+                units["unit"] = np.arange(len(units)) - np.repeat(np.cumsum(counts) - counts, counts)
+                tables.append((torch.from_numpy(units.view(np.uint8)).to(self.device), len(units)))
+            self._prep_units = tables
+        # the item table goes up only when an address or a scalar changed
+        raw = items.tobytes()
+        if self._prepared is None or self._prepared[0] != raw:
+            _lib.check(lib.apexw_check_muon_items(items.ctypes.data, len(items)), "apexw_check_muon_items")
+            staged = torch.from_numpy(items.view(np.uint8)).pin_memory()
+            self._prepared = (raw, staged.to(self.device, non_blocking=True))
+        (um, nm), (ux, nx) = self._prep_units
+        _lib.check(lib.apexw_muon_prepare_grouped(self._prepared[1].data_ptr(), len(items), um.data_ptr(), nm,
+                                                  ux.data_ptr(), nx, NS_EPS, inv_scale, amp, stream),
+                   "apexw_muon_prepare_grouped")
 
     def _upload_applies(self, lib, dev_probs, host, fin, applies, keep_result):
         tbl = host.copy()
@@ -398,7 +435,7 @@ class ApexMuon(Optimizer):
                     shapes[tuple(p.shape)].append(p)
                 for shape, plist in shapes.items():
                     # the reference batches same-shape matrices on the GPU (apexw/muon.py:593-615)
-                    jobs.append(self._prepare(gi, shape, plist, group, inv_scale, amp_ptr))
+                    jobs.append(self._job(gi, shape, plist, group))
             # Newton-Schulz of every matrix, grouped per device; matrices are
             # independent, so running all momenta first and all updates last
             # gives each parameter the result of the reference's per-shape loop
@@ -411,8 +448,11 @@ class ApexMuon(Optimizer):
                 by_dev[j["ws"].device].append(j)
             for dev, djobs in by_dev.items():
                 plan = self._ns_plan(djobs, dev)
+                stream = torch.cuda.current_stream(dev).cuda_stream
+                plan.prepare(stream, np.array([row for j in djobs for row in j["items"]],
+                                              dtype=_lib.MUON_ITEM_DTYPE), inv_scale, amp_ptr)
                 applies = [self._apply_args(j) for j in djobs]
-                plan.run(torch.cuda.current_stream(dev).cuda_stream, applies, self.keep_ns_result, amp_ptr)
+                plan.run(stream, applies, self.keep_ns_result, amp_ptr)
             for j in jobs:
                 if j["steps"] == 0:
                     self._apply(j, amp_ptr)
@@ -487,27 +527,27 @@ class ApexMuon(Optimizer):
         self._amp_unfolded = False
         self._amp_drain(wait=True)
 
-    def _prepare(self, gi, shape, plist, group, inv_scale=1.0, amp=None):
-        """Momentum update and normalised bf16 work matrix (both layouts) of one same-shape batch."""
-        lib = _lib.load()
+    def _job(self, gi, shape, plist, group):
+        """One same-shape batch of a step: its workspace, the momentum update and work
+        matrices to prepare (MUON_ITEM_DTYPE rows), and the tensors its update is written to."""
         p0 = plist[0]
         rows, cols = p0.shape[0], p0.numel() // p0.shape[0]
         m, n = min(rows, cols), max(rows, cols)
         dev = p0.device
-        stream = torch.cuda.current_stream(dev).cuda_stream
         ws = self._workspace((gi, shape, len(plist), dev), m, n, len(plist), dev)
-        mu = float(group["momentum"])
+        mu, nesterov = float(group["momentum"]), int(bool(group["nesterov"]))
+        items, grads = [], []
         for i, p in enumerate(plist):
             st = self._init_param_state(p)
             self._count_step(st)
             g = p.grad if p.grad.is_contiguous() else p.grad.contiguous()
-            _lib.check(lib.apexw_muon_prepare(
-                st["momentum"].data_ptr(), g.data_ptr(), _dtype_code(g.dtype), rows, cols, mu, 1.0 - mu,
-                int(bool(group["nesterov"])), NS_EPS, inv_scale, ws.x[0][i].data_ptr(), ws.xt[0][i].data_ptr(),
-                ws.np_, ws.mp, ws.layout,
-                ws.partial[i].data_ptr(), amp, stream), "apexw_muon_prepare")
+            grads.append(g)     # a contiguous copy lives until the step has been enqueued
+            x, xt, partial = ws.rows[i]
+            items.append((st["momentum"].data_ptr(), g.data_ptr(), x, xt, partial, rows, cols, ws.np_, ws.mp, mu,
+                          1.0 - mu, _dtype_code(g.dtype), ws.layout, nesterov, 0))
         return {"plist": plist, "targets": [self._target(p) for p in plist], "group": group, "ws": ws,
-                "rows": rows, "cols": cols, "steps": int(group["ns_steps"]), "batched": len(plist) > 1}
+                "rows": rows, "cols": cols, "steps": int(group["ns_steps"]), "batched": len(plist) > 1,
+                "items": items, "grads": grads}
 
     def _update_scalars(self, job):
         """(wd_factor, neg_lr, apply_wd) of the decoupled decay and the scaled

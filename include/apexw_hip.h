@@ -663,6 +663,19 @@ int apexw_gemm_grouped_schedule(const apexw_gemm_problem* problems, int32_t n_pr
 int apexw_gemm_nt_grouped(const apexw_gemm_problem* problems, const uint32_t* items, const int32_t* queue_offsets,
                           int32_t n_workgroups, int32_t kind, const apexw_amp_dyn* amp, void* stream);
 
+/* A sequence of grouped launches on one stream (the products of a step's Newton-Schulz
+ * iterations), each as apexw_gemm_nt_grouped; launches: HOST array.  Every launch's
+ * arguments are checked before the first is enqueued. */
+typedef struct apexw_gemm_launch {
+  const apexw_gemm_problem* problems;
+  const uint32_t* items;
+  const int32_t* queue_offsets;
+  int32_t n_workgroups;
+  int32_t kind;
+} apexw_gemm_launch;     /* 32 bytes */
+int apexw_gemm_nt_grouped_run(const apexw_gemm_launch* launches, int32_t n_launches, const apexw_amp_dyn* amp,
+                              void* stream);
+
 /* fp32 workspace (floats) apexw_muon_prepare needs for a [rows x cols] matrix. */
 /* Layout of a Newton-Schulz work matrix in apexw_muon_prepare / apexw_muon_apply:
  * row-major with leading dimension ld, or 32 x 32 panels as APEXW_GEMM_PANEL
@@ -693,6 +706,33 @@ int apexw_muon_prepare(float* buf, const void* g, int32_t g_dtype, int64_t rows,
                        float mu, float one_minus_mu, int32_t nesterov, float eps, float grad_inv_scale,
                        void* x, void* xt, int64_t ldx, int64_t ldxt, int32_t layout, float* workspace,
                        const apexw_amp_dyn* amp, void* stream);
+
+/*
+ * The same for every Muon matrix of a step in two launches (momentum, then work
+ * matrices), replacing one apexw_muon_prepare per matrix.  items: device array, a host
+ * copy checked by apexw_check_muon_items; partial: the item's workspace
+ * (apexw_muon_workspace_floats).  units_m / units_x: device unit tables ({item, index})
+ * of the two launches, each item's apexw_muon_prepare_units indices from 0 up (which = 0:
+ * momentum chunks, 1: 64 x 64 tiles of its [rows x cols] shape).
+ */
+typedef struct apexw_muon_item {
+  float* buf;
+  const void* g;
+  void* x;               /* as apexw_muon_prepare's arguments */
+  void* xt;
+  float* partial;
+  int64_t rows, cols, ldx, ldxt;
+  float mu, one_minus_mu;
+  uint32_t g_dtype;
+  uint32_t layout;
+  uint32_t nesterov;     /* 0 or 1 */
+  uint32_t reserved;     /* 0 */
+} apexw_muon_item;       /* 96 bytes */
+int apexw_check_muon_items(const apexw_muon_item* items, int32_t n_items);
+int64_t apexw_muon_prepare_units(int64_t rows, int64_t cols, int32_t which);
+int apexw_muon_prepare_grouped(const apexw_muon_item* items, int32_t n_items, const apexw_unit* units_m,
+                               int64_t n_units_m, const apexw_unit* units_x, int64_t n_units_x, float eps,
+                               float grad_inv_scale, const apexw_amp_dyn* amp, void* stream);
 
 /*
  * p = round(round(p * wd_factor) + neg_lr_eff * U)   (the decay only if apply_wd)
