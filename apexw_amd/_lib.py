@@ -158,8 +158,9 @@ FV_SUM_COLS = 1
 FV_BAND_ROWS = 32
 FV_UNIT_RANGES = 9   # (bf16, fp32, fp16 parameters) x (INT8, 6-bit, 16-bit m)
 
-GEMM_SYM, GEMM_B_KN, GEMM_ADD_B, GEMM_APPLY, GEMM_APPLY_T, GEMM_APPLY_WD, GEMM_PANEL = 1, 2, 4, 8, 16, 32, 64
-GEMM_OUT_C, GEMM_OUT_CT, GEMM_ADD, GEMM_KIND_NN, GEMM_KIND_PANEL = 1, 2, 4, 8, 16
+GEMM_SYM, GEMM_B_KN, GEMM_ADD_B, GEMM_APPLY, GEMM_APPLY_T, GEMM_APPLY_WD, GEMM_PANEL, GEMM_TILE128 = \
+    1, 2, 4, 8, 16, 32, 64, 128
+GEMM_OUT_C, GEMM_OUT_CT, GEMM_ADD, GEMM_KIND_NN, GEMM_KIND_PANEL, GEMM_KIND_TILE128 = 1, 2, 4, 8, 16, 32
 LAYOUT_ROWS, LAYOUT_PANEL = 0, 1   # Newton-Schulz work matrices: row-major or 32 x 32 panels
 GEMM_MAX_PROBLEMS = 256
 GEMM_QUEUES = 8

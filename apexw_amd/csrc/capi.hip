@@ -346,6 +346,8 @@ namespace {
 
 constexpr int kTile = APEXW_GEMM_TILE;
 
+int problem_tile(const apexw_gemm_problem& p) { return (p.flags & APEXW_GEMM_TILE128) ? 128 : kTile; }
+
 // Epilogue kind of one problem, or minus a status when it is invalid.
 int gemm_problem_kind(const apexw_gemm_problem& p) {
   const bool sym = p.flags & APEXW_GEMM_SYM, kn = p.flags & APEXW_GEMM_B_KN, add_b = p.flags & APEXW_GEMM_ADD_B;
@@ -353,7 +355,10 @@ int gemm_problem_kind(const apexw_gemm_problem& p) {
   const bool add = p.beta != 0.0f;
   if (!p.a || !p.b || (!p.c && !p.ct && !apply)) return -APEXW_ERR_ARG;
   constexpr uint32_t kKnown = APEXW_GEMM_SYM | APEXW_GEMM_B_KN | APEXW_GEMM_ADD_B | APEXW_GEMM_APPLY |
-                              APEXW_GEMM_APPLY_T | APEXW_GEMM_APPLY_WD | APEXW_GEMM_PANEL;
+                              APEXW_GEMM_APPLY_T | APEXW_GEMM_APPLY_WD | APEXW_GEMM_PANEL | APEXW_GEMM_TILE128;
+  const bool small = p.flags & APEXW_GEMM_TILE128;
+  if (small && (kn || !(p.flags & APEXW_GEMM_PANEL))) return -APEXW_ERR_ARG;
+  const int tile = problem_tile(p);
   if ((p.flags & ~kKnown) || p.reserved || p.reserved2) return -APEXW_ERR_ARG;
   if (apply) {
     // the X' product only (X as [K x N] rows, or X^T as the [N x K] operand, which may
@@ -371,8 +376,8 @@ int gemm_problem_kind(const apexw_gemm_problem& p) {
   if (add_b ? (p.et || !add || p.alpha != 1.0f || p.m > p.k) : (add && !p.et)) return -APEXW_ERR_ARG;
   if (kn && (sym || p.ct)) return -APEXW_ERR_ARG;
   if (p.m <= 0 || p.n <= 0 || p.k <= 0) return -APEXW_ERR_ARG;
-  if (p.m % kTile || p.n % kTile || p.k % APEXW_GEMM_KTILE) return -APEXW_ERR_ARG;
-  if (p.m / kTile > 2048 || p.n / kTile > 2048) return -APEXW_ERR_ARG;
+  if (p.m % tile || p.n % tile || p.k % APEXW_GEMM_KTILE) return -APEXW_ERR_ARG;
+  if (p.m / tile > 2048 || p.n / tile > 2048) return -APEXW_ERR_ARG;
   const bool read_e = add && !add_b;
   if (p.lda < p.k || p.ldb < (kn ? p.n : p.k) || (p.c && p.ldc < p.n) || (p.ct && p.ldct < p.m) ||
       (read_e && p.lde < p.m))
@@ -391,11 +396,12 @@ int gemm_problem_kind(const apexw_gemm_problem& p) {
   }
   // the applied update goes through the row-major epilogue (writing c too when given)
   return (p.c || apply ? APEXW_GEMM_OUT_C : 0) | (p.ct ? APEXW_GEMM_OUT_CT : 0) | (add ? APEXW_GEMM_ADD : 0) |
-         (kn ? APEXW_GEMM_KIND_NN : 0) | ((p.flags & APEXW_GEMM_PANEL) ? APEXW_GEMM_KIND_PANEL : 0);
+         (kn ? APEXW_GEMM_KIND_NN : 0) | ((p.flags & APEXW_GEMM_PANEL) ? APEXW_GEMM_KIND_PANEL : 0) |
+         (small ? APEXW_GEMM_KIND_TILE128 : 0);
 }
 
 int64_t gemm_problem_tiles(const apexw_gemm_problem& p) {
-  const int64_t tm = p.m / kTile, tn = p.n / kTile;
+  const int64_t tm = p.m / problem_tile(p), tn = p.n / problem_tile(p);
   return (p.flags & APEXW_GEMM_SYM) ? tm * (tm + 1) / 2 : tm * tn;
 }
 
@@ -471,7 +477,7 @@ int apexw_gemm_grouped_schedule(const apexw_gemm_problem* problems, int32_t n_pr
   int rotate = 0;
   for (int32_t pi = 0; pi < n_problems; ++pi) {
     const apexw_gemm_problem& p = problems[pi];
-    const int tiles_m = p.m / kTile, tiles_n = p.n / kTile;
+    const int tiles_m = p.m / problem_tile(p), tiles_n = p.n / problem_tile(p);
     const bool sym = (p.flags & APEXW_GEMM_SYM) != 0;
     const int64_t kt = p.k / APEXW_GEMM_KTILE;
     const int64_t cost = 20 * (kt + epi), half_cost = 11 * kt + 10 * epi;
@@ -498,7 +504,7 @@ int apexw_gemm_grouped_schedule(const apexw_gemm_problem* problems, int32_t n_pr
     std::vector<Item>& b = band[x];
     std::stable_sort(b.begin(), b.end(), [](const Item& l, const Item& r) { return l.cost > r.cost; });
     size_t split = 0;
-    if (cus_per_queue > 0) {
+    if (cus_per_queue > 0 && !(kind0 & APEXW_GEMM_KIND_TILE128)) {   // small tiles are not split
       int64_t best = -1;
       const size_t most = std::min(b.size(), (size_t)cus_per_queue);
       for (size_t s = 0; s <= most; ++s) {
@@ -538,7 +544,7 @@ int check_grouped(const apexw_gemm_problem* problems, const uint32_t* items, con
   if (!problems || !items || !queue_offsets) return APEXW_ERR_ARG;
   if ((uintptr_t)amp & 15u) return APEXW_ERR_ALIGN;
   if (n_workgroups <= 0 || n_workgroups % APEXW_GEMM_QUEUES) return APEXW_ERR_ARG;
-  if (kind <= 0 || kind > 31 || !(kind & (APEXW_GEMM_OUT_C | APEXW_GEMM_OUT_CT))) return APEXW_ERR_ARG;
+  if (kind <= 0 || kind > 63 || !(kind & (APEXW_GEMM_OUT_C | APEXW_GEMM_OUT_CT))) return APEXW_ERR_ARG;
   if ((kind & APEXW_GEMM_KIND_NN) && (kind & APEXW_GEMM_OUT_CT)) return APEXW_ERR_ARG;
   if (((uintptr_t)problems | (uintptr_t)items | (uintptr_t)queue_offsets) & 3u) return APEXW_ERR_ALIGN;
   return APEXW_OK;

@@ -23,7 +23,6 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) uint16_t u16x4;
 typedef __attribute__((ext_vector_type(4))) short v4i16;
-typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
 
 constexpr int kBM = 256, kBN = 256;
 // K is staged through LDS 32 at a time in kStages rotating buffers of 32 KB
@@ -63,6 +62,8 @@ APEXW_DEV float bf(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 APEXW_DEV uint16_t to_bf(float x) { return (uint16_t)f32_to_bf16_bits(x); }
 
 typedef uint16_t LdsStage[2][kBM * kBK];   // [A | B][256 x 32]
+// Output tiles of a workgroup: 256 x 256, its 128-row halves, or 128 x 128 (APEXW_GEMM_TILE128)
+constexpr int kWhole = 0, kHalfTile = 1, kSmall = 2;
 
 // global -> LDS copy of 16 bytes per lane (global_load_lds_dwordx4): lane L's
 // 16 bytes at gbase + voff land at LDS byte lds_base + 16 L.  Issued as inline
@@ -99,8 +100,8 @@ APEXW_DEV uint32_t lds_address(const void* p) {
 }
 
 // s_waitcnt vmcnt(n) for the n the K loop needs (an immediate operand).
-// Counts are multiples of the copies per stage (8, or 6 for half tiles); any
-// other n waits for the next lower listed count, which is also correct.
+// Counts are multiples of the copies per stage (8, 6 for half tiles, 4 for small
+// ones); any other n waits for the next lower listed count, which is also correct.
 APEXW_DEV void wait_vm(int n) {
   if (n >= 32) asm volatile("s_waitcnt vmcnt(32)" ::: "memory");
   else if (n >= 24) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
@@ -109,6 +110,7 @@ APEXW_DEV void wait_vm(int n) {
   else if (n >= 12) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
   else if (n >= 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
   else if (n >= 6) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+  else if (n >= 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
   else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
@@ -147,11 +149,12 @@ APEXW_DEV void apply_run(const ApplyArgs& ap, int64_t i, const float (&u)[8], in
 }
 
 // One output tile: O = alpha * A B^T + beta * E (bf16 in, fp32 accumulate,
-// bf16 out, round to nearest even), 256 x 256, or 128 x 256 with kHalf (the
-// split tail tiles of a grouped launch).  A and B point at the tile's first row
+// bf16 out, round to nearest even), 256 x 256, 128 x 256 with kHalfTile (the
+// split tail tiles of a grouped launch), or 128 x 128 with kSmall (launches of few
+// tiles: 80 KB of LDS and 64 accumulators, so two workgroups to a CU).  A and B point at the tile's first row
 // of each operand; Et, C and Ct at the tile's origin in their own layouts.  256
-// threads = 4 waves in a 2 x 2 arrangement, each owning a kWM x 128 block
-// (kWM = 128, or 64 with kHalf) as (kWM / 32) x 4 MFMA 32x32x16 accumulators.
+// threads = 4 waves in a 2 x 2 arrangement, each owning a kWM x kWN block
+// as MFMA 32x32x16 accumulators.
 // Template flags select the epilogue: write O row-major (kC), transposed (kCt,
 // skipped at run time when write_ct is false), add beta * E (kAdd).
 //
@@ -185,18 +188,24 @@ APEXW_DEV void apply_run(const ApplyArgs& ap, int64_t i, const float (&u)[8], in
 // beta E with extra MFMAs against a one-hot fragment holding beta on the
 // diagonal (beta split into two bf16 parts, hi + lo, within 2^-18 of beta), so
 // the epilogue reads no addend.
-template <bool kC, bool kCt, bool kAdd, bool kNN, bool kHalf, bool kPanel>
+template <bool kC, bool kCt, bool kAdd, bool kNN, int kShape, bool kPanel>
 APEXW_DEV void gemm_tile(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, int32_t lda, int32_t ldb,
                          int32_t k, const uint16_t* __restrict__ Et, int32_t lde, uint16_t* __restrict__ C,
                          int32_t ldc, uint16_t* __restrict__ Ct, int32_t ldct, bool write_ct, float alpha,
-                         float beta, int32_t diag_k0, const ApplyArgs& ap, LdsStage* lds) {
+                         float beta, int32_t diag_k0, const ApplyArgs& ap, uint16_t* lds) {
   constexpr bool panel = kPanel;   // operands and outputs in 32 x 32 panels (APEXW_GEMM_PANEL)
-  constexpr int kWM = kHalf ? 64 : 128;   // rows of a wave's block
+  constexpr int kWM = kShape == kWhole ? 128 : 64;   // rows of a wave's block
+  constexpr int kWN = kShape == kSmall ? 64 : 128;   // columns of a wave's block
+  static_assert(!(kNN && kShape == kSmall), "small tiles read B as [N x K]");
   constexpr int kFA = kWM / 32;           // A fragments (32-row blocks) per wave and k-step
+  constexpr int kFB = kWN / 32;           // B fragments
   constexpr int kACopies = kWM / 32;      // A copy instructions per wave and stage (16 rows each, 4 waves)
-  constexpr int kCopies = kACopies + 4;   // per stage and wave: A, then the 4 of B
-  constexpr int kFrags = kFA + 4;         // fragment reads per k-step
-  constexpr int kMM = kFA * 4;            // MFMAs per k-step
+  constexpr int kBCopies = kWN / 32;      // B copy instructions
+  constexpr int kCopies = kACopies + kBCopies;
+  constexpr int kFrags = kFA + kFB;       // fragment reads per k-step
+  constexpr int kMM = kFA * kFB;          // MFMAs per k-step
+  // LDS elements of one operand's stage ([256 or 128 rows x 32], kNN B: 32 x 256)
+  constexpr int kOp = (kShape == kSmall ? 128 : 256) * kBK, kStage = 2 * kOp;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
 
@@ -206,7 +215,8 @@ APEXW_DEV void gemm_tile(const uint16_t* __restrict__ A, const uint16_t* __restr
   // rows of 512 bytes, lane L at row 2 q + L / 32, slot L % 32, holding column
   // chunk (L % 32) ^ (4 (row % 4)) (so the transposing reads of 4 consecutive
   // rows hit distinct banks).  A stage is 16 instructions for B and 16 (8 with
-  // kHalf) for A; wave w issues q = kACopies w .. of A and 4 w .. 4 w + 3 of B.
+  // kHalfTile) for A; wave w issues q = kACopies w .. of A and 4 w .. 4 w + 3 of B (small
+  // tiles: 8 for each, 2 per wave).
   // With panels a [rows x K] stage of 16 rows is 1 KB of one panel, contiguous,
   // and a [K x N] stage row band is 8 consecutive panels: full 128-byte lines.
   uint32_t goff[kCopies];
@@ -216,19 +226,19 @@ APEXW_DEV void gemm_tile(const uint16_t* __restrict__ A, const uint16_t* __restr
     goff[i] = poff(row, chunk * 8, lda, panel) * 2u;
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < kBCopies; ++i) {
     if constexpr (kNN) {
       const int krow = 2 * (4 * wave + i) + (lane >> 5), nchunk = (lane & 31) ^ (4 * (krow & 3));
       goff[kACopies + i] = poff(krow, nchunk * 8, ldb, panel) * 2u;
     } else {
-      const int row = 16 * (4 * wave + i) + (lane >> 2), chunk = (lane & 3) ^ ((lane >> 4) & 3);
+      const int row = 16 * (kBCopies * wave + i) + (lane >> 2), chunk = (lane & 3) ^ ((lane >> 4) & 3);
       goff[kACopies + i] = poff(row, chunk * 8, ldb, panel) * 2u;
     }
   }
   // LDS byte addresses of this wave's first A and B chunks in stage 0 (wave-uniform)
-  const uint32_t ldsA0 = __builtin_amdgcn_readfirstlane(lds_address(&lds[0][0][kACopies * wave * 512]));
-  const uint32_t ldsB0 = __builtin_amdgcn_readfirstlane(lds_address(&lds[0][1][4 * wave * 512]));
-  constexpr uint32_t kStageBytes = sizeof(LdsStage), kChunk = 1024;
+  const uint32_t ldsA0 = __builtin_amdgcn_readfirstlane(lds_address(&lds[kACopies * wave * 512]));
+  const uint32_t ldsB0 = __builtin_amdgcn_readfirstlane(lds_address(&lds[kOp + kBCopies * wave * 512]));
+  constexpr uint32_t kStageBytes = kStage * 2, kChunk = 1024;
   const uint16_t* A_s = uniform_ptr(A);
   const uint16_t* B_s = uniform_ptr(B);
   // elements from one K stage to the next along a [rows x K] operand: the next
@@ -242,18 +252,18 @@ APEXW_DEV void gemm_tile(const uint16_t* __restrict__ A, const uint16_t* __restr
                     B_s + (kNN ? (int64_t)h * kBK * ldb : (int64_t)h * kstep));
   };
 
-  f32x16 acc[kFA][4];
+  f32x16 acc[kFA][kFB];
 #pragma unroll
   for (int a = 0; a < kFA; ++a)
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = f32x16{};
+    for (int b = 0; b < kFB; ++b) acc[a][b] = f32x16{};
 
   // MFMA 32x32x16 operand layout: lane l supplies row (l % 32) and k = 8 (l / 32) .. +7.
   const int frag_row = lane & 31, frag_c = lane >> 5;
-  bf16x8 fa[2][kFA], fb[2][4];
+  bf16x8 fa[2][kFA], fb[2][kFB];
   // fragment read i (0 .. kFrags - 1) of k-step s of stage h: A fragments, then B 0..3
   auto frag = [&](int h, int s, int i) {
-    const uint16_t* st = lds[h % kStages][i < kFA ? 0 : 1];
+    const uint16_t* st = lds + (h % kStages) * kStage + (i < kFA ? 0 : kOp);
     if (kNN && i >= kFA) {
       // lane l = 16 g + 4 r + j' of group g addresses K row 16 s + 8 (g / 2) + j'
       // (+ 4 for the upper half), columns n .. n + 3 with n = 16 (g % 2) + 4 r
@@ -270,7 +280,7 @@ APEXW_DEV void gemm_tile(const uint16_t* __restrict__ A, const uint16_t* __restr
       fb[s][i - kFA] = __builtin_bit_cast(bf16x8, u32x4{wl[0], wl[1], wh[0], wh[1]});
       return;
     }
-    const int row = (i < kFA ? wm * kWM + i * 32 : wn * 128 + (i - kFA) * 32) + frag_row;
+    const int row = (i < kFA ? wm * kWM + i * 32 : wn * kWN + (i - kFA) * 32) + frag_row;
     const bf16x8 v = *(const bf16x8*)&st[lds_off(row, s * 2 + frag_c)];
     if (i < kFA) fa[s][i] = v;
     else fb[s][i - kFA] = v;
@@ -281,8 +291,9 @@ APEXW_DEV void gemm_tile(const uint16_t* __restrict__ A, const uint16_t* __restr
   auto mma = [&](int s, auto&& side) {
 #pragma unroll
     for (int j = 0; j < kMM; ++j) {
-      acc[j >> 2][j & 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[s][j >> 2], fb[s][j & 3], acc[j >> 2][j & 3], 0,
-                                                                    0, 0);
+      constexpr int kSh = kFB == 4 ? 2 : 1;
+      const int a = j >> kSh, b = j & (kFB - 1);
+      acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[s][a], fb[s][b], acc[a][b], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
       side(j);
       __builtin_amdgcn_sched_barrier(0);
@@ -312,7 +323,7 @@ APEXW_DEV void gemm_tile(const uint16_t* __restrict__ A, const uint16_t* __restr
     auto add = [&](auto blk_c) {
       constexpr int blk = decltype(blk_c)::value;
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
+      for (int b = 0; b < kFB; ++b) {
         acc[blk][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fh, fb[s][b], acc[blk][b], 0, 0, 0);
         acc[blk][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fl, fb[s][b], acc[blk][b], 0, 0, 0);
       }
@@ -377,25 +388,27 @@ APEXW_DEV void gemm_tile(const uint16_t* __restrict__ A, const uint16_t* __restr
 
   // Epilogue.  Accumulator register r of lane l holds row 8 (r / 4) + 4 (l / 32) + r % 4,
   // column l % 32 of its 32 x 32 block: four consecutive rows of one column per group.
-  // After the last barrier the operand tiles are dead: each wave stages its
-  // kWM x 128 block of O in its own 32 KB of LDS, then writes it row by row to C
-  // and column by column to Ct, both as 16-byte stores along output rows.  The
-  // stage keeps 16-byte chunks XOR-swizzled by row / 8 so that the row reads
-  // (16 lanes per row) and the column reads (lanes down a column) each hit
-  // distinct banks.  A wave reads back only what it wrote itself, and LDS keeps
-  // one wave's accesses in order, so no barrier is needed.
-  uint16_t* stage = lds[wave][0];   // 32 KB per wave
-  auto swz = [](int r, int c) { return r * 128 + ((((c >> 3) ^ (r >> 3)) & 15) << 3) + (c & 7); };
+  // After the last barrier the operand tiles are dead: each wave stages its kWM x kWN
+  // block of O in its own LDS transposed, a column's rows contiguous, so that a group is
+  // one 8-byte write; rows of O^T are then plain 16-byte reads and rows of O transposing
+  // ones (ds_read_b64_tr_b16, two of them for 8 columns).  Both leave as 16-byte stores.
+  // 16-byte chunks are XOR-swizzled by column, so that the writes of 32 columns spread
+  // over all banks.  A wave reads back only what it wrote itself, and LDS keeps one
+  // wave's accesses in order, so no barrier is needed.  This is what bounds products of
+  // short K, where nothing overlaps it (staged the other way round it took 256 2-byte
+  // writes and 256 2-byte reads per lane): EPI
+  uint16_t* stage = lds + wave * (kWM * kWN);
+  constexpr int kCh = kWM / 8;   // 16-byte chunks of a staged column
+  // element offset of rows il .. of staged column jl (il a multiple of 4)
+  auto at = [&](int il, int jl) { return jl * kWM + ((((il >> 3) ^ jl) & (kCh - 1)) << 3) + (il & 7); };
   const int il0 = (lane >> 5) * 4, jl0 = lane & 31;           // within the wave's block
-  const int gi0 = wm * kWM + il0, gj0 = wn * 128 + jl0;       // within the tile
+  const int gi0 = wm * kWM + il0, gj0 = wn * kWN + jl0;       // within the tile
 #pragma unroll
   for (int a = 0; a < kFA; ++a) {
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const int jl = jl0 + b * 32;
+    for (int b = 0; b < kFB; ++b) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int il = il0 + a * 32 + q * 8;
         float v[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = alpha * acc[a][b][q * 4 + r];
@@ -406,43 +419,55 @@ APEXW_DEV void gemm_tile(const uint16_t* __restrict__ A, const uint16_t* __restr
             for (int r = 0; r < 4; ++r) v[r] = fmaf(beta, bf(e[r]), v[r]);
           }
         }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) stage[swz(il + r, jl)] = to_bf(v[r]);
+        *(u32x2*)&stage[at(il0 + a * 32 + q * 8, jl0 + b * 32)] = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
       }
     }
   }
+  // row i0 + lane % 16 of the block, columns j0 + 8 (lane / 16) .. + 7: in each group of 16
+  // lanes, lane r + 4 k addresses rows i0 + 4 r .. + 3 of column j + k, and lane 4 r + c
+  // receives row i0 + 4 r + c of the four columns
+  auto row8 = [&](int i0, int j0) {
+    const int il = i0 + 4 * (lane & 3), j = j0 + 8 * (lane >> 4) + ((lane >> 2) & 3);
+    typedef __attribute__((address_space(3))) v4i16 lds_v4;
+    const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)&stage[at(il, j)]);
+    const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4*)&stage[at(il, j + 4)]);
+    const u32x2 wl = __builtin_bit_cast(u32x2, lo), wh = __builtin_bit_cast(u32x2, hi);
+    return u32x4{wl[0], wl[1], wh[0], wh[1]};
+  };
+  const int ri = lane & 15, rj = 8 * (lane >> 4);
   if constexpr (kC) {
     if (ap.p) {
       // the wave's block of O in O coordinates; p elements outside p's shape
       // (the zero padding of the work matrix) are skipped
-      const int64_t gr0 = ap.row0 + wm * kWM, gc0 = ap.col0 + wn * 128;
+      const int64_t gr0 = ap.row0 + wm * kWM, gc0 = ap.col0 + wn * kWN;
+      auto widen = [](const u32x4& w, float (&u)[8]) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          u[2 * t] = bf((uint16_t)(w[t] & 0xFFFFu));
+          u[2 * t + 1] = bf((uint16_t)(w[t] >> 16));
+        }
+      };
       auto upd = [&](auto pd_c) {
         constexpr int PD = decltype(pd_c)::value;
         if (!ap.transposed) {
-          // row by row: lane chunk = 8 consecutive elements of one row of p
-          for (int it = 0; it < kWM / 4; ++it) {
-            const int c = it * 64 + lane, r = c >> 4, c16 = c & 15;
-            const int64_t gi = gr0 + r, gj = gc0 + c16 * 8;
-            if (gi >= ap.rows || gj >= ap.cols) continue;
-            const u32x4 v = *(const u32x4*)&stage[swz(r, c16 * 8)];
-            float u[8];
+          // 8 consecutive elements of one row of p per lane
+          for (int i0 = 0; i0 < kWM; i0 += 16)
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-              u[2 * t] = bf((uint16_t)(v[t] & 0xFFFFu));
-              u[2 * t + 1] = bf((uint16_t)(v[t] >> 16));
+            for (int j0 = 0; j0 < kWN; j0 += 32) {
+              float u[8];
+              widen(row8(i0, j0), u);     // every lane reads: the transposing read exchanges between lanes
+              const int64_t gi = gr0 + i0 + ri, gj = gc0 + j0 + rj;
+              if (gi < ap.rows && gj < ap.cols)
+                apply_run<PD>(ap, gi * ap.cols + gj, u, (int)min<int64_t>(8, ap.cols - gj));
             }
-            apply_run<PD>(ap, gi * ap.cols + gj, u, (int)min<int64_t>(8, ap.cols - gj));
-          }
         } else {
           // column by column of the block = row by row of p: p[gc0 + jl][gr0 + il + t] = O[gr0 + il + t][gc0 + jl]
-          constexpr int kPerRow = kWM / 8;
-          for (int it = 0; it < kWM / 4; ++it) {
-            const int c = it * 64 + lane, jl = c / kPerRow, il = (c % kPerRow) * 8;
+          for (int it = 0; it < kWM * kWN / 512; ++it) {
+            const int c = it * 64 + lane, jl = c / kCh, il = (c % kCh) * 8;
             const int64_t prow = gc0 + jl, pcol = gr0 + il;
             if (prow >= ap.rows || pcol >= ap.cols) continue;
             float u[8];
-#pragma unroll
-            for (int t = 0; t < 8; ++t) u[t] = bf(stage[swz(il + t, jl)]);
+            widen(*(const u32x4*)&stage[at(il, jl)], u);
             apply_run<PD>(ap, prow * ap.cols + pcol, u, (int)min<int64_t>(8, ap.cols - pcol));
           }
         }
@@ -452,26 +477,21 @@ APEXW_DEV void gemm_tile(const uint16_t* __restrict__ A, const uint16_t* __restr
       else upd(std::integral_constant<int, APEXW_F16>());
     }
     if (C) {
-#pragma unroll 4
-      for (int it = 0; it < kWM / 4; ++it) {
-        const int c = it * 64 + lane, r = c >> 4, c16 = c & 15;
-        const u32x4 v = *(const u32x4*)&stage[swz(r, c16 * 8)];
-        __builtin_nontemporal_store(v, APEXW_GLOBAL(u32x4, C + poff(wm * kWM + r, wn * 128 + c16 * 8, ldc, panel)));
-      }
+#pragma unroll 2
+      for (int i0 = 0; i0 < kWM; i0 += 16)
+#pragma unroll
+        for (int j0 = 0; j0 < kWN; j0 += 32)
+          __builtin_nontemporal_store(
+              row8(i0, j0), APEXW_GLOBAL(u32x4, C + poff(wm * kWM + i0 + ri, wn * kWN + j0 + rj, ldc, panel)));
     }
   }
   if constexpr (kCt) {
     if (write_ct) {
-      constexpr int kPerRow = kWM / 8;   // 16-byte chunks per Ct row of the block
-#pragma unroll 2
-      for (int it = 0; it < kWM / 4; ++it) {
+#pragma unroll 4
+      for (int it = 0; it < kWM * kWN / 512; ++it) {
         // Ct row jl (= column jl of the block), elements il .. il + 7
-        const int c = it * 64 + lane, jl = c / kPerRow, il = (c % kPerRow) * 8;
-        u32x4 v;
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-          v[t] = (uint32_t)stage[swz(il + 2 * t, jl)] | ((uint32_t)stage[swz(il + 2 * t + 1, jl)] << 16);
-        *APEXW_GLOBAL(u32x4, Ct + poff(wn * 128 + jl, wm * kWM + il, ldct, panel)) = v;
+        const int c = it * 64 + lane, jl = c / kCh, il = (c % kCh) * 8;
+        *APEXW_GLOBAL(u32x4, Ct + poff(wn * kWN + jl, wm * kWM + il, ldct, panel)) = *(const u32x4*)&stage[at(il, jl)];
       }
     }
   }
@@ -497,11 +517,12 @@ __global__ __launch_bounds__(256, 1) void gemm_nt_kernel(GemmArgs g) {
 
   const int64_t batch = blockIdx.y;
   const int64_t row0 = (int64_t)tm * kBM, col0 = (int64_t)tn * kBN;
-  gemm_tile<kC, kCt, kAdd, false, false, false>(
+  gemm_tile<kC, kCt, kAdd, false, kWhole, false>(
       g.a + batch * g.sa + row0 * g.lda, g.b + batch * g.sb + col0 * g.ldb, g.lda, g.ldb, g.k,
       kAdd ? g.et + batch * g.se + col0 * g.lde + row0 : nullptr, g.lde,
       kC ? g.c + batch * g.sc + row0 * g.ldc + col0 : nullptr, g.ldc,
-      kCt ? g.ct + batch * g.sct + col0 * g.ldct + row0 : nullptr, g.ldct, true, g.alpha, g.beta, -1, ApplyArgs{}, lds);
+      kCt ? g.ct + batch * g.sct + col0 * g.ldct + row0 : nullptr, g.ldct, true, g.alpha, g.beta, -1, ApplyArgs{},
+      lds[0][0]);
 }
 
 // Grouped GEMM: every problem of a launch (different shapes, K and operands)
@@ -519,12 +540,13 @@ __global__ __launch_bounds__(256, 1) void gemm_nt_kernel(GemmArgs g) {
 // transposed store (ct == c).
 constexpr int kQueues = APEXW_GEMM_QUEUES;
 
-template <bool kC, bool kCt, bool kAdd, bool kNN, bool kPanel>
-__global__ __launch_bounds__(256, 1) void gemm_nt_grouped_kernel(const apexw_gemm_problem* __restrict__ probs,
+template <bool kC, bool kCt, bool kAdd, bool kNN, bool kPanel, bool kTile128>
+__global__ __launch_bounds__(256, kTile128 ? 2 : 1) void gemm_nt_grouped_kernel(const apexw_gemm_problem* __restrict__ probs,
                                                                  const uint32_t* __restrict__ items,
                                                                  const int32_t* __restrict__ queue_offsets,
                                                                  const apexw_amp_dyn* __restrict__ amp) {
-  __shared__ __attribute__((aligned(16))) LdsStage lds[kStages];
+  constexpr int kTM = kTile128 ? 128 : kBM;
+  __shared__ __attribute__((aligned(16))) uint16_t lds[kStages * 2 * kTM * kBK];
   if (amp && amp->skip) return;   // GradScaler found an inf / NaN: no product, no update
   const int q = (int)(blockIdx.x % kQueues), i = (int)(blockIdx.x / kQueues);
   const int begin = queue_offsets[q];
@@ -533,7 +555,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt_grouped_kernel(const apexw_gem
   const apexw_gemm_problem& p = probs[code >> 24];
   const int part = (int)((code >> 22) & 3u);
   const int tm = (int)((code >> 11) & 0x7ffu), tn = (int)(code & 0x7ffu);
-  const int64_t row0 = (int64_t)tm * kBM + (part == 2 ? kBM / 2 : 0), col0 = (int64_t)tn * kBN;
+  const int64_t row0 = (int64_t)tm * kTM + (part == 2 ? kBM / 2 : 0), col0 = (int64_t)tn * kTM;
   const bool mirror = !(p.flags & APEXW_GEMM_SYM) || tm != tn;
   // APEXW_GEMM_ADD_B: the addend is the B operand read at K = row0 + i,
   // accumulated on the matrix cores (validated: alpha == 1, m <= k, no et)
@@ -561,12 +583,16 @@ __global__ __launch_bounds__(256, 1) void gemm_nt_grouped_kernel(const apexw_gem
     ap.wd = (p.flags & APEXW_GEMM_APPLY_WD) != 0;
     ap.vec = p.p_cols % 8 == 0 && ((uintptr_t)p.p & 15u) == 0;
   }
-  if (part)
-    gemm_tile<kC, kCt, kAdd, kNN, true, kPanel>(A, B, p.lda, p.ldb, p.k, Et, p.lde, C, p.ldc, Ct, p.ldct, mirror,
-                                                p.alpha, p.beta, dk, ap, lds);
-  else
-    gemm_tile<kC, kCt, kAdd, kNN, false, kPanel>(A, B, p.lda, p.ldb, p.k, Et, p.lde, C, p.ldc, Ct, p.ldct, mirror,
-                                                 p.alpha, p.beta, dk, ap, lds);
+  auto tile = [&](auto shape_c) {
+    gemm_tile<kC, kCt, kAdd, kNN, decltype(shape_c)::value, kPanel>(A, B, p.lda, p.ldb, p.k, Et, p.lde, C, p.ldc, Ct,
+                                                                    p.ldct, mirror, p.alpha, p.beta, dk, ap, lds);
+  };
+  if constexpr (kTile128) {
+    tile(std::integral_constant<int, kSmall>());
+  } else {
+    if (part) tile(std::integral_constant<int, kHalfTile>());
+    else tile(std::integral_constant<int, kWhole>());
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -965,13 +991,13 @@ namespace {
 
 // one grouped launch of the epilogue kind's instantiation (kind without the
 // panel bit, which selects kPanel)
-template <bool kPanel>
+template <bool kPanel, bool kTile128>
 int launch_grouped(const apexw_gemm_problem* probs, const uint32_t* items, const int32_t* offsets, int32_t n_wg,
                    int32_t kind, const apexw_amp_dyn* amp, hipStream_t stream) {
   const dim3 grid(n_wg), block(256);
-#define APEXW_GROUPED(C, CT, ADD, NN)                                                                              \
-  hipLaunchKernelGGL((gemm_nt_grouped_kernel<C, CT, ADD, NN, kPanel>), grid, block, 0, stream, probs, items, offsets, \
-                     amp)
+#define APEXW_GROUPED(C, CT, ADD, NN)                                                                                \
+  hipLaunchKernelGGL((gemm_nt_grouped_kernel<C, CT, ADD, NN, kPanel, kTile128>), grid, block, 0, stream, probs, items, \
+                     offsets, amp)
   switch (kind) {
     case APEXW_GEMM_OUT_C: APEXW_GROUPED(true, false, false, false); break;
     case APEXW_GEMM_OUT_C | APEXW_GEMM_ADD: APEXW_GROUPED(true, false, true, false); break;
@@ -979,9 +1005,18 @@ int launch_grouped(const apexw_gemm_problem* probs, const uint32_t* items, const
     case APEXW_GEMM_OUT_CT | APEXW_GEMM_ADD: APEXW_GROUPED(false, true, true, false); break;
     case APEXW_GEMM_OUT_C | APEXW_GEMM_OUT_CT: APEXW_GROUPED(true, true, false, false); break;
     case APEXW_GEMM_OUT_C | APEXW_GEMM_OUT_CT | APEXW_GEMM_ADD: APEXW_GROUPED(true, true, true, false); break;
-    case APEXW_GEMM_OUT_C | APEXW_GEMM_KIND_NN: APEXW_GROUPED(true, false, false, true); break;
-    case APEXW_GEMM_OUT_C | APEXW_GEMM_ADD | APEXW_GEMM_KIND_NN: APEXW_GROUPED(true, false, true, true); break;
-    default: return APEXW_ERR_ARG;
+    default:
+      if constexpr (!kTile128) {
+        if (kind == (APEXW_GEMM_OUT_C | APEXW_GEMM_KIND_NN)) {
+          APEXW_GROUPED(true, false, false, true);
+          break;
+        }
+        if (kind == (APEXW_GEMM_OUT_C | APEXW_GEMM_ADD | APEXW_GEMM_KIND_NN)) {
+          APEXW_GROUPED(true, false, true, true);
+          break;
+        }
+      }
+      return APEXW_ERR_ARG;
   }
 #undef APEXW_GROUPED
   return hipGetLastError() == hipSuccess ? APEXW_OK : APEXW_ERR_LAUNCH;
@@ -991,9 +1026,12 @@ int launch_grouped(const apexw_gemm_problem* probs, const uint32_t* items, const
 
 int apexw_launch_gemm_grouped(const apexw_gemm_problem* probs, const uint32_t* items, const int32_t* offsets,
                               int32_t n_wg, int32_t kind, const apexw_amp_dyn* amp, hipStream_t stream) {
-  const int32_t base = kind & ~APEXW_GEMM_KIND_PANEL;
-  return (kind & APEXW_GEMM_KIND_PANEL) ? launch_grouped<true>(probs, items, offsets, n_wg, base, amp, stream)
-                                        : launch_grouped<false>(probs, items, offsets, n_wg, base, amp, stream);
+  const int32_t base = kind & ~(APEXW_GEMM_KIND_PANEL | APEXW_GEMM_KIND_TILE128);
+  if (kind & APEXW_GEMM_KIND_TILE128)
+    return (kind & APEXW_GEMM_KIND_PANEL) ? launch_grouped<true, true>(probs, items, offsets, n_wg, base, amp, stream)
+                                          : APEXW_ERR_ARG;
+  return (kind & APEXW_GEMM_KIND_PANEL) ? launch_grouped<true, false>(probs, items, offsets, n_wg, base, amp, stream)
+                                        : launch_grouped<false, false>(probs, items, offsets, n_wg, base, amp, stream);
 }
 
 int64_t apexw_muon_units(int64_t rows, int64_t cols, bool tiles) {

@@ -116,30 +116,62 @@ class NSWorkspace:
         return _to_panels(mat) if self.panel else mat
 
 
-def _ns_problems(ws, phase, cur, out, tag=None, tags=None):
+def _ns_problems(ws, phase, cur, out, tag=None, tags=None, tile=_lib.GEMM_TILE):
     """Append the GEMM problems of one Newton-Schulz product for every matrix of ws.
 
     phase 0: A = X X^T (symmetric); phase 1: B = c A A + b A (symmetric);
     phase 2: X' = B X + a X with X^T as the [N x K] operand, the addend a X taken
     from that same operand on the matrix cores, and X' written in both layouts.
     cur is the ping-pong slot holding the current X.  With tags, (tag, entry) is
-    appended per row.
+    appended per row.  tile: the output tiles' size (256 or 128); outputs cover the
+    matrix padded to it, K the matrix padded to the K tile (X' needs K to cover its
+    rows, for the addend), and what the buffers hold beyond stays zero.
     """
     mp, np_ = ws.mp, ws.np_
-    pf = _lib.GEMM_PANEL if ws.panel else 0
+    m, n = _pad(ws.m, tile), _pad(ws.n, tile)
+    km, kn = _pad(ws.m, _lib.GEMM_KTILE), _pad(ws.n, _lib.GEMM_KTILE)
+    pf = (_lib.GEMM_PANEL if ws.panel else 0) | (_lib.GEMM_TILE128 if tile == 128 else 0)
     for e in range(ws.batch):
         if tags is not None:
             tags.append((tag, e))
         x = ws.x[cur][e].data_ptr()
         a, b = ws.a[e].data_ptr(), ws.b[e].data_ptr()
         if phase == 0:
-            out.append((x, x, 0, a, a, mp, mp, np_, np_, np_, 0, mp, mp, 1.0, 0.0, _lib.GEMM_SYM | pf, 0))
+            out.append((x, x, 0, a, a, m, m, kn, np_, np_, 0, mp, mp, 1.0, 0.0, _lib.GEMM_SYM | pf, 0))
         elif phase == 1:
-            out.append((a, a, a, b, b, mp, mp, mp, mp, mp, mp, mp, mp, NS_C, NS_B, _lib.GEMM_SYM | pf, 0))
+            out.append((a, a, a, b, b, m, m, km, mp, mp, mp, mp, mp, NS_C, NS_B, _lib.GEMM_SYM | pf, 0))
         else:
             xt = ws.xt[cur][e].data_ptr()
             nx, nxt = ws.x[cur ^ 1][e].data_ptr(), ws.xt[cur ^ 1][e].data_ptr()
-            out.append((b, xt, 0, nx, nxt, mp, np_, mp, mp, mp, 0, np_, mp, 1.0, NS_A, _lib.GEMM_ADD_B | pf, 0))
+            out.append((b, xt, 0, nx, nxt, m, n, m, mp, mp, 0, np_, mp, 1.0, NS_A, _lib.GEMM_ADD_B | pf, 0))
+
+
+def _products(wss, active, phase, tile):
+    """(tiles, K) of each matrix's product of a phase."""
+    for j in active:
+        ws = wss[j]
+        tm, tn = _pad(ws.m, tile) // tile, _pad(ws.n, tile) // tile
+        k = (_pad(ws.n, _lib.GEMM_KTILE), _pad(ws.m, _lib.GEMM_KTILE), _pad(ws.m, tile))[phase]
+        for _ in range(ws.batch):
+            yield (tm * (tm + 1) // 2 if phase < 2 else tm * tn), k
+
+
+def _tile_of(wss, active, phase, cus):
+    """256 or 128: the output tile of a phase's launch on `cus` compute units.
+
+    A 256 x 256 tile moves half the operand bytes per FLOP of a 128 x 128 one, but fills
+    the chip only from about one tile per unit on, and its epilogue overlaps nothing.  So
+    128 up to as many 256-tiles T as measured faster (us, 256 / 128, one MI355X, 256 units):
+      A (K the long side): T 9: 10.8 / 8.0, 72: 27.3 / 25.5; 200: 63.7 / 72.7, 288: 99.7 / 126.7
+      B (K <= 2048):       T 9: 14.9 / 10.0, 200: 54.1 / 48.9, 288: 67.3 / 55.5; 680 (K 4096): 333 / 345
+      X' (K <= 2048):      T 12: 13.2 / 9.6, 288: 44.3 / 40.0, 595: 146 / 138; 784: 228 / 234
+    """
+    prods = list(_products(wss, active, phase, _lib.GEMM_TILE))
+    tiles, k = sum(t for t, _ in prods), max((k for _, k in prods), default=0)
+    most = cus / 2
+    if phase > 0 and k <= 2048:
+        most = cus * (1.25 if phase == 1 else 2.5)
+    return 128 if tiles <= most else _lib.GEMM_TILE
 
 
 class NSPlan:
@@ -163,10 +195,6 @@ class NSPlan:
         # FLOPs the kernels execute (padded; upper-triangle tiles of A and B)
         self.flops = sum(ws.batch * s * (4 * ws.m * ws.m * ws.n + 2 * ws.m ** 3) for ws, s in zip(wss, steps))
         self.exec_flops = 0
-        for ws, s in zip(wss, steps):
-            t = ws.mp // _lib.GEMM_TILE
-            tri = (t + 1) / (2 * t)
-            self.exec_flops += ws.batch * s * (tri * (2 * ws.mp ** 2 * ws.np_ + 2 * ws.mp ** 3) + 2 * ws.mp ** 2 * ws.np_)
         self.device = device
         self._applied = {}      # id(host table) -> (applies key, device table with the fused update)
         # the preparation's unit tables (momentum chunks, 64 x 64 tiles) over every matrix, in order
@@ -184,11 +212,20 @@ class NSPlan:
                 built[key] = [self._launches(wss, active, final if phase == 2 else (), phase, i % 2, device)
                               for phase in range(3)]
             self.iters.append(built[key])
+            for phase in range(3):
+                tile = self._tile(wss, active, phase)
+                self.exec_flops += sum(2 * tile * tile * t * k for t, k in _products(wss, active, phase, tile))
+
+    def _tile(self, wss, active, phase):
+        if any(not wss[j].panel for j in active):
+            return _lib.GEMM_TILE
+        return _tile_of(wss, active, phase, _lib.GEMM_QUEUES * _lib.cus_per_queue(self.device))
 
     def _launches(self, wss, active, final, phase, cur, device):
         rows, tags = [], []
+        tile = self._tile(wss, active, phase)
         for j in active:
-            _ns_problems(wss[j], phase, cur, rows, j, tags)
+            _ns_problems(wss[j], phase, cur, rows, j, tags, tile)
         out = []
         for c0 in range(0, len(rows), _lib.GEMM_MAX_PROBLEMS):
             probs = _lib.gemm_problems(rows[c0:c0 + _lib.GEMM_MAX_PROBLEMS])

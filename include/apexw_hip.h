@@ -615,6 +615,10 @@ typedef struct apexw_gemm_problem {
  * of an operand is then a run of whole 128-byte lines.  Leading dimensions must
  * be multiples of 32.  p (APEXW_GEMM_APPLY) stays row-major. */
 #define APEXW_GEMM_PANEL 64u
+/* The problem is tiled 128 x 128 (m, n multiples of 128) instead of 256 x 256: for
+ * launches whose 256 x 256 tiles would leave most of the chip idle.  With
+ * APEXW_GEMM_PANEL and without APEXW_GEMM_B_KN only; every problem of a launch alike. */
+#define APEXW_GEMM_TILE128 128u
 
 /* epilogue kinds of a grouped launch (bit mask) */
 #define APEXW_GEMM_OUT_C 1   /* row-major output */
@@ -622,6 +626,7 @@ typedef struct apexw_gemm_problem {
 #define APEXW_GEMM_ADD 4     /* beta * E added */
 #define APEXW_GEMM_KIND_NN 8 /* B given as [k x n] (APEXW_GEMM_B_KN) */
 #define APEXW_GEMM_KIND_PANEL 16 /* matrices in 32 x 32 panels (APEXW_GEMM_PANEL) */
+#define APEXW_GEMM_KIND_TILE128 32 /* 128 x 128 tiles (APEXW_GEMM_TILE128) */
 
 /* Tile queues of a grouped launch: one per XCD of MI355X. */
 #define APEXW_GEMM_QUEUES 8
