@@ -116,12 +116,13 @@ class NSWorkspace:
         return _to_panels(mat) if self.panel else mat
 
 
-def _ns_problems(ws, phase, cur, out, tag=None, tags=None, tile=_lib.GEMM_TILE):
+def _ns_problems(ws, phase, cur, out, tag=None, tags=None, tile=_lib.GEMM_TILE, nn=False):
     """Append the GEMM problems of one Newton-Schulz product for every matrix of ws.
 
     phase 0: A = X X^T (symmetric); phase 1: B = c A A + b A (symmetric);
     phase 2: X' = B X + a X with X^T as the [N x K] operand, the addend a X taken
-    from that same operand on the matrix cores, and X' written in both layouts.
+    from that same operand on the matrix cores, and X' written in both layouts; or, nn,
+    with X as the [K x N] operand and X' written once (no X^T is kept).
     cur is the ping-pong slot holding the current X.  With tags, (tag, entry) is
     appended per row.  tile: the output tiles' size (256 or 128); outputs cover the
     matrix padded to it, K the matrix padded to the K tile (X' needs K to cover its
@@ -140,6 +141,10 @@ def _ns_problems(ws, phase, cur, out, tag=None, tags=None, tile=_lib.GEMM_TILE):
             out.append((x, x, 0, a, a, m, m, kn, np_, np_, 0, mp, mp, 1.0, 0.0, _lib.GEMM_SYM | pf, 0))
         elif phase == 1:
             out.append((a, a, a, b, b, m, m, km, mp, mp, mp, mp, mp, NS_C, NS_B, _lib.GEMM_SYM | pf, 0))
+        elif nn:
+            nx = ws.x[cur ^ 1][e].data_ptr()
+            out.append((b, x, 0, nx, 0, m, n, m, mp, np_, 0, np_, 0, 1.0, NS_A,
+                        _lib.GEMM_B_KN | _lib.GEMM_ADD_B | pf, 0))
         else:
             xt = ws.xt[cur][e].data_ptr()
             nx, nxt = ws.x[cur ^ 1][e].data_ptr(), ws.xt[cur ^ 1][e].data_ptr()
@@ -174,6 +179,13 @@ def _tile_of(wss, active, phase, cus):
     return 128 if tiles <= most else _lib.GEMM_TILE
 
 
+# X' = B X + a X up to this K (the wide work matrix's rows) reads X as [K x N] rows: its
+# fragment reads are dearer than X^T's, but X'^T is neither written nor prepared (us, X^T /
+# [K x N], 256 x 256 tiles, one MI355X: K 768: 229 / 202, 1024: 131 / 126, 1280: 512 / 495,
+# 2048: 233 / 231, 4096: 1484 / 1521)
+NN_MAX_K = 1536
+
+
 class NSPlan:
     """Newton-Schulz for every Muon matrix of a step on one device, as grouped launches.
 
@@ -202,6 +214,10 @@ class NSPlan:
         self._prep_units = None
         self._prepared = None   # (bytes of the last item table, its device copy)
         self._seq = None        # host array of the launch sequence
+        # one form of X' for the whole plan: a later iteration reads what an earlier one wrote
+        every = tuple(range(len(wss)))
+        self.nn = (bool(wss) and self._tile(wss, every, 2) == _lib.GEMM_TILE
+                   and max(ws.mp for ws in wss) <= NN_MAX_K)
         built = {}
         self.iters = []
         for i in range(max(steps, default=0)):
@@ -217,7 +233,7 @@ class NSPlan:
                 self.exec_flops += sum(2 * tile * tile * t * k for t, k in _products(wss, active, phase, tile))
 
     def _tile(self, wss, active, phase):
-        if any(not wss[j].panel for j in active):
+        if any(not wss[j].panel for j in active) or (phase == 2 and getattr(self, "nn", False)):
             return _lib.GEMM_TILE
         return _tile_of(wss, active, phase, _lib.GEMM_QUEUES * _lib.cus_per_queue(self.device))
 
@@ -225,7 +241,7 @@ class NSPlan:
         rows, tags = [], []
         tile = self._tile(wss, active, phase)
         for j in active:
-            _ns_problems(wss[j], phase, cur, rows, j, tags, tile)
+            _ns_problems(wss[j], phase, cur, rows, j, tags, tile, self.nn)
         out = []
         for c0 in range(0, len(rows), _lib.GEMM_MAX_PROBLEMS):
             probs = _lib.gemm_problems(rows[c0:c0 + _lib.GEMM_MAX_PROBLEMS])
@@ -486,8 +502,10 @@ class ApexMuon(Optimizer):
             for dev, djobs in by_dev.items():
                 plan = self._ns_plan(djobs, dev)
                 stream = torch.cuda.current_stream(dev).cuda_stream
-                plan.prepare(stream, np.array([row for j in djobs for row in j["items"]],
-                                              dtype=_lib.MUON_ITEM_DTYPE), inv_scale, amp_ptr)
+                items = np.array([row for j in djobs for row in j["items"]], dtype=_lib.MUON_ITEM_DTYPE)
+                if plan.nn:
+                    items["xt"] = 0       # its products read no X^T
+                plan.prepare(stream, items, inv_scale, amp_ptr)
                 applies = [self._apply_args(j) for j in djobs]
                 plan.run(stream, applies, self.keep_ns_result, amp_ptr)
             for j in jobs:

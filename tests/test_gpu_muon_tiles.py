@@ -33,6 +33,28 @@ def test_tiles_agree_bit_for_bit(dtype, monkeypatch):
         assert torch.equal(x, y)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_kn_form_agrees_bit_for_bit(dtype, monkeypatch):
+    """X as the [K x N] operand of X' = B X + a X against X^T as its [N x K] one."""
+    from apexw_amd import muon
+    out = []
+    monkeypatch.setattr(muon, "_tile_of", lambda *a: 256)
+    for most in (0, 1536):
+        monkeypatch.setattr(muon, "NN_MAX_K", most)
+        gen = torch.Generator(device="cuda").manual_seed(4)
+        params = [torch.nn.Parameter((torch.randn(s, device="cuda", generator=gen) * 0.02).to(dtype)) for s in SHAPES]
+        for p in params:
+            p.grad = (torch.randn(p.shape, device="cuda", generator=gen) * 1e-2).to(dtype)
+        # groups of different step counts: later iterations run on a part of the matrices
+        opt = muon.ApexMuon([dict(params=params[:4], ns_steps=2), dict(params=params[4:], ns_steps=5)], lr=1e-2)
+        for _ in range(2):
+            opt.step()
+        assert [p.nn for p in opt._ns_plans.values()] == [bool(most)]
+        out.append([p.detach().clone() for p in params])
+    for x, y in zip(*out):
+        assert torch.equal(x, y)
+
+
 def test_tile_rule():
     """Few tiles take 128, a chip's worth of long ones 256."""
     from apexw_amd.muon import NSWorkspace, _tile_of
