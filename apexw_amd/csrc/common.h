@@ -222,6 +222,31 @@ APEXW_DEV float wave_sum(float x) {
   return x;
 }
 
+// x / y rounded to nearest for a normal y > 0 and a finite quotient, the hardware
+// reciprocal and one FMA residual (Markstein), wrong only within ~2^-45 of a rounding
+// midpoint: a quarter of the IEEE sequence's instructions.
+APEXW_DEV float div_once(float x, float y) {
+  const float r = __builtin_amdgcn_rcpf(y), q = x * r;
+  return fmaf(fmaf(-q, y, x), r, q);
+}
+
+// The four INT8 codes of a word times a scale: bytes biased by 128 convert in one
+// instruction each, and fma(b, s, -128 s) is the exact (b - 128) s rounded once.
+APEXW_DEV void i8_decode4(uint32_t w, float s, float* x) {
+  const uint32_t u = w ^ 0x80808080u;
+  const float z = -128.0f * s;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) x[j] = fmaf((float)((u >> (8 * j)) & 0xFFu), s, z);
+}
+// Four INT8 codes from m / scale: clamped to +-127, rounded to nearest even by adding
+// 1.5 x 2^23 (the code is then the low byte), gathered by byte permutes.
+APEXW_DEV uint32_t i8_encode4(const float* y) {
+  uint32_t z[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) z[j] = __float_as_uint(__builtin_amdgcn_fmed3f(y[j], -127.0f, 127.0f) + 12582912.0f);
+  const uint32_t lo = __builtin_amdgcn_perm(z[1], z[0], 0x0c0c0400u), hi = __builtin_amdgcn_perm(z[3], z[2], 0x0c0c0400u);
+  return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
 APEXW_DEV int lane_id() { return (int)(threadIdx.x & 63u); }
 
 // Grid for a 256-thread (4-wave) kernel that strides over `n_units` work units,

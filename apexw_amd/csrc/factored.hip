@@ -588,9 +588,8 @@ APEXW_DEV void fv_unit_full(const apexw_tensor& t, const apexw_fv_tensor& e, uin
       for (int j = 0; j < 8; ++j)
         m[j] = j & 1 ? __uint_as_float(mw[j >> 1] & 0xFFFF0000u) : bf16_bits_to_f32(mw[j >> 1] & 0xFFFFu);
     } else if constexpr (MK == kM8) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        m[j] = (float)(int8_t)(((j < 4 ? mw8[k].x : mw8[k].y) >> (8 * (j & 3))) & 0xFFu) * ms_old;
+      i8_decode4(mw8[k].x, ms_old, m);
+      i8_decode4(mw8[k].y, ms_old, m + 4);
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j)
@@ -628,7 +627,7 @@ APEXW_DEV void fv_unit_full(const apexw_tensor& t, const apexw_fv_tensor& e, uin
     for (int j = 0; j < 8; ++j) {
       const float gj = fv_grad<GD>(g[j], c);
       m[j] = lerp_to(m[j], gj, hp.lerp_coef, hp.flags & APEXW_HP_LERP_HI);
-      const float upd = div_refined(m[j], den[j], rcp_refined(den[j])) * hp.step_size;
+      const float upd = div_once(m[j], den[j]) * hp.step_size;
       if constexpr (PD == APEXW_F32) {
         p[j] = (wd ? p[j] * hp.wd_factor : p[j]) - upd;
       } else {
@@ -648,7 +647,6 @@ APEXW_DEV void fv_unit_full(const apexw_tensor& t, const apexw_fv_tensor& e, uin
   float ms = fmaxf(amax, 1e-12f) / (MK == kM8 ? 127.0f : 31.0f);
   ms = fmaxf(ms, ms_old * 0.9f);
   if (lane == 0) t.m_scale[unit] = ms;
-  const float lim = MK == kM8 ? 127.0f : 31.0f;
   const float rms = rcp_refined(ms);
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
@@ -667,16 +665,13 @@ APEXW_DEV void fv_unit_full(const apexw_tensor& t, const apexw_fv_tensor& e, uin
         y[j + 1] = y[j + 1] + n1;
       }
     }
-    uint32_t q[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int32_t qi = (int32_t)fminf(fmaxf(rintf(y[j]), -lim), lim);
-      q[j] = MK == kM8 ? ((uint32_t)qi & 0xFFu) : (uint32_t)(qi + 31);
-    }
     if constexpr (MK == kM8) {
-      const u32x2 v = {q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24), q[4] | (q[5] << 8) | (q[6] << 16) | (q[7] << 24)};
+      const u32x2 v = {i8_encode4(y), i8_encode4(y + 4)};
       __builtin_nontemporal_store(v, APEXW_GLOBAL(u32x2, (int8_t*)t.m + e0));
     } else {
+      uint32_t q[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = (uint32_t)((int32_t)__builtin_amdgcn_fmed3f(rintf(y[j]), -31.0f, 31.0f) + 31);
       const uint32_t w0 = q[0] | (q[1] << 6) | (q[2] << 12) | (q[3] << 18);
       const uint32_t w1 = q[4] | (q[5] << 6) | (q[6] << 12) | (q[7] << 18);
       const auto mp = APEXW_GLOBAL(uint16_t, (uint8_t*)t.m + (e0 >> 2) * 3);
@@ -690,8 +685,9 @@ APEXW_DEV void fv_unit_full(const apexw_tensor& t, const apexw_fv_tensor& e, uin
 // A whole unit inside one row of the matrix (cols % 4 == 0).  PLAIN: no grad-dtype
 // sanitize / clip / AMP unscale and a lerp weight below 0.5; otherwise the grad
 // goes through fv_grad_sel and the lerp picks its form per launch.  The row factor is one value for the unit and the column roots
-// are 16-byte loads; the update's division is the refined one of fv_unit, and
-// bf16 roundings convert pairs.  Returns false, before any load, when the unit
+// are 16-byte loads; the update's division is the one-residual one of div_once, m's codes
+// move by byte permutes, and bf16 roundings convert pairs: bound by memory and vector issue
+// alike (four Llama layers, INT8 m, 7 GB: 1420 -> 1371 us, 5.1 TB/s).  Returns false, before any load, when the unit
 // crosses a row: the caller then runs fv_unit_full on it.
 template <int PD, int MK, bool PLAIN>
 APEXW_DEV bool fv_unit_row(const apexw_tensor& t, const apexw_fv_tensor& e, uint32_t tix, uint32_t unit,
@@ -775,9 +771,8 @@ APEXW_DEV bool fv_unit_row(const apexw_tensor& t, const apexw_fv_tensor& e, uint
       for (int j = 0; j < 8; ++j)
         m[j] = j & 1 ? __uint_as_float(mw[j >> 1] & 0xFFFF0000u) : __uint_as_float(mw[j >> 1] << 16);
     } else if constexpr (MK == kM8) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        m[j] = (float)(int8_t)(((j < 4 ? mw8[k].x : mw8[k].y) >> (8 * (j & 3))) & 0xFFu) * ms_old;
+      i8_decode4(mw8[k].x, ms_old, m);
+      i8_decode4(mw8[k].y, ms_old, m + 4);
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j)
@@ -796,7 +791,7 @@ APEXW_DEV bool fv_unit_row(const apexw_tensor& t, const apexw_fv_tensor& e, uint
       m[j] = PLAIN ? fmaf(hp.lerp_coef, g[k][j] - m[j], m[j])
                    : lerp_to(m[j], g[k][j], hp.lerp_coef, hp.flags & APEXW_HP_LERP_HI);
       const float den = fmaxf(rv * cs[j] + hp.eps_scaled, hp.eps);
-      upd[j] = div_refined(m[j], den, rcp_refined(den)) * hp.step_size;
+      upd[j] = div_once(m[j], den) * hp.step_size;
       if constexpr (MK != kM16) {
         mnew[k][j] = m[j];
         amax = fmaxf(amax, fabsf(m[j]));
@@ -861,16 +856,13 @@ APEXW_DEV bool fv_unit_row(const apexw_tensor& t, const apexw_fv_tensor& e, uint
 #pragma unroll
         for (int j = 0; j < 8; ++j) y[j] = rintf(div_refined(mnew[k][j], ms, rms));
       }
-      uint32_t q[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int32_t qi = (int32_t)fminf(fmaxf(y[j], -lim), lim);
-        q[j] = MK == kM8 ? ((uint32_t)qi & 0xFFu) : (uint32_t)(qi + 31);
-      }
       if constexpr (MK == kM8) {
-        const u32x2 v = {q[0] | (q[1] << 8) | (q[2] << 16) | (q[3] << 24), q[4] | (q[5] << 8) | (q[6] << 16) | (q[7] << 24)};
+        const u32x2 v = {i8_encode4(y), i8_encode4(y + 4)};
         __builtin_nontemporal_store(v, APEXW_GLOBAL(u32x2, (int8_t*)t.m + e0));
       } else {
+        uint32_t q[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j] = (uint32_t)((int32_t)__builtin_amdgcn_fmed3f(y[j], -31.0f, 31.0f) + 31);
         const uint32_t w0 = q[0] | (q[1] << 6) | (q[2] << 12) | (q[3] << 18);
         const uint32_t w1 = q[4] | (q[5] << 6) | (q[6] << 12) | (q[7] << 18);
         const auto mp = APEXW_GLOBAL(uint16_t, (uint8_t*)t.m + (e0 >> 2) * 3);

@@ -319,13 +319,7 @@ APEXW_DEV float sqrt_shared(float x) {
   const float s = x * y;
   return fmaf(fmaf(-s, s, x), 0.5f * y, s);
 }
-// x / y rounded to nearest for a normal y > 0 and a finite quotient, likewise: the
-// hardware reciprocal and one FMA residual.
-APEXW_DEV float div_once(float x, float y) {
-  const float r = __builtin_amdgcn_rcpf(y), q = x * r;
-  return fmaf(fmaf(-q, y, x), r, q);
-}
-// ... both with every denominator at least this (any real eps is)
+// sqrt_shared and div_once (common.h) want every denominator at least this (any real eps is)
 constexpr float kFastEps = 1e-12f;
 
 // x rounded to DT in place, and stored rounded to DT: bf16 in pairs
@@ -353,23 +347,6 @@ template <int DT> APEXW_DEV void store8_rnd(void* base, int64_t i, float (&x)[8]
   }
 }
 
-// The four INT8 codes of a word times a scale: bytes biased by 128 convert in one
-// instruction each, and fma(b, s, -128 s) is the exact (b - 128) s rounded once.
-APEXW_DEV void i8_decode4(uint32_t w, float s, float* x) {
-  const uint32_t u = w ^ 0x80808080u;
-  const float z = -128.0f * s;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) x[j] = fmaf((float)((u >> (8 * j)) & 0xFFu), s, z);
-}
-// Four INT8 codes from m / scale: clamped to +-127, rounded to nearest even by adding
-// 1.5 x 2^23 (the code is then the low byte), gathered by byte permutes.
-APEXW_DEV uint32_t i8_encode4(const float* y) {
-  uint32_t z[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) z[j] = __float_as_uint(__builtin_amdgcn_fmed3f(y[j], -127.0f, 127.0f) + 12582912.0f);
-  const uint32_t lo = __builtin_amdgcn_perm(z[1], z[0], 0x0c0c0400u), hi = __builtin_amdgcn_perm(z[3], z[2], 0x0c0c0400u);
-  return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
-}
 // unit_uniform(r) - 1/2 for the 16 bits r = h >> 16, exact in one FMA.
 APEXW_DEV float half_noise(uint32_t h) { return fmaf((float)(h >> 16), 0x1p-16f, 0x1p-17f - 0.5f); }
 
