@@ -402,6 +402,24 @@ APEXW_DEV void update8(float (&p)[8], float (&g)[8], float (&m)[8], float (&v)[8
   }
 }
 
+// Elements i .. i + 3 and i + 256 .. i + 259 of an fp32 tensor.
+APEXW_DEV void load4x2(const void* base, int64_t i, float (&x)[8]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const u32x4 w = __builtin_nontemporal_load(APEXW_GLOBAL(const u32x4, (const float*)base + i + 256 * h));
+    x[4 * h] = __uint_as_float(w.x); x[4 * h + 1] = __uint_as_float(w.y);
+    x[4 * h + 2] = __uint_as_float(w.z); x[4 * h + 3] = __uint_as_float(w.w);
+  }
+}
+APEXW_DEV void store4x2(void* base, int64_t i, const float (&x)[8]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const u32x4 w = {__float_as_uint(x[4 * h]), __float_as_uint(x[4 * h + 1]), __float_as_uint(x[4 * h + 2]),
+                     __float_as_uint(x[4 * h + 3])};
+    __builtin_nontemporal_store(w, APEXW_GLOBAL(u32x4, (float*)base + i + 256 * h));
+  }
+}
+
 // Group k (512 elements, 8 per lane) of the unit starting at element `start`.
 // vmax: amsgrad's running max of v for this tensor (hparams.max_v), else NULL.
 template <int PD, int GD, int MD, int VD, bool QUAD, bool SR, bool VAR>
@@ -415,6 +433,28 @@ APEXW_DEV void compact_group(const apexw_tensor& t, int64_t start, int k, const 
     const int cnt = (int)((n - e0) < 8 ? (n - e0) : 8);
     float p[8], g[8], m[8], v[8], x[8], ms[8];
     const bool full = vec && cnt == 8;
+    // all-fp32 tensors ("full" precision): a lane takes two runs of 4 elements, 256 apart,
+    // instead of 8 consecutive ones, so that each 16-byte access of the wave is one
+    // contiguous KiB (8 consecutive ones leave every other 16 bytes to a second access).
+    // The update is element by element and draws no noise for fp32.  GPT-2-small with clip,
+    // 28 bytes per parameter: 800 -> 742 us per step.
+    constexpr bool kSplit = !VAR && !QUAD && PD == APEXW_F32 && GD == APEXW_F32 && MD == APEXW_F32 && VD == APEXW_F32;
+    if constexpr (kSplit) {
+      const int64_t s0 = start + (int64_t)k * 512;
+      if (vec && s0 + 512 <= n && !(c.tflags & APEXW_FLAG_GC) && c.hp->mode != APEXW_MODE_SINGLE) {
+        const int64_t lo = s0 + lane * 4;
+        load4x2(t.p, lo, p);
+        load4x2(t.g, lo, g);
+        load4x2(t.m, lo, m);
+        load4x2(t.v, lo, v);
+        const float mean[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+        update8<PD, GD, MD, VD, QUAD, SR, VAR>(p, g, m, v, x, ms, 8, (uint32_t)lo, c, false, mean, false, false, 8);
+        store4x2(t.p, lo, p);
+        store4x2(t.m, lo, m);
+        store4x2(t.v, lo, v);
+        return;
+      }
+    }
     const bool ams = VAR && !QUAD && vmax != nullptr;
     const bool slow = VAR && !QUAD && mslow != nullptr;
     // lion keeps no second moment: v is neither read nor written
@@ -649,8 +689,9 @@ __global__ __launch_bounds__(256) void compact_counts_zero_kernel(unsigned long 
   if (i < n) counts[i] = 0ull;
 }
 
+// (the plain instantiation holds five waves per SIMD: 96 registers)
 template <bool VAR>
-__global__ __launch_bounds__(256) void compact_step_kernel(const apexw_tensor* __restrict__ tensors,
+__global__ __launch_bounds__(256, VAR ? 1 : 5) void compact_step_kernel(const apexw_tensor* __restrict__ tensors,
                                                            const apexw_unit* __restrict__ units,
                                                            int64_t n_units, apexw_hparams hp_in) {
   apexw_hparams hp = hp_in;

@@ -176,17 +176,23 @@ APEXW_DEV NormSpan norm_span(const apexw_tensor* tensors, int64_t t, const int64
   return {partial + unit_begin[t], unit_begin[t + 1] - unit_begin[t]};
 }
 
-// The sum of `s` by `step` lanes, this one the `first`: eight loads in flight and
-// eight running sums (a plain loop waits for memory at each addition).
-APEXW_DEV float span_sum(const NormSpan& s, int64_t first, int64_t step) {
-  float a[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+// The sum of `s` by `step` lanes, this one the `first`, in float64: eight loads in
+// flight and eight running sums (a plain loop waits for memory at each addition).
+APEXW_DEV double span_sum(const NormSpan& s, int64_t first, int64_t step) {
+  double a[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   int64_t i = first;
   for (; i + 7 * step < s.n; i += 8 * step) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) a[j] += s.p[i + j * step];
+    for (int j = 0; j < 8; ++j) a[j] += (double)s.p[i + j * step];
   }
-  for (; i < s.n; i += step) a[0] += s.p[i];
+  for (; i < s.n; i += step) a[0] += (double)s.p[i];
   return ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+}
+
+APEXW_DEV double wave_sum64(double x) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+  return x;
 }
 
 // Each tensor's norm, rounded to its grad dtype, as torch._foreach_norm does.  A
@@ -200,31 +206,34 @@ __global__ __launch_bounds__(kNormWaves * 64) void tensor_norm_kernel(
     const apexw_tensor* __restrict__ tensors, int32_t n_tensors, const int64_t* __restrict__ unit_begin,
     const float* __restrict__ partial, float* __restrict__ norm, int32_t per, uint32_t flags,
     const apexw_row_means* __restrict__ rows) {
-  __shared__ float s_part[kNormWaves];
+  __shared__ double s_part[kNormWaves];
   const int wave = (int)uniform(threadIdx.x >> 6);
-  auto store = [&](int64_t t, float acc) {
+  auto store = [&](int64_t t, double acc) {
     const uint32_t gd = (tensors[t].flags >> APEXW_FLAG_GDT_SHIFT) & 3u;
-    float nrm = sqrtf(acc);
+    float nrm = sqrtf((float)acc);
     nrm = gd == APEXW_BF16 ? rnd<APEXW_BF16>(nrm) : (gd == APEXW_F16 ? rnd<APEXW_F16>(nrm) : nrm);
     norm[t] = nrm;
   };
   for (int64_t t0 = (int64_t)blockIdx.x * per; t0 < n_tensors; t0 += (int64_t)gridDim.x * per) {
     const int64_t t_end = t0 + per < n_tensors ? t0 + per : n_tensors;
+    bool large = false;
     if (t0 + wave < t_end) {
       const NormSpan s = norm_span(tensors, t0 + wave, unit_begin, partial, flags, rows);
-      if (s.n <= kNormWave) {
-        const float acc = wave_sum(span_sum(s, lane_id(), 64));
+      large = s.n > kNormWave;
+      if (!large) {
+        const double acc = wave_sum64(span_sum(s, lane_id(), 64));
         if (lane_id() == 0) store(t0 + wave, acc);
       }
     }
+    if (!__syncthreads_or(large)) continue;   // (the same for every wave)
     for (int64_t t = t0; t < t_end; ++t) {
       const NormSpan s = norm_span(tensors, t, unit_begin, partial, flags, rows);
       if (s.n <= kNormWave) continue;
-      const float acc = wave_sum(span_sum(s, threadIdx.x, kNormWaves * 64));
+      const double acc = wave_sum64(span_sum(s, threadIdx.x, kNormWaves * 64));
       if (lane_id() == 0) s_part[wave] = acc;
       __syncthreads();
       if (threadIdx.x == 0) {
-        float tot = 0.0f;
+        double tot = 0.0;
         for (int w = 0; w < kNormWaves; ++w) tot += s_part[w];
         store(t, tot);
       }
@@ -235,16 +244,16 @@ __global__ __launch_bounds__(kNormWaves * 64) void tensor_norm_kernel(
 
 __global__ __launch_bounds__(1024) void clip_coef_kernel(const float* __restrict__ norm, int32_t n_tensors, float clip,
                                                          float* __restrict__ coef) {
-  __shared__ float s_part[16];
-  float acc = 0.0f;
-  for (int32_t t = threadIdx.x; t < n_tensors; t += blockDim.x) acc = fmaf(norm[t], norm[t], acc);
-  acc = wave_sum(acc);
+  __shared__ double s_part[16];
+  double acc = 0.0;
+  for (int32_t t = threadIdx.x; t < n_tensors; t += blockDim.x) acc += (double)norm[t] * (double)norm[t];
+  acc = wave_sum64(acc);
   if (lane_id() == 0) s_part[threadIdx.x >> 6] = acc;
   __syncthreads();
   if (threadIdx.x == 0) {
-    float tot = 0.0f;
+    double tot = 0.0;
     for (int w = 0; w < (int)(blockDim.x >> 6); ++w) tot += s_part[w];
-    const float total = sqrtf(tot);
+    const float total = sqrtf((float)tot);
     float c = clip / (total + 1e-6f);
     // torch.clamp(c, max=1) then "multiply only if c < 1": NaN / >= 1 leave grads unscaled
     coef[0] = (c < 1.0f) ? c : 1.0f;
