@@ -230,13 +230,12 @@ APEXW_DEV float div_once(float x, float y) {
   return fmaf(fmaf(-q, y, x), r, q);
 }
 
-// The four INT8 codes of a word times a scale: bytes biased by 128 convert in one
-// instruction each, and fma(b, s, -128 s) is the exact (b - 128) s rounded once.
+// The four INT8 codes of a word times a scale: a sign-extending byte convert and one
+// product each, finite for every finite scale (a form biased by 128 overflows in 128 s
+// where the moments reach the top of the fp32 range).
 APEXW_DEV void i8_decode4(uint32_t w, float s, float* x) {
-  const uint32_t u = w ^ 0x80808080u;
-  const float z = -128.0f * s;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) x[j] = fmaf((float)((u >> (8 * j)) & 0xFFu), s, z);
+  for (int j = 0; j < 4; ++j) x[j] = (float)(int8_t)((w >> (8 * j)) & 0xFFu) * s;
 }
 // Four INT8 codes from m / scale: clamped to +-127, rounded to nearest even by adding
 // 1.5 x 2^23 (the code is then the low byte), gathered by byte permutes.
