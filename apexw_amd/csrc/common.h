@@ -230,12 +230,15 @@ APEXW_DEV float div_once(float x, float y) {
   return fmaf(fmaf(-q, y, x), r, q);
 }
 
-// The four INT8 codes of a word times a scale: a sign-extending byte convert and one
-// product each, finite for every finite scale (a form biased by 128 overflows in 128 s
-// where the moments reach the top of the fp32 range).
-APEXW_DEV void i8_decode4(uint32_t w, float s, float* x) {
+// The eight INT8 codes of two words times a scale: bytes biased by 128 convert in one
+// instruction each, fma(b, 1/2, -64) is half the code, exactly.  (With -128 s as the addend a
+// product fewer, but that overflows where the moments reach the top of the fp32 range.)
+APEXW_DEV void i8_decode8(uint32_t w0, uint32_t w1, float s, float* x) {
+  const uint32_t w[2] = {w0 ^ 0x80808080u, w1 ^ 0x80808080u};
+  const float s2 = 2.0f * s;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) x[j] = (float)(int8_t)((w >> (8 * j)) & 0xFFu) * s;
+  for (int j = 0; j < 8; ++j)
+    x[j] = fmaf((float)((w[j >> 2] >> (8 * (j & 3))) & 0xFFu), 0.5f, -64.0f) * s2;
 }
 // Four INT8 codes from m / scale: clamped to +-127, rounded to nearest even by adding
 // 1.5 x 2^23 (the code is then the low byte), gathered by byte permutes.

@@ -588,8 +588,7 @@ APEXW_DEV void fv_unit_full(const apexw_tensor& t, const apexw_fv_tensor& e, uin
       for (int j = 0; j < 8; ++j)
         m[j] = j & 1 ? __uint_as_float(mw[j >> 1] & 0xFFFF0000u) : bf16_bits_to_f32(mw[j >> 1] & 0xFFFFu);
     } else if constexpr (MK == kM8) {
-      i8_decode4(mw8[k].x, ms_old, m);
-      i8_decode4(mw8[k].y, ms_old, m + 4);
+      i8_decode8(mw8[k].x, mw8[k].y, ms_old, m);
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j)
@@ -771,8 +770,7 @@ APEXW_DEV bool fv_unit_row(const apexw_tensor& t, const apexw_fv_tensor& e, uint
       for (int j = 0; j < 8; ++j)
         m[j] = j & 1 ? __uint_as_float(mw[j >> 1] & 0xFFFF0000u) : __uint_as_float(mw[j >> 1] << 16);
     } else if constexpr (MK == kM8) {
-      i8_decode4(mw8[k].x, ms_old, m);
-      i8_decode4(mw8[k].y, ms_old, m + 4);
+      i8_decode8(mw8[k].x, mw8[k].y, ms_old, m);
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j)

@@ -430,8 +430,7 @@ APEXW_DEV void q8_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, const
 #pragma unroll
         for (int j = 0; j < 8; ++j) m[j] = c.code[(mw[0] >> (8 * (j >> 1) + ((j & 1) ? 0 : 4))) & 15u] * ms_old;
       } else {
-        i8_decode4(mw[0], ms_old, m);
-        i8_decode4(mw[1], ms_old, m + 4);
+        i8_decode8(mw[0], mw[1], ms_old, m);
       }
 #pragma unroll
       for (int j = 0; j < NV; ++j) v[j] = c.vlut[(vw[j >> 2] >> (8 * (j & 3))) & 0xFFu] * vs_old;
@@ -1197,8 +1196,7 @@ APEXW_DEV void ultra_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, co
       unpack8<PD>(rp, p);
       unpack8<GD>(rg, g);
       unpack8<VD>(rv, v);
-      i8_decode4(w.x, ms_old, m);
-      i8_decode4(w.y, ms_old, m + 4);
+      i8_decode8(w.x, w.y, ms_old, m);
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
