@@ -310,14 +310,22 @@ APEXW_DEV float q8_param(float p, float upd, float decay, uint32_t tflags, bool 
 // before memory): one quotient, root or rounding costs a few instructions instead of an
 // IEEE sequence, and results go to 16-bit and 8-bit words without an fp32 round trip.
 //
-// sqrt(x) for finite x >= 0, rounded to nearest: s = x y with y ~ rsqrt(x), then one FMA
-// residual (Markstein), wrong only within ~2^-45 of a rounding midpoint.  Below 2^-126
-// the result is off by at most 2^-63, added by every caller to an eps of kFastEps or more.
+// sqrt(x) for x = 0 or a normal finite x > 0, rounded to nearest: s = x y with y ~ rsqrt(x),
+// then one FMA residual (Markstein), wrong only within ~2^-45 of a rounding midpoint (2^31
+// values of 2^-40 to 2^8: all equal to sqrtf's).  Subnormal x is any_subnormal's.
 APEXW_DEV float sqrt_shared(float x) {
   // (an integer maximum: the float one first quiets NaNs)
   const float y = __builtin_amdgcn_rsqf(__uint_as_float((uint32_t)max((int)__float_as_uint(x), 0x00800000)));
   const float s = x * y;
   return fmaf(fmaf(-s, s, x), 0.5f * y, s);
+}
+// Whether any of the values is a positive subnormal, whose reciprocal root sqrt_shared cannot
+// use (grads below 1e-17 leave such second moments): the callers then take the IEEE sequences.
+template <int N> APEXW_DEV bool any_subnormal(const float (&x)[N]) {
+  uint32_t t = 0xFFFFFFFFu;
+#pragma unroll
+  for (int j = 0; j < N; ++j) t = min(t, __float_as_uint(x[j]) - 1u);   // (0 wraps to the top)
+  return t < 0x007FFFFFu;
 }
 // sqrt_shared and div_once (common.h) want every denominator at least this (any real eps is)
 constexpr float kFastEps = 1e-12f;
@@ -524,7 +532,7 @@ APEXW_DEV void q8_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, const
         for (int j = 0; j < NV; ++j) den[j] = fmaxf(sqrt_shared(v[j]) + hp.eps_scaled, hp.eps);
 #pragma unroll
         for (int j = 0; j < 8; ++j) q[j] = div_once(num[j], den[QUAD ? j >> 2 : j]);
-        ieee = q8_any_nonfinite8(q);   // an overflowing quotient (rare)
+        ieee = q8_any_nonfinite8(q) || any_subnormal(v);   // an overflowing quotient (rare)
       }
       if (ieee) {
 #pragma unroll
@@ -1236,7 +1244,7 @@ APEXW_DEV void ultra_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, co
     if (!ieee) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) q[j] = div_once(num[j], sqrt_shared(vf[j]) + hp.eps_scaled);
-      ieee = q8_any_nonfinite8(q);   // an overflowed second moment or quotient (rare)
+      ieee = q8_any_nonfinite8(q) || any_subnormal(vf);   // an overflowed second moment or quotient (rare)
     }
     if (ieee) {
 #pragma unroll
@@ -1438,8 +1446,9 @@ __global__ __launch_bounds__(256) void q8_fast_kernel(const apexw_tensor* __rest
   }
 }
 
+// (the grouped instantiation holds five waves per SIMD: 96 registers)
 template <bool SINGLE>
-__global__ __launch_bounds__(256) void q8_step_kernel(const apexw_tensor* __restrict__ tensors,
+__global__ __launch_bounds__(256, SINGLE ? 1 : 5) void q8_step_kernel(const apexw_tensor* __restrict__ tensors,
                                                       const apexw_unit* __restrict__ units,
                                                       int64_t n_units, apexw_hparams hp_in) {
   apexw_hparams hp = hp_in;

@@ -55,3 +55,23 @@ def test_int8_moments_at_the_top_of_the_range(precision, factored, shape):
     assert torch.allclose(sa["exp_avg_scales"].cpu().reshape(-1), sb["exp_avg_scales"].reshape(-1), rtol=1e-6, atol=0.0)
     d = sa["exp_avg"].cpu().reshape(-1).to(torch.int32) - sb["exp_avg"].reshape(-1).to(torch.int32)
     assert int(d.abs().max()) <= 1
+
+
+@pytest.mark.parametrize("precision,shape", [("8bit", (4096,)), ("8bit", (4099,)), ("ultra", (64, 64)),
+                                             ("ultra", (63, 65))])
+def test_subnormal_second_moments(precision, shape):
+    """Grads of 1e-17 to 1e-20 leave second moments below the smallest normal number beside normal ones
+    and zeros, under a denominator eps of one unit of 2^-63: fp32 parameters equal the oracle's IEEE root
+    and quotient bit for bit."""
+    print(f"subnormal v {precision} {shape}", flush=True)
+    gen = torch.Generator().manual_seed(11)
+    mag = 10.0 ** (-17.0 - 3.0 * torch.rand(shape, generator=gen, dtype=torch.float64))
+    grad = (mag * torch.randn(shape, generator=gen, dtype=torch.float64).sign()).float()
+    grad.view(-1)[::7] = 0.0
+    # the step's eps is eps sqrt(1 - beta2) = 1.26e-12
+    gp, cp, a, b = _pair(shape, grad, precision=precision, eps=4e-11)
+    a.step()
+    b.step()
+    x, y = gp.detach().cpu(), cp.detach()
+    assert int((y != 0).sum()) > y.numel() // 2
+    assert torch.equal(x, y), int((x != y).sum())
