@@ -12,8 +12,10 @@
 //      (contiguous) units -> rounded norm
 //   3. one workgroup combines the tensor norms -> coefficient
 // With grad centralization the pass that forms the row means also forms each row's
-// sum of squares about its mean (apexw_grad_row_stats), and 1 skips those tensors.
+// sum of squares about its mean (apexw_grad_row_stats; rows of up to APEXW_ROW_SUMSQ_MAX
+// elements), and 1 skips those tensors.
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 
@@ -115,7 +117,15 @@ APEXW_DEV float unit_sumsq(const apexw_tensor& t, int64_t start, int64_t cnt, bo
   return wave_sum(acc);
 }
 
-__global__ __launch_bounds__(256) void sumsq_kernel(const apexw_tensor* __restrict__ tensors,
+// Whether tensor t's squares are its rows', written after its row means by
+// row_means_kernel<true> (under APEXW_HP_ROW_SUMSQ, rows of up to APEXW_ROW_SUMSQ_MAX).
+APEXW_DEV bool norm_by_rows(const apexw_tensor& d, int64_t t, uint32_t flags, const apexw_row_means* rows) {
+  if (!(flags & APEXW_HP_ROW_SUMSQ) || !(d.flags & APEXW_FLAG_GC)) return false;
+  return (rows ? rows[t].row_len : (int64_t)d.block) <= APEXW_ROW_SUMSQ_MAX;
+}
+
+// (six waves per SIMD: 80 registers)
+__global__ __launch_bounds__(256, 6) void sumsq_kernel(const apexw_tensor* __restrict__ tensors,
                                                     const apexw_unit* __restrict__ units, int64_t n_units,
                                                     int64_t unit_size, float* __restrict__ partial, uint32_t flags,
                                                     float inv, const apexw_amp_dyn* __restrict__ amp,
@@ -132,11 +142,11 @@ __global__ __launch_bounds__(256) void sumsq_kernel(const apexw_tensor* __restri
   // a chunk inside one tensor whose row sums the row pass has formed: nothing to do
   // (a tensor's units are contiguous)
   const uint32_t t0 = units[base].tensor;
-  if (row_sums && (tensors[t0].flags & APEXW_FLAG_GC) && units[u_end - 1].tensor == t0) continue;
+  if (row_sums && units[u_end - 1].tensor == t0 && norm_by_rows(tensors[t0], t0, flags, rows)) continue;
   for (int64_t u = base + wave; u < u_end; u += 4) {
     const apexw_unit un = units[u];
     const apexw_tensor& t = tensors[un.tensor];
-    if (row_sums && (t.flags & APEXW_FLAG_GC)) continue;
+    if (row_sums && norm_by_rows(t, un.tensor, flags, rows)) continue;
     const int64_t us = unit_size > 0 ? unit_size : (t.block > 0 ? (int64_t)t.block : 64);
     const int64_t start = (int64_t)un.unit * us;
     const int64_t cnt = (t.n - start) < us ? (t.n - start) : us;
@@ -158,9 +168,7 @@ __global__ __launch_bounds__(256) void sumsq_kernel(const apexw_tensor* __restri
   }
 }
 
-// The partial sums of one tensor: its units' (from sumsq_kernel), or, for a
-// centralized tensor under APEXW_HP_ROW_SUMSQ, its rows' (written after its row means
-// by row_means_kernel<true>).
+// The partial sums of one tensor: its units' (from sumsq_kernel) or its rows' (norm_by_rows).
 struct NormSpan {
   const float* p;
   int64_t n;
@@ -168,7 +176,7 @@ struct NormSpan {
 APEXW_DEV NormSpan norm_span(const apexw_tensor* tensors, int64_t t, const int64_t* unit_begin, const float* partial,
                              uint32_t flags, const apexw_row_means* rows) {
   const apexw_tensor& d = tensors[t];
-  if ((flags & APEXW_HP_ROW_SUMSQ) && (d.flags & APEXW_FLAG_GC)) {
+  if (norm_by_rows(d, t, flags, rows)) {
     const float* means = rows ? rows[t].means : d.m_scale;
     const int64_t n_rows = d.n / (rows ? rows[t].row_len : (int64_t)d.block);
     return {means + n_rows, n_rows};
@@ -344,7 +352,8 @@ APEXW_DEV void prep_unit(const apexw_grad_prep& d, int64_t unit, bool san, bool 
 // row of a descriptor with row_len > 0; d.out is a float array of one mean per
 // row, each the grad dtype's rounding of the fp32 row sum over row_len of the
 // sanitized, unscaled grads.  SUMSQ (a clip follows): the row's sum of squares about
-// that mean, each difference rounded to the grad dtype, goes to d.out[rows + row].
+// that mean, each difference rounded to the grad dtype, goes to d.out[rows + row] for
+// rows of up to APEXW_ROW_SUMSQ_MAX elements.
 //
 // Bound by the read of the grads.  A lane holds its first kRowVecs 8-element vectors
 // (rows of up to 4096 16-bit elements whole), loaded before they are added, so the
@@ -352,63 +361,99 @@ APEXW_DEV void prep_unit(const apexw_grad_prep& d, int64_t unit, bool san, bool 
 // for the second sum, again.  Sanitizing changes only NaN / +-Inf grads, and one of
 // those makes the row's sum non-finite: the sums are formed without it, and a row
 // whose sum is not finite (rare) forms them again with it.
-// Four Llama layers (0.87 B bf16 grads, 1.75 GB, all centralized): 723 us for the means and
-// 644 us for the clip's own pass over them before, 527 us for both here.
+// Four Llama layers (0.87 B bf16 grads, 1.75 GB, all centralized), 8-bit step with clip: 3098 us
+// with the means' and the clip's passes apart, 1840 us with both here and the unscale flag
+// tested per element, 1751 us with each preparation (plain, unscaled, sanitized) its own loop.
+//
+// One wave walks a row twice in series where the clip's unit pass would spread its second
+// read over the chip.  Means, clip and norms of one bf16 tensor by the unit pass / here, us:
+// 64 x 4096: 94 / 20, 64 x 16384: 110 / 44, 64 x 32768: 128 / 75; without a limit
+// 64 x 65536: 190 / 228, 8 x 262144: 284 / 452, 8 x 1048576: 869 / 1789; fp32 alike.  So rows
+// beyond APEXW_ROW_SUMSQ_MAX leave their squares to the unit pass.
 // Sixteen rows to a workgroup: enough workgroups for small models, whose rows are few.
 constexpr int64_t kRowChunk = 16;
 template <int GD> constexpr int kRowVecs = GD == APEXW_F32 ? 4 : 8;
 
-template <int GD, bool SAN>
+// A grad as it enters the row's sums: as given, unscaled, or sanitized (and unscaled by a
+// run-time flag: rows of non-finite grads are rare).
+constexpr int kPlain = 0, kUnscale = 1, kSanitize = 2;
+template <int GD, int PREP>
 APEXW_DEV float row_value(float x, bool unscale, float inv) {
-  if constexpr (SAN) x = sanitize<GD>(x);
-  return unscale ? rnd<GD>(x * inv) : x;
+  if constexpr (PREP == kPlain) return x;
+  if constexpr (PREP == kSanitize) {
+    x = sanitize<GD>(x);
+    if (!unscale) return x;
+  }
+  return rnd<GD>(x * inv);
 }
 
 // The row's sum (MEAN false) or its sum of squares about mean (MEAN true) over a lane's
-// share: the held vectors r, the rest of [a, b) and the ragged ends.
-template <int GD, bool SAN, bool MEAN>
+// share: the held vectors r, the rest of [a, b) and the ragged ends.  Squares go to eight
+// running sums, folded after each batch of at most kRowVecs additions, so that no chain of
+// additions is longer than in the unit pass (32 terms) up to APEXW_ROW_SUMSQ_MAX elements.
+template <int GD, int PREP, bool MEAN>
 APEXW_DEV float row_sum(const apexw_grad_prep& d, const Raw8<GD> (&r)[kRowVecs<GD>], const PrepSpan& sp, int64_t lo,
                         int64_t hi, bool unscale, float inv, float mean) {
   constexpr int NV = kRowVecs<GD>;
   const int lane = lane_id();
-  float s = 0.0f;
-  auto add = [&](float x) {
-    x = row_value<GD, SAN>(x, unscale, inv);
+  float s = 0.0f, q[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  auto add = [&](int j, float x) {
+    x = row_value<GD, PREP>(x, unscale, inv);
     if constexpr (MEAN) {
       x = rnd<GD>(x - mean);
-      s = fmaf(x, x, s);
+      q[j] = fmaf(x, x, q[j]);
     } else {
       s += x;
     }
   };
+  auto fold = [&]() {
+    if constexpr (MEAN) {
+      s += ((q[0] + q[1]) + (q[2] + q[3])) + ((q[4] + q[5]) + (q[6] + q[7]));
+#pragma unroll
+      for (int j = 0; j < 8; ++j) q[j] = 0.0f;
+    }
+  };
   int64_t i = sp.a + (int64_t)lane * 8;
 #pragma unroll
-  for (int q = 0; q < NV; ++q, i += 512) {
+  for (int v = 0; v < NV; ++v, i += 512) {
     if (i < sp.b) {
       float x[8];
-      unpack8<GD>(r[q], x);
+      unpack8<GD>(r[v], x);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) add(x[j]);
+      for (int j = 0; j < 8; ++j) add(j, x[j]);
     }
   }
+  fold();
   for (; i + 3 * 512 < sp.b; i += 4 * 512) {
-    float x[4][8];
+    Raw8<GD> w[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) load8<GD>(d.g, i + q * 512, x[q]);
+    for (int v = 0; v < 4; ++v) raw_load8<GD>(d.g, i + v * 512, w[v]);
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+    for (int v = 0; v < 4; ++v) {
+      float x[8];
+      unpack8<GD>(w[v], x);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) add(x[q][j]);
+      for (int j = 0; j < 8; ++j) add(j, x[j]);
+    }
+    fold();
   }
   for (; i < sp.b; i += 512) {
     float x[8];
     load8<GD>(d.g, i, x);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) add(x[j]);
+    for (int j = 0; j < 8; ++j) add(j, x[j]);
   }
   // ragged ends: [lo, a) and [b, hi) (the whole row when not vectorized)
   const int64_t head = sp.a - lo, n_end = head + (hi - sp.b);
-  for (int64_t k = lane; k < n_end; k += 64) add(load1<GD>(d.g, k < head ? lo + k : sp.b + (k - head)));
+  for (int64_t k0 = lane; k0 < n_end; k0 += 8 * 64) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int64_t k = k0 + j * 64;
+      if (k < n_end) add(j, load1<GD>(d.g, k < head ? lo + k : sp.b + (k - head)));
+    }
+    fold();
+  }
+  fold();
   return wave_sum(s);
 }
 
@@ -424,15 +469,24 @@ APEXW_DEV void mean_row(const apexw_grad_prep& d, int64_t row, bool san, bool un
     const int64_t i = sp.a + (int64_t)lane * 8 + q * 512;
     if (i < sp.b) raw_load8<GD>(d.g, i, r[q]);
   }
-  float s = row_sum<GD, false, false>(d, r, sp, lo, hi, unscale, inv, 0.0f);
-  const bool redo = san && !(s - s == 0.0f);   // wave-uniform: every lane holds the sum
-  if (redo) s = row_sum<GD, true, false>(d, r, sp, lo, hi, unscale, inv, 0.0f);
-  const float mean = rnd<GD>(s / (float)d.row_len);
-  if (lane == 0) ((float*)d.out)[row] = mean;
-  if constexpr (SUMSQ) {
-    const float q = redo ? row_sum<GD, true, true>(d, r, sp, lo, hi, unscale, inv, mean)
-                         : row_sum<GD, false, true>(d, r, sp, lo, hi, unscale, inv, mean);
-    if (lane == 0) ((float*)d.out)[d.n / d.row_len + row] = q;
+  // both sums under one preparation of the grads
+  auto sums = [&](auto prep_c, float& mean, float& s, float& q) {
+    constexpr int PREP = decltype(prep_c)::value;
+    s = row_sum<GD, PREP, false>(d, r, sp, lo, hi, unscale, inv, 0.0f);
+    mean = rnd<GD>(s / (float)d.row_len);
+    q = 0.0f;
+    if (PREP != kSanitize && san && !(s - s == 0.0f)) return;   // formed again, sanitized
+    if (SUMSQ && d.row_len <= APEXW_ROW_SUMSQ_MAX)
+      q = row_sum<GD, PREP, true>(d, r, sp, lo, hi, unscale, inv, mean);
+  };
+  float mean, s, q;
+  if (unscale) sums(std::integral_constant<int, kUnscale>(), mean, s, q);
+  else sums(std::integral_constant<int, kPlain>(), mean, s, q);
+  // wave-uniform: every lane holds the sum
+  if (san && !(s - s == 0.0f)) sums(std::integral_constant<int, kSanitize>(), mean, s, q);
+  if (lane == 0) {
+    ((float*)d.out)[row] = mean;
+    if (SUMSQ && d.row_len <= APEXW_ROW_SUMSQ_MAX) ((float*)d.out)[d.n / d.row_len + row] = q;
   }
 }
 

@@ -201,9 +201,12 @@ typedef struct apexw_unit {
                                           when this flag is set and skipped otherwise.  The grads are
                                           prepared in their own dtype and read as fp32 values, as the
                                           reference's foreach order does. */
-#define APEXW_HP_ROW_SUMSQ (1u << 16)  /* apexw_grad_clip_coef: the centralized tensors' sums of squares are
-                                          those that apexw_grad_row_stats wrote after their row means in
-                                          this step; their grads are not read again */
+#define APEXW_HP_ROW_SUMSQ (1u << 16)  /* apexw_grad_clip_coef: the sums of squares of the centralized tensors
+                                          with rows of up to APEXW_ROW_SUMSQ_MAX elements are those that
+                                          apexw_grad_row_stats wrote after their row means in this step;
+                                          their grads are not read again */
+/* Longer rows' squares are summed by the clip's own pass: one wave would walk such a row twice. */
+#define APEXW_ROW_SUMSQ_MAX 32768
 
 /* Step scalars of one launch, written on the device by apexw_amp_prepare (32 bytes). */
 typedef struct apexw_amp_dyn {
@@ -520,9 +523,9 @@ int apexw_grad_row_means(const apexw_grad_prep* preps, int32_t n_preps, const ap
 
 /*
  * apexw_grad_row_means with the global-norm clip's sums in the same pass: out holds
- * 2 n / row_len floats, and entry n / row_len + r receives the sum of squares of
- * dtype_round(g - mean) over row r.  The clip of the same step then takes
- * APEXW_HP_ROW_SUMSQ.
+ * 2 n / row_len floats, and for rows of up to APEXW_ROW_SUMSQ_MAX elements entry
+ * n / row_len + r receives the sum of squares of dtype_round(g - mean) over row r.  The clip
+ * of the same step then takes APEXW_HP_ROW_SUMSQ.
  */
 int apexw_grad_row_stats(const apexw_grad_prep* preps, int32_t n_preps, const apexw_unit* units, int64_t n_units,
                          float grad_inv_scale, uint32_t flags, const apexw_amp_dyn* amp, void* stream);
