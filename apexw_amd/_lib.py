@@ -13,7 +13,7 @@ import numpy as np
 
 from ._build import LIB_PATH
 
-ABI_VERSION = 25
+ABI_VERSION = 26
 
 # dtype codes
 F32, BF16, F16, U8, I8 = 0, 1, 2, 3, 4
@@ -185,6 +185,7 @@ SIGNATURES = {
                                           _i32, _i64, _i64, _i64, _i64, _i64, _f32, _f32, _vp]),
     "apexw_check_grad_prep": (ctypes.c_int, [_vp]),
     "apexw_check_row_means": (ctypes.c_int, [_vp]),
+    "apexw_check_row_stats": (ctypes.c_int, [_vp]),
     "apexw_grad_prep_units": (ctypes.c_int64, [_vp]),
     "apexw_grad_prepare": (ctypes.c_int, [_vp, _i32, _vp, _i64, _f32, _u32, _vp, _vp]),
     "apexw_grad_row_means": (ctypes.c_int, [_vp, _i32, _vp, _i64, _f32, _u32, _vp, _vp]),

@@ -456,12 +456,13 @@ class StepPlan:
         squares when a clip follows.  amp_dyn: device scalars of a GradScaler step (the
         unscale factor is read there)."""
         flags = L.HP_SANITIZE | (L.HP_UNSCALE if inv_scale is not None else 0)
-        fn = self._lib.apexw_grad_prepare
+        name = "apexw_grad_prepare"
         if self.gc_fold:
-            fn = self._lib.apexw_grad_row_stats if clip else self._lib.apexw_grad_row_means
-        st = fn(self.d_prep.data_ptr(), len(self.params), self.d_prep_units.data_ptr(), self.n_prep_units,
-                1.0 if inv_scale is None else inv_scale, flags, amp_dyn, stream)
-        L.check(st, "apexw_grad_row_means" if self.gc_fold else "apexw_grad_prepare")
+            name = "apexw_grad_row_stats" if clip else "apexw_grad_row_means"
+        st = getattr(self._lib, name)(
+            self.d_prep.data_ptr(), len(self.params), self.d_prep_units.data_ptr(), self.n_prep_units,
+            1.0 if inv_scale is None else inv_scale, flags, amp_dyn, stream)
+        L.check(st, name)
 
     def _layout_units(self, fast):
         """Device table in launch order and its unit table.  8-bit: full-block-kernel
@@ -575,7 +576,7 @@ class StepPlan:
                 for i in range(len(self.params)):
                     if self.gc_fold:
                         if self.host_prep["row_len"][i]:
-                            L.check(self._lib.apexw_check_row_means(self.host_prep[i:i + 1].ctypes.data),
+                            L.check(self._lib.apexw_check_row_stats(self.host_prep[i:i + 1].ctypes.data),
                                     f"row means of tensor {i}")
                         continue
                     L.check(self._lib.apexw_check_grad_prep(self.host_prep[i:i + 1].ctypes.data),

@@ -684,17 +684,26 @@ int apexw_check_grad_prep(const apexw_grad_prep* d) {
   return APEXW_OK;
 }
 
-int apexw_check_row_means(const apexw_grad_prep* d) {
+namespace {
+
+// A descriptor of the row passes whose out holds `per_row` floats for each row.
+int check_rows(const apexw_grad_prep* d, int64_t per_row) {
   if (!d || !d->g || !d->out || d->n <= 0 || d->row_len <= 0 || d->reserved) return APEXW_ERR_ARG;
   if (d->dtype != APEXW_F32 && d->dtype != APEXW_BF16 && d->dtype != APEXW_F16) return APEXW_ERR_DTYPE;
   if (d->n % d->row_len) return APEXW_ERR_ARG;
   const int64_t size = d->dtype == APEXW_F32 ? 4 : 2;
   const uintptr_t g = (uintptr_t)d->g, o = (uintptr_t)d->out;
-  const uintptr_t g_end = g + (uintptr_t)(d->n * size), o_end = o + (uintptr_t)(d->n / d->row_len * 4);
-  if (g < o_end && o < g_end) return APEXW_ERR_ARG;   // the means must not alias the grad
+  const uintptr_t g_end = g + (uintptr_t)(d->n * size), o_end = o + (uintptr_t)(d->n / d->row_len * per_row * 4);
+  if (g < o_end && o < g_end) return APEXW_ERR_ARG;   // what is written must not alias the grad
   if ((g & (uintptr_t)(size - 1)) || (o & 3u)) return APEXW_ERR_ALIGN;
   return APEXW_OK;
 }
+
+}  // namespace
+
+int apexw_check_row_means(const apexw_grad_prep* d) { return check_rows(d, 1); }
+
+int apexw_check_row_stats(const apexw_grad_prep* d) { return check_rows(d, 2); }
 
 int64_t apexw_grad_prep_units(const apexw_grad_prep* d) {
   const int st = apexw_check_grad_prep(d);

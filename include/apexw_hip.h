@@ -44,7 +44,7 @@
 extern "C" {
 #endif
 
-#define APEXW_ABI_VERSION 25
+#define APEXW_ABI_VERSION 26
 
 /* status codes */
 enum apexw_status {
@@ -533,6 +533,8 @@ int apexw_grad_row_stats(const apexw_grad_prep* preps, int32_t n_preps, const ap
 /* Validate one descriptor (host copy) of apexw_grad_row_means: row_len > 0 divides n, out holds
  * n / row_len floats that do not overlap the grad. */
 int apexw_check_row_means(const apexw_grad_prep* d);
+/* The same for apexw_grad_row_stats: out holds 2 n / row_len floats. */
+int apexw_check_row_stats(const apexw_grad_prep* d);
 
 /* ------------------------------------------------------------------------- */
 /* Muon: Newton-Schulz on the matrix cores                                    */
