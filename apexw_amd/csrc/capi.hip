@@ -546,6 +546,9 @@ int check_grouped(const apexw_gemm_problem* problems, const uint32_t* items, con
   if (n_workgroups <= 0 || n_workgroups % APEXW_GEMM_QUEUES) return APEXW_ERR_ARG;
   if (kind <= 0 || kind > 63 || !(kind & (APEXW_GEMM_OUT_C | APEXW_GEMM_OUT_CT))) return APEXW_ERR_ARG;
   if ((kind & APEXW_GEMM_KIND_NN) && (kind & APEXW_GEMM_OUT_CT)) return APEXW_ERR_ARG;
+  // 128 x 128 tiles: in panels, B as [n x k]
+  if ((kind & APEXW_GEMM_KIND_TILE128) && (!(kind & APEXW_GEMM_KIND_PANEL) || (kind & APEXW_GEMM_KIND_NN)))
+    return APEXW_ERR_ARG;
   if (((uintptr_t)problems | (uintptr_t)items | (uintptr_t)queue_offsets) & 3u) return APEXW_ERR_ALIGN;
   return APEXW_OK;
 }
