@@ -6,10 +6,11 @@
 //   A  = X X^T                 (symmetric, K = n)
 //   B  = c A A + b A           (symmetric, K = m)
 //   X' = B X + a X             (K = m)
-// Every product is computed as an "NT" GEMM (both operands K-contiguous): X is
-// kept in both layouts, X [m x n] and X^T [n x m], so B X = B (X^T)^T reads X^T
-// rows.  The epilogue of the last product writes X' in both layouts; the
-// symmetric products are written through the transposed store (same matrix).
+// A and B are "NT" GEMMs (both operands K-contiguous), their results written through
+// the transposed store too (same matrix).  X' is one as well where X is kept in both
+// layouts, X [m x n] and X^T [n x m]: B X = B (X^T)^T reads X^T rows, and the epilogue
+// writes X' in both layouts; or it reads X as [K x N] rows by transposing fragment reads
+// and writes X' once (the caller's choice per plan, by K).
 // Work matrices are zero-padded to multiples of the 256 x 256 tile; zero rows
 // and columns stay zero through every product, so the kernel has no bounds
 // checks.
@@ -396,7 +397,7 @@ APEXW_DEV void gemm_tile(const uint16_t* __restrict__ A, const uint16_t* __restr
   // over all banks.  A wave reads back only what it wrote itself, and LDS keeps one
   // wave's accesses in order, so no barrier is needed.  This is what bounds products of
   // short K, where nothing overlaps it (staged the other way round it took 256 2-byte
-  // writes and 256 2-byte reads per lane): EPI
+  // writes and 256 2-byte reads per lane).
   uint16_t* stage = lds + wave * (kWM * kWN);
   constexpr int kCh = kWM / 8;   // 16-byte chunks of a staged column
   // element offset of rows il .. of staged column jl (il a multiple of 4)

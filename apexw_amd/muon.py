@@ -9,8 +9,9 @@ handling.  The step runs through libapexw_hip.so:
   wide orientation) normalised by its Frobenius norm, of every matrix in two launches;
 * ``NSPlan``: per iteration three bf16 MFMA GEMMs
   (``A = X X^T``; ``B = c A A + b A``; ``X = B X + a X``), each one grouped
-  launch (``apexw_gemm_nt_grouped``) over every Muon matrix of the step; the
-  two symmetric products compute only the tiles on and above the diagonal;
+  launch over every Muon matrix of the step, all of them enqueued by one call
+  (``apexw_gemm_nt_grouped_run``); the two symmetric products compute only the
+  tiles on and above the diagonal;
 * the last ``X`` product of each matrix applies the decoupled weight decay and
   ``p -= lr * scale * U`` in its epilogue (``APEXW_GEMM_APPLY``);
   ``apexw_muon_apply`` does it as a separate pass when ``ns_steps == 0``.
@@ -80,13 +81,14 @@ class NSWorkspace:
     """bf16 Newton-Schulz buffers for `batch` matrices whose wide work shape is m x n.
 
     Dimensions are padded to the GEMM tile; the padding is zero and stays zero
-    through every product.  X and its transpose X^T are kept for two iterations
-    (ping-pong), plus the symmetric A and B: X' = B X + a X reads X^T as its [N x K]
-    operand (direct fragment reads, measured 3% faster than X as [K x N] rows with
-    transposing reads) and writes X' and X'^T.  The buffers hold their matrices in 32 x 32 panels
-    (APEXW_GEMM_PANEL): each K stage of a product's operand is then whole
-    128-byte lines, which the grouped GEMM reads with fewer L2 requests than
-    the 64-byte row pieces of a row-major operand (panel=False keeps row-major).
+    through every product.  X is kept for two iterations (ping-pong), plus the
+    symmetric A and B.  X' = B X + a X reads either X^T as its [N x K] operand and
+    writes X' and X'^T, or X itself as [K x N] rows (NSPlan.nn, NN_MAX_K); X^T, kept
+    for two iterations too, is allocated when a plan of the first form asks for it.
+    The buffers hold their matrices in 32 x 32 panels (APEXW_GEMM_PANEL): each K
+    stage of a product's operand is then whole 128-byte lines, which the grouped
+    GEMM reads with fewer L2 requests than the 64-byte row pieces of a row-major
+    operand (panel=False keeps row-major).
     """
 
     def __init__(self, m, n, batch, device, panel=True):
@@ -95,17 +97,24 @@ class NSWorkspace:
         self.layout = _lib.LAYOUT_PANEL if self.panel else _lib.LAYOUT_ROWS
         t = _lib.GEMM_TILE
         self.mp, self.np_ = _pad(m, t), _pad(n, t)
-        z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=device)  # noqa: E731
-        self.x = [z(batch, self.mp, self.np_), z(batch, self.mp, self.np_)]
-        self.xt = [z(batch, self.np_, self.mp), z(batch, self.np_, self.mp)]
-        self.a = z(batch, self.mp, self.mp)
-        self.b = z(batch, self.mp, self.mp)
+        self.x = [self._zeros(self.mp, self.np_), self._zeros(self.mp, self.np_)]
+        self._xt = None
+        self.a = self._zeros(self.mp, self.mp)
+        self.b = self._zeros(self.mp, self.mp)
         lib = _lib.load()
         per = int(lib.apexw_muon_workspace_floats(m, n))
         self.partial = torch.empty(batch, max(per, 1), dtype=torch.float32, device=device)
-        # per entry the addresses the preparation writes: X, X^T and the norm's partial sums
-        self.rows = [(self.x[0][e].data_ptr(), self.xt[0][e].data_ptr(), self.partial[e].data_ptr())
-                     for e in range(batch)]
+        # per entry the addresses that every preparation writes: X and the norm's partial sums
+        self.rows = [(self.x[0][e].data_ptr(), self.partial[e].data_ptr()) for e in range(batch)]
+
+    def _zeros(self, *shape):
+        return torch.zeros(self.batch, *shape, dtype=torch.bfloat16, device=self.device)
+
+    @property
+    def xt(self):
+        if self._xt is None:
+            self._xt = [self._zeros(self.np_, self.mp), self._zeros(self.np_, self.mp)]
+        return self._xt
 
     def rows_of(self, buf):
         """One matrix of x, a or b as a row-major tensor (a copy when in panels)."""
@@ -218,6 +227,10 @@ class NSPlan:
         every = tuple(range(len(wss)))
         self.nn = (bool(wss) and self._tile(wss, every, 2) == _lib.GEMM_TILE
                    and max(ws.mp for ws in wss) <= NN_MAX_K)
+        # where the preparation writes X^T, in the plan's order (None: no product reads it)
+        self.xt = None
+        if not self.nn and max(steps, default=0) > 0:
+            self.xt = np.array([ws.xt[0][e].data_ptr() for ws in wss for e in range(ws.batch)], dtype=np.uint64)
         built = {}
         self.iters = []
         for i in range(max(steps, default=0)):
@@ -286,8 +299,10 @@ class NSPlan:
 
     def prepare(self, stream, items, inv_scale, amp=None):
         """Momentum and normalised work matrices of every matrix (MUON_ITEM_DTYPE rows in the
-        plan's order) in two launches."""
+        plan's order, their xt filled in here) in two launches."""
         lib = _lib.load()
+        if self.xt is not None:
+            items["xt"] = self.xt
         if self._prep_units is None:
             tables = []
             for which in (0, 1):
@@ -503,8 +518,6 @@ class ApexMuon(Optimizer):
                 plan = self._ns_plan(djobs, dev)
                 stream = torch.cuda.current_stream(dev).cuda_stream
                 items = np.array([row for j in djobs for row in j["items"]], dtype=_lib.MUON_ITEM_DTYPE)
-                if plan.nn:
-                    items["xt"] = 0       # its products read no X^T
                 plan.prepare(stream, items, inv_scale, amp_ptr)
                 applies = [self._apply_args(j) for j in djobs]
                 plan.run(stream, applies, self.keep_ns_result, amp_ptr)
@@ -597,8 +610,8 @@ class ApexMuon(Optimizer):
             self._count_step(st)
             g = p.grad if p.grad.is_contiguous() else p.grad.contiguous()
             grads.append(g)     # a contiguous copy lives until the step has been enqueued
-            x, xt, partial = ws.rows[i]
-            items.append((st["momentum"].data_ptr(), g.data_ptr(), x, xt, partial, rows, cols, ws.np_, ws.mp, mu,
+            x, partial = ws.rows[i]
+            items.append((st["momentum"].data_ptr(), g.data_ptr(), x, 0, partial, rows, cols, ws.np_, ws.mp, mu,
                           1.0 - mu, _dtype_code(g.dtype), ws.layout, nesterov, 0))
         return {"plist": plist, "targets": [self._target(p) for p in plist], "group": group, "ws": ws,
                 "rows": rows, "cols": cols, "steps": int(group["ns_steps"]), "batched": len(plist) > 1,
