@@ -221,7 +221,7 @@ class NSPlan:
         # the preparation's unit tables (momentum chunks, 64 x 64 tiles) over every matrix, in order
         self.n_items = sum(ws.batch for ws in wss)
         self._prep_units = None
-        self._prepared = None   # (bytes of the last item table, its device copy)
+        self._prepared = None   # (bytes of the last item table, its stream, its device copy)
         self._seq = None        # host array of the launch sequence
         # one form of X' for the whole plan: a later iteration reads what an earlier one wrote
         every = tuple(range(len(wss)))
@@ -277,7 +277,7 @@ class NSPlan:
         lib = _lib.load()
         key = None
         if applies is not None:
-            key = (tuple(tuple(a) for a in applies), bool(keep_result))
+            key = (tuple(tuple(a) for a in applies), bool(keep_result), stream)
         # the tables never move, but for the fused update's, whose rows change with the
         # parameters' addresses and the step's scalars
         if self._seq is None:
@@ -313,14 +313,16 @@ class NSPlan:
                 units["unit"] = np.arange(len(units)) - np.repeat(np.cumsum(counts) - counts, counts)
                 tables.append((torch.from_numpy(units.view(np.uint8)).to(self.device), len(units)))
             self._prep_units = tables
-        # the item table goes up only when an address or a scalar changed
+        # the item table goes up only when an address or a scalar changed, and again on another
+        # stream: a table's memory belongs to the stream it was allocated on, and is given back
+        # behind that stream's work alone
         raw = items.tobytes()
-        if self._prepared is None or self._prepared[0] != raw:
+        if self._prepared is None or self._prepared[:2] != (raw, stream):
             _lib.check(lib.apexw_check_muon_items(items.ctypes.data, len(items)), "apexw_check_muon_items")
             staged = torch.from_numpy(items.view(np.uint8)).pin_memory()
-            self._prepared = (raw, staged.to(self.device, non_blocking=True))
+            self._prepared = (raw, stream, staged.to(self.device, non_blocking=True))
         (um, nm), (ux, nx) = self._prep_units
-        _lib.check(lib.apexw_muon_prepare_grouped(self._prepared[1].data_ptr(), len(items), um.data_ptr(), nm,
+        _lib.check(lib.apexw_muon_prepare_grouped(self._prepared[2].data_ptr(), len(items), um.data_ptr(), nm,
                                                   ux.data_ptr(), nx, NS_EPS, inv_scale, amp, stream),
                    "apexw_muon_prepare_grouped")
 

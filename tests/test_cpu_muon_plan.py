@@ -51,3 +51,13 @@ def test_x_transposed_is_kept_only_where_a_product_reads_it(lib, m, n, batch, st
     assert items["xt"].tolist() == want
     if reads:
         assert not any(bool(t.any()) for t in ws.xt)      # the padding starts, and stays, zero
+
+
+def test_item_table_is_not_shared_between_streams(lib):
+    ws, plan = _plan(64, 64, 1)
+    keep = []
+    for stream in (1, 1, 2, 2):
+        plan.prepare(stream, _items(ws, 64, 64), 1.0)
+        keep.append(plan._prepared)
+    assert lib.tables[0] == lib.tables[1] and lib.tables[2] == lib.tables[3]
+    assert lib.tables[2] != lib.tables[1]
