@@ -32,6 +32,7 @@ FLAG_GC = 1 << 16
 FLAG_ULTRA = 1 << 17
 FLAG_VSCALE = 1 << 18
 
+UNIT_GROUP, UNIT_GROUP_MAX = 1 << 31, 512   # up to 4 small units of a q8 / ultra launch in one entry
 COMPACT_UNIT = 2048
 
 MODE_COLD, MODE_REPLAY, MODE_NATIVE, MODE_SINGLE = 0, 1, 2, 3

@@ -58,6 +58,12 @@ _DT = {torch.float32: L.F32, torch.bfloat16: L.BF16, torch.float16: L.F16, torch
 CHUNKED_MIN_NUMEL = 262144  # larger 8-bit tensors take the reference's chunked rounding order
 _GRAD = operator.attrgetter("grad")
 
+# General 8-bit / ultra units beyond which small ones share a workgroup (_step_entries): about
+# four to a CU.  One bf16 tensor, us per step with a workgroup each / in groups: blocks of 256,
+# 1024 units 18.1 / 18.1, 4096 units 23.9 / 18.4, 262144 units 1277 / 444; blocks of 64, 4096
+# units 26.3 / 18.3, 1048576 units 5051 / 1734.
+GROUP_FROM = 1024
+
 # status of _host.scan (csrc/host.cpp)
 SCAN_SAME, SCAN_GRADS_MOVED, SCAN_MISSING, SCAN_REBUILT, SCAN_SLOW, SCAN_GRAD_DTYPE = range(6)
 
@@ -495,22 +501,51 @@ class StepPlan:
         if self.slow_ptrs is not None:
             self.d_slow = _upload(np.ascontiguousarray(self.slow_ptrs[perm]), self.device)
         self.d_unit_begin = _upload(self.unit_begin, self.device)
-        # the step kernels' units: all but the factored rows' (apexw_factored_step steps
-        # those; the clip's norm pass still covers every unit).  Factored tensors are
-        # never full-block 8-bit tensors, so the fast prefix is unchanged.
+        # the step kernels' entries: all units but the factored rows' (apexw_factored_step steps
+        # those; the clip's norm pass still covers every unit), small ones in groups.  Factored
+        # tensors are never full-block 8-bit tensors, so the fast prefix is unchanged.
+        tab = self.host_table[perm]
         fac_rows = self.factored[perm]
-        if fac_rows.any():
-            self._step_keep = ~fac_rows[units["tensor"]]
-            step_units = units[self._step_keep]
-            self.n_step_units = len(step_units)
-            self.d_step_units = _upload(step_units.view(np.uint8), self.device) \
-                if len(step_units) else self.d_units
-        else:
-            self._step_keep, self.n_step_units, self.d_step_units = None, total, self.d_units
+        small = np.zeros(n, dtype=bool)
+        if self.kind == "q8":
+            small = np.minimum(tab["block"].astype(np.int64), tab["n"]) <= L.UNIT_GROUP_MAX
+            small[:n_bf + n_f32] = False
+        self._step_keep = np.repeat(~fac_rows, counts)
+        self._small_units = np.repeat(small, counts)
+        entries, self.n_step_units, _, _ = self._step_entries(np.ones(total, dtype=bool))
+        # (entries None: the whole unit table as it is)
+        self.d_step_units = self.d_units if entries is None or not len(entries) else \
+            _upload(entries.view(np.uint8), self.device)
         self.clip_ws = None
         self._fv_subsets = {}
         self.fv = self._fv_layout(tuple(int(i) for i in np.nonzero(self.factored[perm])[0])) \
             if self.factored.any() else None
+
+    def _step_entries(self, mask):
+        """The unit table of a step launch over the units chosen by mask (table order): (entries,
+        entries of the launch, full-block bf16 ones, full-block fp32 ones); entries is None when
+        they are the whole unit table as it is.
+
+        General and ultra units of up to UNIT_GROUP_MAX elements go last, in groups of four that
+        share a workgroup, a wave each (APEXW_UNIT_GROUP), when there are more general units
+        than the chip holds workgroups at once: below that each has a workgroup to itself
+        without waiting (GROUP_FROM)."""
+        sel = np.flatnonzero(mask & self._step_keep)
+        units = self._host_units
+        nb = int(np.searchsorted(sel, self.n_fast_units))
+        n_fast = int(np.searchsorted(sel, self.n_fast_units + self.n_fast_f32_units))
+        small = self._small_units[sel]
+        n_small = int(small.sum())
+        if n_small == 0 or len(sel) - n_fast <= GROUP_FROM:
+            return (None if len(sel) == len(units) else units[sel]), len(sel), nb, n_fast - nb
+        large, small = sel[~small], sel[small]
+        k = (n_small + 3) // 4
+        groups = np.zeros(k, dtype=L.UNIT_DTYPE)
+        at = 4 * np.arange(k, dtype=np.int64)
+        groups["tensor"] = L.UNIT_GROUP | np.minimum(n_small - at, 4)
+        groups["unit"] = len(large) - n_fast + k + at      # counted from the general range's start
+        entries = np.concatenate([units[large], groups, units[small]])
+        return entries, len(large) + k, nb, n_fast - nb
 
     def _fv_layout(self, rows):
         """Factored-v table, workspace and units for the device-table rows ``rows``."""
@@ -1005,16 +1040,11 @@ class StepPlan:
         out = []
         for val, srv in sorted(set(keys), key=keys.index):
             keep = (vals == val) & (srp == srv)
-            mask = np.repeat(keep, self.unit_counts)
-            if self._step_keep is not None:
-                mask = mask[self._step_keep]
-            if not mask.any():
+            entries, n_units, nb, nf = self._step_entries(np.repeat(keep, self.unit_counts))
+            if n_units == 0:
                 continue
-            idx = _upload(np.flatnonzero(mask), self.device)
-            sel = self.d_step_units.view(-1, 8).index_select(0, idx).reshape(-1)
-            nb, nf = self.n_fast_units, self.n_fast_f32_units
-            out.append(((sel, int(mask.sum()), int(mask[:nb].sum()), int(mask[nb:nb + nf].sum())), int(val),
-                        bool(srv)))
+            sel = self.d_step_units if entries is None else _upload(entries.view(np.uint8), self.device)
+            out.append(((sel, n_units, nb, nf), int(val), bool(srv)))
         return out
 
     def _hparams(self, lr, b1, b2, eps, wd, step, sr, sanitize, coef, seed, cold, inv_scale=None):

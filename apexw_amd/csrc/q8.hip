@@ -1,12 +1,14 @@
 // 8-bit fused multi-tensor AdamW step (gfx950).
 //
-// One wavefront owns one quantization block (<= 2048 elements, 32 per lane in 4
-// groups of 8 consecutive elements one wave-width apart).  A block is
-// dequantized, updated and requantized entirely in registers: the absmax of the
-// new momentum and the max of the new variance are wavefront reductions, so no
-// LDS round trip or barrier is needed between the update and the requantization.
-// LDS only holds the decode tables (256-entry log-uint8 LUT, NF4 codebook),
-// loaded once per persistent workgroup.
+// A block is dequantized, updated and requantized entirely in registers.  In the
+// full-block kernel (bf16 / fp32 parameters, NF4 m, quad v, blocks of 2048) one
+// wavefront owns a block, 32 elements per lane in 4 groups of 8 consecutive ones one
+// wave-width apart, and the absmax of the new momentum and the max of the new variance
+// are wavefront reductions.  In the general and ultra kernels a workgroup owns a block,
+// 8 elements per thread, and its waves' maxima meet in LDS (one barrier); units of up to
+// 512 elements may come in groups (APEXW_UNIT_GROUP), one to a wave.
+// LDS otherwise holds the decode tables (256-entry log-uint8 LUT, NF4 codebook),
+// loaded once per workgroup.
 //
 // Arithmetic restates the reference's CPU 8-bit path ApexW._step_ultra
 // (apexw/optimizer.py:4313-4735): chunked order for large tensors (:4402-4499),
@@ -358,11 +360,15 @@ template <int DT> APEXW_DEV void store8_rnd(void* base, int64_t i, float (&x)[8]
 // unit_uniform(r) - 1/2 for the 16 bits r = h >> 16, exact in one FMA.
 APEXW_DEV float half_noise(uint32_t h) { return fmaf((float)(h >> 16), 0x1p-16f, 0x1p-17f - 0.5f); }
 
-// Maximum over a workgroup of 4 waves of two non-negative values; red: 8 floats of LDS,
+// A unit's threads: those of a workgroup of 4 waves, or of one wave (solo).
+APEXW_DEV int unit_thread(bool solo) { return solo ? lane_id() : (int)threadIdx.x; }
+
+// Maximum over the unit's threads of two non-negative values; red: 8 floats of LDS,
 // alternated between two such buffers by the caller so that one barrier suffices.
-APEXW_DEV void block_max2(float& a, float& b, float* red) {
+APEXW_DEV void unit_max2(float& a, float& b, float* red, bool solo) {
   a = wave_max(a);
   b = wave_max(b);
+  if (solo) return;
   const int w = (int)(threadIdx.x >> 6);
   if (lane_id() == 0) {
     red[w] = a;
@@ -375,7 +381,8 @@ APEXW_DEV void block_max2(float& a, float& b, float* red) {
 
 // One quantization block per workgroup, any layout (INT8 m, fp32 params, other block
 // sizes, unaligned tensors): each of the four waves takes 512 of the up to 2048
-// elements, 8 per lane, and the block's two maxima meet in LDS.
+// elements, 8 per lane, and the block's two maxima meet in LDS.  A block of up to 512
+// elements leaves waves without work: one of a group (APEXW_UNIT_GROUP) takes one wave.
 //
 // The block's serial path is what bounds small launches (16 blocks of 2048 elements:
 // 35 us when one wave walked a block's four groups, 9 us here) and its instruction
@@ -389,7 +396,7 @@ APEXW_DEV void block_max2(float& a, float& b, float* red) {
 // floor, p decayed in fp32 then p + (-step_size * num) / den, INT8 m
 // requantised from its own absmax (no EMA, no SR).
 template <int PD, bool NF4, bool QUAD, bool SINGLE>
-APEXW_DEV void q8_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, const Q8Ctx& c, float* red) {
+APEXW_DEV void q8_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, const Q8Ctx& c, float* red, bool solo) {
   constexpr int GD = PD;
   constexpr int NV = QUAD ? 2 : 8;   // second moments per lane
   const apexw_hparams& hp = *c.hp;
@@ -401,7 +408,8 @@ APEXW_DEV void q8_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, const
   const float ms_old = t.m_scale[blk];
   const float vs_old = t.v_scale[blk];
   const bool generic = tflags & APEXW_FLAG_GENERIC;
-  const int64_t rel = (int64_t)threadIdx.x * 8;
+  const int tid = unit_thread(solo);
+  const int64_t rel = (int64_t)tid * 8;
   const int cnt = rel >= cnt_blk ? 0 : (int)((cnt_blk - rel) < 8 ? (cnt_blk - rel) : 8);
   const int64_t e0 = start + rel;
   const bool full = !(tflags & APEXW_FLAG_SCALAR) && cnt == 8;
@@ -577,13 +585,13 @@ APEXW_DEV void q8_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, const
     }
   }
   // ---- block scales (EMA-max smoothing against the previous scales)
-  block_max2(amax, vmax, red);
+  unit_max2(amax, vmax, red, solo);
   float ms = fmaxf(amax, 1e-12f);
   if (!NF4) ms = ms / 127.0f;
   if (NF4 || !SINGLE) ms = fmaxf(ms, ms_old * 0.9f);
   float vs = fmaxf(vmax, 1e-12f);
   vs = fmaxf(vs, vs_old * 0.95f);
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     t.m_scale[blk] = ms;
     t.v_scale[blk] = vs;
   }
@@ -1131,12 +1139,12 @@ APEXW_DEV void q8_block_fast(const apexw_tensor& t, uint32_t tix, uint32_t blk, 
 // (apexw/optimizer.py:2458-2471): p.mul_(wd) in the parameter dtype, fp32
 // moments, p.addcdiv_ rounded once, m and v rounded once on store.
 template <int PD, int MD, int VD, bool SINGLE>
-APEXW_DEV void q8_dense(const apexw_tensor& t, uint32_t unit, const Q8Ctx& c) {
+APEXW_DEV void q8_dense(const apexw_tensor& t, uint32_t unit, const Q8Ctx& c, bool solo) {
   constexpr int GD = PD;
   const apexw_hparams& hp = *c.hp;
   const int64_t start = (int64_t)unit * 2048;
   const int64_t end = (t.n - start) < 2048 ? t.n : start + 2048;
-  for (int64_t i = start + threadIdx.x; i < end; i += blockDim.x) {
+  for (int64_t i = start + unit_thread(solo); i < end; i += solo ? 64 : 256) {
     float p = load1<PD>(t.p, i);
     if constexpr (SINGLE) {
       const float g = load1<GD>(t.g, i);
@@ -1177,7 +1185,7 @@ APEXW_DEV void q8_dense(const apexw_tensor& t, uint32_t unit, const Q8Ctx& c) {
 // sequence and one wave held a block's 32 elements per lane (134 VGPRs): four Llama
 // layers (0.87 B bf16 parameters, 10.5 GB) 2610 -> 2013 us per step, 5.2 TB/s.
 template <int PD, int VD>
-APEXW_DEV void ultra_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, const Q8Ctx& c, float* red) {
+APEXW_DEV void ultra_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, const Q8Ctx& c, float* red, bool solo) {
   constexpr int GD = PD;
   const apexw_hparams& hp = *c.hp;
   const bool sr = hp.flags & APEXW_HP_SR;
@@ -1185,7 +1193,8 @@ APEXW_DEV void ultra_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, co
   const int64_t start = (int64_t)blk * bs;
   const int64_t cnt_blk = (t.n - start) < bs ? (t.n - start) : bs;
   const float ms_old = t.m_scale[blk];
-  const int64_t rel = (int64_t)threadIdx.x * 8;
+  const int tid = unit_thread(solo);
+  const int64_t rel = (int64_t)tid * 8;
   const int cnt = rel >= cnt_blk ? 0 : (int)((cnt_blk - rel) < 8 ? (cnt_blk - rel) : 8);
   const int64_t e0 = start + rel;
   const bool full = !(t.flags & APEXW_FLAG_SCALAR) && cnt == 8;
@@ -1272,9 +1281,9 @@ APEXW_DEV void ultra_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, co
       if (j < cnt) amax = fmaxf(amax, fabsf(m[j]));
   }
   // the block scale and the INT8 codes, as the 8-bit step's (quantize_blockwise_int8)
-  block_max2(amax, none, red);
+  unit_max2(amax, none, red, solo);
   const float ms = fmaxf(fmaxf(amax, 1e-12f) / 127.0f, ms_old * 0.9f);
-  if (threadIdx.x == 0) t.m_scale[blk] = ms;
+  if (tid == 0) t.m_scale[blk] = ms;
   if (!cnt) return;
   const uint32_t key = sr ? rng_key(hp.seed, tix, hp.step, 1u, (uint32_t)(start >> 32)) : 0u;
   float y[8];
@@ -1304,21 +1313,21 @@ APEXW_DEV void ultra_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, co
 // parameters) with v in it or fp32, or fp32 m and v.
 template <bool SINGLE>
 APEXW_DEV void dense_dispatch(const apexw_tensor& t, uint32_t unit, const Q8Ctx& c, uint32_t pd, uint32_t md,
-                              uint32_t vd) {
+                              uint32_t vd, bool solo) {
   if (md == APEXW_F32) {
     // fp32 m implies fp32 v (checked on the host)
-    if (pd == APEXW_F32) q8_dense<APEXW_F32, APEXW_F32, APEXW_F32, SINGLE>(t, unit, c);
-    else if (pd == APEXW_BF16) q8_dense<APEXW_BF16, APEXW_F32, APEXW_F32, SINGLE>(t, unit, c);
-    else q8_dense<APEXW_F16, APEXW_F32, APEXW_F32, SINGLE>(t, unit, c);
+    if (pd == APEXW_F32) q8_dense<APEXW_F32, APEXW_F32, APEXW_F32, SINGLE>(t, unit, c, solo);
+    else if (pd == APEXW_BF16) q8_dense<APEXW_BF16, APEXW_F32, APEXW_F32, SINGLE>(t, unit, c, solo);
+    else q8_dense<APEXW_F16, APEXW_F32, APEXW_F32, SINGLE>(t, unit, c, solo);
   } else if (pd == APEXW_F32) {
-    if (vd == APEXW_F32) q8_dense<APEXW_F32, APEXW_BF16, APEXW_F32, SINGLE>(t, unit, c);
-    else q8_dense<APEXW_F32, APEXW_BF16, APEXW_BF16, SINGLE>(t, unit, c);
+    if (vd == APEXW_F32) q8_dense<APEXW_F32, APEXW_BF16, APEXW_F32, SINGLE>(t, unit, c, solo);
+    else q8_dense<APEXW_F32, APEXW_BF16, APEXW_BF16, SINGLE>(t, unit, c, solo);
   } else if (pd == APEXW_BF16) {
-    if (vd == APEXW_F32) q8_dense<APEXW_BF16, APEXW_BF16, APEXW_F32, SINGLE>(t, unit, c);
-    else q8_dense<APEXW_BF16, APEXW_BF16, APEXW_BF16, SINGLE>(t, unit, c);
+    if (vd == APEXW_F32) q8_dense<APEXW_BF16, APEXW_BF16, APEXW_F32, SINGLE>(t, unit, c, solo);
+    else q8_dense<APEXW_BF16, APEXW_BF16, APEXW_BF16, SINGLE>(t, unit, c, solo);
   } else {
-    if (vd == APEXW_F32) q8_dense<APEXW_F16, APEXW_F16, APEXW_F32, SINGLE>(t, unit, c);
-    else q8_dense<APEXW_F16, APEXW_F16, APEXW_F16, SINGLE>(t, unit, c);
+    if (vd == APEXW_F32) q8_dense<APEXW_F16, APEXW_F16, APEXW_F32, SINGLE>(t, unit, c, solo);
+    else q8_dense<APEXW_F16, APEXW_F16, APEXW_F16, SINGLE>(t, unit, c, solo);
   }
 }
 
@@ -1349,11 +1358,18 @@ __global__ __launch_bounds__(256) void ultra_step_kernel(const apexw_tensor* __r
   c.coef = (hp.flags & APEXW_HP_CLIP) ? *hp.clip_coef : 1.0f;
   c.gc_means = nullptr;
   c.gc_rl = 0;
-  // block_max2's two buffers, exchanged after each unit that meets its barrier
+  // unit_max2's two buffers, exchanged after each unit that meets its barrier
   __shared__ float s_red[2][8];
   int par = 0;
+  const uint32_t wave = uniform(threadIdx.x >> 6);
   for (int64_t u = blockIdx.x; u < n_units; u += gridDim.x) {
-    const apexw_unit un = units[u];
+    apexw_unit un = units[u];
+    const bool solo = un.tensor & APEXW_UNIT_GROUP;
+    if (solo) {
+      // a unit per wave, none meets a barrier
+      if (wave >= (un.tensor & 7u)) continue;
+      un = units[un.unit + wave];
+    }
     const apexw_tensor& t = tensors[un.tensor];
     q8_set_rows(c, t, un.tensor);
     q8_set_gains(c, t, un.tensor);
@@ -1362,21 +1378,21 @@ __global__ __launch_bounds__(256) void ultra_step_kernel(const apexw_tensor* __r
     const uint32_t md = (f >> APEXW_FLAG_MDT_SHIFT) & 3u;
     const uint32_t vd = (f >> APEXW_FLAG_VDT_SHIFT) & 3u;
     if (f & APEXW_FLAG_DENSE) {
-      dense_dispatch<false>(t, un.unit, c, pd, md, vd);
+      dense_dispatch<false>(t, un.unit, c, pd, md, vd, solo);
     } else if (f & APEXW_FLAG_ULTRA) {
       // (the flags are the workgroup's: every wave takes the same branch)
       // v in the parameter's compact dtype (fp16 for fp16 parameters, else bf16) or fp32
       if (pd == APEXW_F32) {
-        if (vd == APEXW_F32) ultra_block<APEXW_F32, APEXW_F32>(t, un.tensor, un.unit, c, s_red[par]);
-        else ultra_block<APEXW_F32, APEXW_BF16>(t, un.tensor, un.unit, c, s_red[par]);
+        if (vd == APEXW_F32) ultra_block<APEXW_F32, APEXW_F32>(t, un.tensor, un.unit, c, s_red[par], solo);
+        else ultra_block<APEXW_F32, APEXW_BF16>(t, un.tensor, un.unit, c, s_red[par], solo);
       } else if (pd == APEXW_BF16) {
-        if (vd == APEXW_F32) ultra_block<APEXW_BF16, APEXW_F32>(t, un.tensor, un.unit, c, s_red[par]);
-        else ultra_block<APEXW_BF16, APEXW_BF16>(t, un.tensor, un.unit, c, s_red[par]);
+        if (vd == APEXW_F32) ultra_block<APEXW_BF16, APEXW_F32>(t, un.tensor, un.unit, c, s_red[par], solo);
+        else ultra_block<APEXW_BF16, APEXW_BF16>(t, un.tensor, un.unit, c, s_red[par], solo);
       } else {
-        if (vd == APEXW_F32) ultra_block<APEXW_F16, APEXW_F32>(t, un.tensor, un.unit, c, s_red[par]);
-        else ultra_block<APEXW_F16, APEXW_F16>(t, un.tensor, un.unit, c, s_red[par]);
+        if (vd == APEXW_F32) ultra_block<APEXW_F16, APEXW_F32>(t, un.tensor, un.unit, c, s_red[par], solo);
+        else ultra_block<APEXW_F16, APEXW_F16>(t, un.tensor, un.unit, c, s_red[par], solo);
       }
-      par ^= 1;
+      if (!solo) par ^= 1;
     }
   }
 }
@@ -1478,11 +1494,18 @@ __global__ __launch_bounds__(256, SINGLE ? 1 : 5) void q8_step_kernel(const apex
   c.coef = (hp.flags & APEXW_HP_CLIP) ? *hp.clip_coef : 1.0f;
   c.gc_means = nullptr;
   c.gc_rl = 0;
-  // block_max2's two buffers, exchanged after each unit that meets its barrier
+  // unit_max2's two buffers, exchanged after each unit that meets its barrier
   __shared__ float s_red[2][8];
   int par = 0;
+  const uint32_t wave = uniform(threadIdx.x >> 6);
   for (int64_t u = blockIdx.x; u < n_units; u += gridDim.x) {
-    const apexw_unit un = units[u];
+    apexw_unit un = units[u];
+    const bool solo = un.tensor & APEXW_UNIT_GROUP;
+    if (solo) {
+      // a unit per wave, none meets a barrier
+      if (wave >= (un.tensor & 7u)) continue;
+      un = units[un.unit + wave];
+    }
     const apexw_tensor& t = tensors[un.tensor];
     q8_set_rows(c, t, un.tensor);
     q8_set_gains(c, t, un.tensor);
@@ -1491,26 +1514,26 @@ __global__ __launch_bounds__(256, SINGLE ? 1 : 5) void q8_step_kernel(const apex
     if (f & APEXW_FLAG_FACTORED) continue;  // stepped by apexw_factored_step
     const uint32_t vd = (f >> APEXW_FLAG_VDT_SHIFT) & 3u;
     if (f & APEXW_FLAG_DENSE) {
-      dense_dispatch<SINGLE>(t, un.unit, c, pd, (f >> APEXW_FLAG_MDT_SHIFT) & 3u, vd);
+      dense_dispatch<SINGLE>(t, un.unit, c, pd, (f >> APEXW_FLAG_MDT_SHIFT) & 3u, vd, solo);
       continue;
     }
     // ultra rows belong to ultra_step_kernel (apexw_ultra_step): never read their dense v as codes
     if (f & APEXW_FLAG_ULTRA) continue;
     const bool nf4 = f & APEXW_FLAG_NF4, quad = f & APEXW_FLAG_QUAD;
     if (pd == APEXW_F32) {
-      if (nf4 && quad) q8_block<APEXW_F32, true, true, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
-      else if (nf4) q8_block<APEXW_F32, true, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
-      else q8_block<APEXW_F32, false, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
+      if (nf4 && quad) q8_block<APEXW_F32, true, true, SINGLE>(t, un.tensor, un.unit, c, s_red[par], solo);
+      else if (nf4) q8_block<APEXW_F32, true, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par], solo);
+      else q8_block<APEXW_F32, false, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par], solo);
     } else if (pd == APEXW_BF16) {
-      if (nf4 && quad) q8_block<APEXW_BF16, true, true, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
-      else if (nf4) q8_block<APEXW_BF16, true, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
-      else q8_block<APEXW_BF16, false, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
+      if (nf4 && quad) q8_block<APEXW_BF16, true, true, SINGLE>(t, un.tensor, un.unit, c, s_red[par], solo);
+      else if (nf4) q8_block<APEXW_BF16, true, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par], solo);
+      else q8_block<APEXW_BF16, false, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par], solo);
     } else {
-      if (nf4 && quad) q8_block<APEXW_F16, true, true, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
-      else if (nf4) q8_block<APEXW_F16, true, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
-      else q8_block<APEXW_F16, false, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par]);
+      if (nf4 && quad) q8_block<APEXW_F16, true, true, SINGLE>(t, un.tensor, un.unit, c, s_red[par], solo);
+      else if (nf4) q8_block<APEXW_F16, true, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par], solo);
+      else q8_block<APEXW_F16, false, false, SINGLE>(t, un.tensor, un.unit, c, s_red[par], solo);
     }
-    par ^= 1;
+    if (!solo) par ^= 1;
   }
 }
 

@@ -122,6 +122,15 @@ typedef struct apexw_unit {
   uint32_t unit;
 } apexw_unit;
 
+/* An entry of the general range of apexw_q8_step, or of apexw_ultra_step, may stand for 1 to
+ * 4 units of at most APEXW_UNIT_GROUP_MAX elements each (min(block, n) of their tensors), one
+ * to a wave of its workgroup: tensor = APEXW_UNIT_GROUP | count, unit = the index of the first
+ * of them, plain entries that lie one after another behind the n_units of the launch in the
+ * same array, counted from the range's first entry.  Large models with small blocks: one
+ * workgroup per block leaves three of its four waves idle. */
+#define APEXW_UNIT_GROUP (1u << 31)
+#define APEXW_UNIT_GROUP_MAX 512
+
 #define APEXW_COMPACT_UNIT 2048
 
 /* apexw_hparams.mode */
