@@ -322,7 +322,8 @@ APEXW_DEV float sqrt_shared(float x) {
   return fmaf(fmaf(-s, s, x), 0.5f * y, s);
 }
 // Whether any of the values is a positive subnormal, whose reciprocal root sqrt_shared cannot
-// use (grads below 1e-17 leave such second moments): the callers then take the IEEE sequences.
+// use (grads below 1e-17 leave such second moments): the 8-bit step then takes the IEEE
+// sequences (the ultra step scales every value instead).
 template <int N> APEXW_DEV bool any_subnormal(const float (&x)[N]) {
   uint32_t t = 0xFFFFFFFFu;
 #pragma unroll
@@ -1251,9 +1252,12 @@ APEXW_DEV void ultra_block(const apexw_tensor& t, uint32_t tix, uint32_t blk, co
     float q[8];
     bool ieee = !(hp.eps_scaled >= kFastEps);
     if (!ieee) {
+      // 2^12 times the root of every vf, subnormal ones too; the FMA scales it exactly, so the
+      // sum rounds as root + eps does (vf beyond 2^104 overflows here: NaN, and IEEE below)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) q[j] = div_once(num[j], sqrt_shared(vf[j]) + hp.eps_scaled);
-      ieee = q8_any_nonfinite8(q) || any_subnormal(vf);   // an overflowed second moment or quotient (rare)
+      for (int j = 0; j < 8; ++j)
+        q[j] = div_once(num[j], fmaf(sqrt_shared(vf[j] * 0x1p24f), 0x1p-12f, hp.eps_scaled));
+      ieee = q8_any_nonfinite8(q);   // a second moment near overflow, or an overflowed quotient (rare)
     }
     if (ieee) {
 #pragma unroll
