@@ -390,7 +390,7 @@ APEXW_DEV void unit_max2(float& a, float& b, float* red, bool solo) {
 // count the large ones: so one division per denominator (rcp_refined, div_shared)
 // instead of an IEEE sequence per element, the noise hashed once, and 8 elements'
 // state per lane instead of 32 (159 -> 96 VGPRs).  25 M parameters of a convolutional
-// network, nearly all INT8 rows: 140 -> 87 us per step.
+// network, nearly all INT8 rows: 140 -> 84 us per step.
 // SINGLE: the per-parameter in-backward update (ApexW._step_single_param_fused,
 // apexw/optimizer.py:2411-2457): raw fp32 grads, m = b1 m + (1-b1) g,
 // lookahead b1 m' + (1-b1) g, denominator sqrt(v) + eps_scaled without the eps
